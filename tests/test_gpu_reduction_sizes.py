@@ -1,0 +1,61 @@
+"""The tridiagonal reduction and the back-transformation at the edges of their tiles.
+
+Stacks of H2 molecules (one AO per atom, a helium atom for odd counts) give
+systems of every AO count: around the 16-column phases and 32-row tiles of the
+register reduction, the 192-column switch between its two forms, the
+16-reflector blocks and 16-row tiles of the back-transformation, and the
+256-AO limit of the register kernels.  Energies, forces and charges against the
+oracle at the package's bars.
+"""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from xtbloom_amd import interface, workloads
+
+pytestmark = pytest.mark.gpu
+
+E_TOL, F_TOL, Q_TOL = 1e-7, 1e-6, 1e-6
+
+
+def stack(n, rng):
+    """n atoms with one AO each: H2 molecules on a grid, one He when n is odd."""
+    z, xyz = [], []
+    for m in range(n // 2):
+        c = 5.0 * np.array([m % 5, (m // 5) % 5, m // 25]) + rng.normal(0.0, 0.1, 3)
+        u = rng.normal(size=3)
+        u *= 0.5 * (1.40 + rng.uniform(-0.05, 0.05)) / np.linalg.norm(u)
+        z += [1, 1]
+        xyz += [c - u, c + u]
+    if n % 2:
+        z.append(2)
+        xyz.append(np.array([-5.0, -5.0, 0.0]))
+    return dict(Z=np.array(z, np.int32), xyz=np.array(xyz), charge=0.0, uhf=0)
+
+
+@pytest.mark.parametrize("sizes", [
+    [1, 2, 3, 4, 5, 6],                       # no, one or a few reflectors
+    [14, 15, 16, 17, 18, 19, 31, 32, 33, 34],  # first phases and row tiles, one or two WY blocks
+    [47, 48, 49, 63, 64, 65, 66, 95, 97],
+    [127, 128, 129, 130, 175, 176, 177],
+    [190, 191, 192, 193, 194, 195],           # the switch between the two forms
+    [208, 223, 225, 240, 254, 255, 256],
+    [257, 258, 259, 272, 289],                # the blocked reduction
+], ids=lambda s: f"{s[0]}-{s[-1]}")
+def test_sizes_against_the_oracle(sizes):
+    rng = np.random.default_rng(sizes[0])
+    b = workloads.from_systems([stack(n, rng) for n in sizes])
+    ctx = interface.Context("hip", 0)
+    try:
+        print("case reduction sizes", sizes, flush=True)
+        out = interface.compute_arrays(ctx, b.atom_offsets, b.atomic_numbers, b.positions,
+                                       b.molecular_charges, b.unpaired_electrons)
+    finally:
+        ctx.close()
+    ref = O.batch(b.atom_offsets, b.atomic_numbers, b.positions, b.molecular_charges,
+                  b.unpaired_electrons, threads=4)
+    assert np.all(out.per_system_status == 0) and np.all(ref["status"] == 0)
+    assert np.abs(out.scc_iterations - ref["iterations"]).max() <= 1
+    assert np.abs(out.energies - ref["energies"]).max() <= E_TOL
+    assert np.abs(out.forces + ref["gradient"]).max() <= F_TOL
+    assert np.abs(out.charges - ref["charges"]).max() <= Q_TOL

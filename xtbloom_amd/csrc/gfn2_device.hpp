@@ -275,11 +275,27 @@ __device__ __forceinline__ double dpp_move(double x) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
+// a permutation of the lanes within their rows (quad_perm, row_ror, mirrors):
+// every lane has a source, so no old value is set up
+template <int CTRL>
+__device__ __forceinline__ double dpp_permute(double x) {
+  const long long b = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// sum over the 16 lanes of a DPP row, in every lane
+__device__ __forceinline__ double row16_sum(double v) {
+  v += dpp_permute<0xb1>(v);   // quad_perm [1,0,3,2]
+  v += dpp_permute<0x4e>(v);   // quad_perm [2,3,0,1]
+  v += dpp_permute<0x124>(v);  // row_ror:4
+  v += dpp_permute<0x128>(v);  // row_ror:8
+  return v;
+}
+
 __device__ __forceinline__ double wave_sum(double v) {
-  v += dpp_move<0xb1, 0xf>(v);   // quad_perm [1,0,3,2]
-  v += dpp_move<0x4e, 0xf>(v);   // quad_perm [2,3,0,1]
-  v += dpp_move<0x124, 0xf>(v);  // row_ror:4
-  v += dpp_move<0x128, 0xf>(v);  // row_ror:8
+  v = row16_sum(v);
   v += dpp_move<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
   v += dpp_move<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
   const long long b = __double_as_longlong(v);

@@ -346,79 +346,6 @@ struct ClusterOut {
 };
 constexpr int kInverseIterations = 3;
 
-// Householder reduction with the trailing matrix in global memory, one
-// reflector at a time (any n).  The register kernel below keeps it as its
-// general branch; the host sends systems above 256 AOs to the blocked
-// reduction (k_tridiag_blocked), which reads the matrix a sixth as often.
-__device__ __forceinline__ void tridiag_global(double* A, int n, double* d, double* e, double* v, double* pq,
-                               double* red, double* bc) {
-  const int tid = threadIdx.x, nt = blockDim.x;
-  for (int k = 0; k + 2 < n; ++k) {
-    const int m = n - k - 1;
-    double ss = 0.0;
-    for (int i = tid; i < m; i += nt) {
-      const double x = A[(k + 1 + i) + (int64_t)k * n];
-      v[i] = x;
-      ss += x * x;
-    }
-    ss = block_sum(ss, red);
-    if (tid == 0) {
-      const double x0 = v[0];
-      const double xn = sqrt(ss);
-      d[k] = A[k + (int64_t)k * n];
-      if (xn == 0.0 || ss - x0 * x0 == 0.0) {
-        e[k] = x0;  // already reduced: no reflection
-        bc[0] = 0.0;
-      } else {
-        const double alpha = x0 >= 0.0 ? -xn : xn;
-        const double v0 = x0 - alpha;
-        const double vv = ss - x0 * x0 + v0 * v0;
-        e[k] = alpha;
-        v[0] = v0;
-        bc[0] = 1.0 / sqrt(vv);
-      }
-    }
-    __syncthreads();
-    const double inv = bc[0];
-    if (inv == 0.0) {
-      for (int i = tid; i < m; i += nt) A[(k + 1 + i) + (int64_t)k * n] = 0.0;
-      __syncthreads();
-      continue;
-    }
-    for (int i = tid; i < m; i += nt) {
-      v[i] *= inv;
-      A[(k + 1 + i) + (int64_t)k * n] = v[i];
-    }
-    __syncthreads();
-    // p = A22 v, q = p - (v^T p) v
-    double kp = 0.0;
-    for (int i = tid; i < m; i += nt) {
-      double p = 0.0;
-      for (int j = 0; j < m; ++j) p += A[(k + 1 + i) + (int64_t)(k + 1 + j) * n] * v[j];
-      pq[i] = p;
-      kp += v[i] * p;
-    }
-    const double K = block_sum(kp, red);
-    for (int i = tid; i < m; i += nt) pq[i] -= K * v[i];
-    __syncthreads();
-    // A22 -= 2 (v q^T + q v^T)
-    for (int j = 0; j < m; ++j) {
-      const double vj = v[j], qj = pq[j];
-      for (int i = tid; i < m; i += nt)
-        A[(k + 1 + i) + (int64_t)(k + 1 + j) * n] -= 2.0 * (v[i] * qj + pq[i] * vj);
-    }
-    __syncthreads();
-  }
-  if (tid == 0) {
-    if (n >= 2) {
-      d[n - 2] = A[(n - 2) + (int64_t)(n - 2) * n];
-      e[n - 2] = A[(n - 1) + (int64_t)(n - 2) * n];
-    }
-    d[n - 1] = A[(n - 1) + (int64_t)(n - 1) * n];
-    e[n - 1] = 0.0;
-  }
-}
-
 // Householder reduction for n > 256 in panels of kTriPanel reflectors, the
 // arrangement of LAPACK's dsytrd/dlatrd.  Within a panel the trailing matrix
 // is not written: after reflectors 0 .. j-1 of the panel it equals
@@ -829,9 +756,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 }
 
 constexpr int kTriPad = 257;  // row stride of the partial-sum buffers (bank spread)
-constexpr int kTriTail = 64;    // trailing columns reduced by one wavefront
-constexpr int kTriTailLd = 65;  // row stride of that trailing block in LDS
-static_assert(kTriTail * kTriTailLd <= 32 * kTriPad, "the trailing block reuses the row partials");
+constexpr int kFullN = 192;  // columns reduced with both triangles in registers (tridiag_full)
 
 template <int NR>
 __device__ __forceinline__ void tridiag_registers(double* A, int n, double* d, double* e, double* v,
@@ -868,7 +793,7 @@ __device__ __forceinline__ void tridiag_registers(double* A, int n, double* d, d
   }
   __syncthreads();
   int k = 0;
-  for (; k + 2 < n && n - k > kTriTail; ++k) {
+  for (; n - k > kFullN; ++k) {
     // Reflector of column k, formed redundantly (and identically) by every
     // wavefront: v = (x - alpha e_{k+1}) / |x - alpha e_{k+1}|.
     double part = 0.0;
@@ -984,86 +909,242 @@ __device__ __forceinline__ void tridiag_registers(double* A, int n, double* d, d
     }
     __syncthreads();
   }
-  if (k + 2 >= n) {  // n < 3: nothing was reduced
-    static_for<0, NE>([&](auto S) __attribute__((always_inline)) {
-      constexpr int sl = decltype(S)::value;
-      constexpr int TI = tri_row(sl), TJ = tri_col(sl);
-      const int i = 16 * TI + lr, j = 32 * TJ + lc;
-      if (i == n - 2 && j == n - 2) d[n - 2] = 2.0 * a[sl];
-      if (i == n - 1 && j == n - 2) e[n - 2] = a[sl];
-      if (i == n - 1 && j == n - 1) d[n - 1] = 2.0 * a[sl];
-    });
-    if (tid == 0) e[n - 1] = 0.0;
-    return;
-  }
-  // The last n - k0 <= kTriTail columns: one wavefront finishes them on the
-  // trailing block, stored whole (symmetric, full diagonal) in LDS, without
-  // block barriers.  Lane l owns row k + 1 + l of the step-k update.
-  const int k0 = k;
-  double* tb = rowpart;  // (n - k0) x kTriTailLd
+  // the trailing kFullN x kFullN block goes back to A, both triangles with the
+  // full diagonal, for tridiag_full.  The indices are opaque copies: addresses
+  // shared with the loads at the top would stay live through the loop, in
+  // scratch memory.
+  int wr = lr, wc = lc;
+  asm volatile("" : "+v"(wr), "+v"(wc));
   static_for<0, NE>([&](auto S) __attribute__((always_inline)) {
     constexpr int sl = decltype(S)::value;
     constexpr int TI = tri_row(sl), TJ = tri_col(sl);
-    const int i = 16 * TI + lr, j = 32 * TJ + lc;
-    if (i >= k0 && j >= k0 && i < n && j < n && i >= j) {
+    const int i = 16 * TI + wr, j = 32 * TJ + wc;
+    if (j >= k && i < n && i >= j) {
       const double x = a[sl];
       if (i > j) {
-        tb[(i - k0) * kTriTailLd + (j - k0)] = x;
-        tb[(j - k0) * kTriTailLd + (i - k0)] = x;
+        A[i + (int64_t)j * n] = x;
+        A[j + (int64_t)i * n] = x;
       } else {
-        tb[(i - k0) * kTriTailLd + (i - k0)] = 2.0 * x;
+        A[i + (int64_t)i * n] = 2.0 * x;
       }
     }
   });
   __syncthreads();
-  if (tid < 64) {
-    const int l = tid;
-    auto lds_fence = [] __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
-    for (; k + 2 < n; ++k) {
-      const int m1 = n - k - 1;  // rows below the diagonal
-      const int rl = k + 1 + l - k0, ck = k - k0;
-      const double x = l < m1 ? tb[rl * kTriTailLd + ck] : 0.0;
-      const double ss = wave_sum(x * x);
-      const double x0 = tb[(ck + 1) * kTriTailLd + ck];
-      const double xn = sqrt(ss);
-      const bool noref = xn == 0.0 || ss - x0 * x0 == 0.0;  // already reduced
-      const double alpha = x0 >= 0.0 ? -xn : xn;
-      const double v0 = x0 - alpha;
-      const double inv = noref ? 0.0 : 1.0 / sqrt(ss - x0 * x0 + v0 * v0);
-      if (l == 0) {
-        d[k] = tb[ck * kTriTailLd + ck];
-        e[k] = noref ? x0 : alpha;
-      }
-      const double vl = l < m1 ? inv * (l == 0 ? v0 : x) : 0.0;
-      if (l < m1) A[(k + 1 + l) + (int64_t)k * n] = vl;
-      v[l] = vl;
-      lds_fence();
-      // p = A v over the trailing rows (v broadcast from LDS)
-      double p = 0.0;
-      if (l < m1) {
-        const double* row = tb + rl * kTriTailLd + ck + 1;
-        for (int j = 0; j < m1; ++j) p = fma(row[j], v[j], p);
-      }
-      // K = v.p; with q = p - K v,  A -= 2 (v q^T + q v^T) = 2 (v p^T + (p - 2 K v) v^T)
-      const double K2 = 2.0 * wave_sum(vl * p);
-      const double rq = fma(-K2, vl, p);
-      pq[l] = p;
-      lds_fence();
-      if (l < m1) {
-        double* row = tb + rl * kTriTailLd + ck + 1;
-        for (int j = 0; j < m1; ++j) row[j] -= 2.0 * (vl * pq[j] + rq * v[j]);
-      }
-      lds_fence();
-    }
-    if (l == 0) {
-      const int c2 = n - 2 - k0;
-      d[n - 2] = tb[c2 * kTriTailLd + c2];
-      e[n - 2] = tb[(c2 + 1) * kTriTailLd + c2];
-      d[n - 1] = tb[(c2 + 1) * kTriTailLd + c2 + 1];
-      e[n - 1] = 0.0;
+}
+
+// 1 / sqrt(x) for x > 0, finite and not subnormal: the hardware estimate y with
+// one third-order correction y (1 + e / 2 + 3 e^2 / 8), e = 1 - x y^2 (within
+// 1 ulp; a fraction of the IEEE square root's and division's instructions,
+// which sit on the serial chain of a reduction step)
+__device__ __forceinline__ double rsqrt_refined(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
+// Sums of R values over the 16 lanes of a DPP row, scattered: on return lane lc
+// of the row holds the row's sum of value row16_index<R>(lc).  Four exchange
+// stages (lane ^ 15, ^ 7, ^ 2, ^ 1); each of the first three halves the number
+// of live values by sending away the one the partner keeps.
+template <int CTRL, int M, int NV>
+__device__ __forceinline__ void row16_stage(double (&v)[NV], bool hi) {
+#pragma unroll
+  for (int q = 0; q < (M + 1) / 2; ++q) {
+    if (2 * q + 1 < M) {
+      const double keep = hi ? v[2 * q + 1] : v[2 * q];
+      const double send = hi ? v[2 * q] : v[2 * q + 1];
+      v[q] = keep + dpp_permute<CTRL>(send);
+    } else {
+      v[q] = v[2 * q] + dpp_permute<CTRL>(v[2 * q]);
     }
   }
+}
+constexpr int half_up(int m) { return (m + 1) / 2; }
+template <int R, int NV>
+__device__ __forceinline__ double row16_sums(double (&v)[NV], int lc) {
+  constexpr int M1 = half_up(R), M2 = half_up(M1), M3 = half_up(M2);
+  static_assert(M3 == 1, "at most eight values");
+  row16_stage<0x140, R>(v, (lc & 8) != 0);   // row_mirror: lane ^ 15
+  row16_stage<0x141, M1>(v, (lc & 4) != 0);  // row_half_mirror: lane ^ 7
+  row16_stage<0x4e, M2>(v, (lc & 2) != 0);   // quad_perm [2,3,0,1]: lane ^ 2
+  return v[0] + dpp_permute<0xb1>(v[0]);     // quad_perm [1,0,3,2]: lane ^ 1
+}
+template <int R>
+__device__ __forceinline__ int row16_index(int lc) {
+  constexpr int M1 = half_up(R), M2 = half_up(M1);
+  int q = 0;
+  if (M2 > 1) q = (lc & 2) ? 1 : 0;
+  if (M1 > 1) q = (2 * q + 1 < M1 && (lc & 4)) ? 2 * q + 1 : 2 * q;
+  if (R > 1) q = (2 * q + 1 < R && (lc & 8)) ? 2 * q + 1 : 2 * q;
+  return q;
+}
+
+// Householder reduction of an n x n symmetric matrix, n <= kFullN, with the
+// whole matrix (both triangles) in registers: thread (lr, lc) = (tid / 16,
+// tid % 16) of 512 owns the elements (32 TI + lr, 16 TJ + lc), 72 doubles.
+// The indices are right-aligned (local index = global + kFullN - n), so that
+// the last tiles are always full and one code sequence serves every n.
+//
+// Holding both triangles doubles the multiply-adds of a triangle, but every
+// row of the product then ends inside the 16 lanes of one DPP row: no partial
+// sum crosses wavefronts and a step needs two barriers instead of four.
+//   1. (column k published in xb) A u is formed row by row; the 16 lanes of a
+//      DPP row hold every column of u, so the norm of u and later u.p are row
+//      sums too.  Only the entry k+1 of the reflector depends on the norm: its
+//      column tile is multiplied last.  p = A u goes to pb.
+//   2. (barrier) A -= beta u p^T + (beta p - beta^2 (u.p) u) u^T with
+//      H = I - beta u u^T, u unnormalized; the owners of column k+1 publish it
+//      (barrier).
+// The steps run in twelve phases of 16, phase E with the row and column tiles
+// below column 16 E dropped at compile time.
+//
+// Bound: the latency and instruction issue of one step (LDS round trips, row
+// sums, reciprocal square roots, two barriers), about 0.75 us at 122 AOs.
+// Measured against the triangle with four barriers a step (and the last 64
+// columns on one wavefront): k_tridiag 233 -> 95 us for one system of 122 AOs,
+// 648 -> 397 us a round for 512 systems of 14-235 AOs.
+constexpr int kFullTI = kFullN / 32, kFullTJ = kFullN / 16;
+constexpr double kTinyNorm = 1e-290;  // squared norms below it: already reduced
+
+// column L of the local matrix (L in column tile TJ) goes to xb, zero above the
+// subdiagonal, and its diagonal entry to d
+template <int TJ>
+__device__ __forceinline__ void full_publish(const double (&a)[kFullTI][kFullTJ], int lr, int lc, int L, double* dL,
+                                             double* xb) {
+  if (lc == (L & 15)) {
+    static_for<TJ / 2, kFullTI>([&](auto CI) __attribute__((always_inline)) {
+      constexpr int TI = decltype(CI)::value;
+      const int row = 32 * TI + lr;
+      if constexpr (TI == TJ / 2) {
+        xb[row] = row > L ? a[TI][TJ] : 0.0;
+        if (row == L) *dL = a[TI][TJ];
+      } else {
+        xb[row] = a[TI][TJ];
+      }
+    });
+  }
+}
+
+// the reflectors k with k + 1 in column tile E
+template <int E>
+__device__ __forceinline__ void full_phase(double (&a)[kFullTI][kFullTJ], int& k, double* A, int64_t ld, int off,
+                                           double* d, double* e, double* xb, double* pb) {
+  constexpr int T0 = E / 2, R = kFullTI - T0;  // live row tiles
+  const int tid = threadIdx.x, lc = tid & 15, lr = tid >> 4;
+  const bool first = __builtin_amdgcn_readfirstlane(tid) < kFullN;  // a wavefront with rows tid < kFullN
+  const int prow = 32 * (T0 + row16_index<R>(lc)) + lr;  // the row whose sum this lane ends with
+  for (; k < 16 * E + 15 && k + 2 < kFullN; ++k) {
+    double uj[kFullTJ], ui[kFullTI], p[R];
+    const double x0 = xb[k + 1];
+#pragma unroll
+    for (int TJ = E; TJ < kFullTJ; ++TJ) uj[TJ] = xb[16 * TJ + lc];
+#pragma unroll
+    for (int TI = T0; TI < kFullTI; ++TI) ui[TI] = xb[32 * TI + lr];
+    const bool at_j = 16 * E + lc == k + 1, at_i = 32 * T0 + lr == k + 1;
+    const double xe = at_j ? 0.0 : uj[E];
+    double part = xe * xe;
+#pragma unroll
+    for (int TJ = E + 1; TJ < kFullTJ; ++TJ) part = fma(uj[TJ], uj[TJ], part);
+    const double tail = row16_sum(part);
+    const double ss = fma(x0, x0, tail);
+    const bool noref = tail == 0.0 || ss < kTinyNorm;  // already reduced: inv = beta = 0
+    const double xn = ss * rsqrt_refined(fmax(ss, kTinyNorm));
+    const double alpha = x0 >= 0.0 ? -xn : xn;
+    const double v0 = x0 - alpha;
+#pragma unroll
+    for (int q = 0; q < R; ++q) p[q] = 0.0;
+    static_for<E + 1, kFullTJ>([&](auto CJ) __attribute__((always_inline)) {
+      constexpr int TJ = decltype(CJ)::value;
+#pragma unroll
+      for (int q = 0; q < R; ++q) p[q] = fma(a[T0 + q][TJ], uj[TJ], p[q]);
+    });
+    uj[E] = at_j ? v0 : uj[E];
+    ui[T0] = at_i ? v0 : ui[T0];
+#pragma unroll
+    for (int q = 0; q < R; ++q) p[q] = fma(a[T0 + q][E], uj[E], p[q]);
+    pb[prow] = row16_sums<R>(p, lc);
+    // the unit reflector for the back-transformation (zero for no reflection)
+    const double inv = noref ? 0.0 : rsqrt_refined(fmax(fma(v0, v0, tail), kTinyNorm));
+    if (first) {
+      if (tid > k) A[(tid - off) + (int64_t)(k - off) * ld] = (tid == k + 1 ? v0 : xb[tid]) * inv;
+      if (tid == 0) e[k - off] = noref ? x0 : alpha;
+    }
+    const double beta = 2.0 * (inv * inv);
+    __syncthreads();
+    double pj[kFullTJ], pi[kFullTI];
+#pragma unroll
+    for (int TJ = E; TJ < kFullTJ; ++TJ) pj[TJ] = pb[16 * TJ + lc];
+#pragma unroll
+    for (int TI = T0; TI < kFullTI; ++TI) pi[TI] = pb[32 * TI + lr];
+    double kp = uj[E] * pj[E];
+#pragma unroll
+    for (int TJ = E + 1; TJ < kFullTJ; ++TJ) kp = fma(uj[TJ], pj[TJ], kp);
+    const double bK = beta * row16_sum(kp);
+    double bu[kFullTI], rf[kFullTI];
+#pragma unroll
+    for (int TI = T0; TI < kFullTI; ++TI) {
+      bu[TI] = -beta * ui[TI];
+      static_for<E, kFullTJ>([&](auto CJ) __attribute__((always_inline)) {
+        constexpr int TJ = decltype(CJ)::value;
+        a[TI][TJ] = fma(bu[TI], pj[TJ], a[TI][TJ]);
+      });
+    }
+#pragma unroll
+    for (int TI = T0; TI < kFullTI; ++TI) {
+      rf[TI] = -beta * fma(-bK, ui[TI], pi[TI]);
+      static_for<E, kFullTJ>([&](auto CJ) __attribute__((always_inline)) {
+        constexpr int TJ = decltype(CJ)::value;
+        a[TI][TJ] = fma(rf[TI], uj[TJ], a[TI][TJ]);
+      });
+    }
+    full_publish<E>(a, lr, lc, k + 1, d + (k + 1 - off), xb);
+    __syncthreads();
+  }
+}
+
+// A (leading dimension ld) is read whole; on return its column k holds the unit
+// reflector k below the diagonal.  xb and pb hold kFullN doubles.
+__device__ __forceinline__ void tridiag_full(double* A, int64_t ld, int n, double* d, double* e, double* xb,
+                                             double* pb) {
+  const int tid = threadIdx.x, lc = tid & 15, lr = tid >> 4;
+  const int off = kFullN - n;
+  double a[kFullTI][kFullTJ];
+  static_for<0, kFullTI>([&](auto CI) __attribute__((always_inline)) {
+    constexpr int TI = decltype(CI)::value;
+    const int row = 32 * TI + lr - off;
+#pragma unroll
+    for (int TJ = 0; TJ < kFullTJ; ++TJ) a[TI][TJ] = 0.0;
+    if (32 * TI + 31 >= off) {  // small systems: only the tiles they reach
+      static_for<0, kFullTJ>([&](auto CJ) __attribute__((always_inline)) {
+        constexpr int TJ = decltype(CJ)::value;
+        const int col = 16 * TJ + lc - off;
+        if (row >= 0 && col >= 0) a[TI][TJ] = A[col + row * ld];
+      });
+    }
+    // keep one row tile of loads in flight (address registers would spill the matrix)
+    __builtin_amdgcn_sched_barrier(0);
+  });
+  // every wavefront's loads are done before the first reflector is stored to A
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (tid < kFullN) {
+    xb[tid] = 0.0;
+    pb[tid] = 0.0;
+  }
   __syncthreads();
+  static_for<0, kFullTJ>([&](auto CJ) __attribute__((always_inline)) {
+    constexpr int TJ = decltype(CJ)::value;
+    if (TJ == off >> 4) full_publish<TJ>(a, lr, lc, off, d, xb);
+  });
+  __syncthreads();
+  int k = off;
+  static_for<0, kFullTJ>([&](auto CE) __attribute__((always_inline)) {
+    full_phase<decltype(CE)::value>(a, k, A, ld, off, d, e, xb, pb);
+  });
+  if (lr == 31 && lc == 15) d[n - 1] = a[kFullTI - 1][kFullTJ - 1];
+  if (tid == 0) {
+    if (n >= 2) e[n - 2] = xb[kFullN - 1];
+    e[n - 1] = 0.0;
+  }
 }
 
 // The back-transformation applies the reflectors in compact WY blocks of
@@ -1138,9 +1219,9 @@ __device__ __forceinline__ void wy_factors(const double* A, int n, double* Ts, d
   __syncthreads();
 }
 
-// 512 threads per system (two waves per SIMD, 256 VGPRs per thread): the
-// register reduction for n <= 256, the global-memory one otherwise (the host
-// launches the systems of at most 256 AOs only)
+// n <= 256, 512 threads per system (two waves per SIMD, 256 VGPRs per thread):
+// the columns before the last kFullN from the triangle in registers, the rest
+// with both triangles.
 __global__ __launch_bounds__(512) void k_tridiag(Topo t, const int* order, double* Aall, double* dall,
                                                  double* eall, double* Tall,
                                                  const unsigned char* active) {
@@ -1150,21 +1231,20 @@ __global__ __launch_bounds__(512) void k_tridiag(Topo t, const int* order, doubl
   double* A = Aall + t.mat_off[s];  // column-major view of the symmetric matrix
   double* d = dall + t.ao_off[s];
   double* e = eall + t.ao_off[s];
-  __shared__ double v[kMaxAO];
-  __shared__ double pq[kMaxAO];
-  __shared__ double col[512];  // published column of the register path
+  __shared__ double v[512];
+  __shared__ double pq[512];
+  __shared__ double col[512];  // published column of the triangle
   __shared__ double rowpart[32 * kTriPad];
   __shared__ double colpart[16 * kTriPad];
-  __shared__ double red[16];
-  __shared__ double bc[2];
-  if (n <= 64) tridiag_registers<4>(A, n, d, e, v, col, pq, rowpart, colpart);
-  else if (n <= 128) tridiag_registers<8>(A, n, d, e, v, col, pq, rowpart, colpart);
-  else if (n <= 192) tridiag_registers<12>(A, n, d, e, v, col, pq, rowpart, colpart);
-  else if (n <= 256) tridiag_registers<16>(A, n, d, e, v, col, pq, rowpart, colpart);
-  else tridiag_global(A, n, d, e, v, pq, red, bc);
+  int k0 = 0;
+  if (n > kFullN) {
+    tridiag_registers<16>(A, n, d, e, v, col, pq, rowpart, colpart);
+    k0 = n - kFullN;
+  }
+  tridiag_full(A + k0 + (int64_t)k0 * n, n, n - k0, d + k0, e + k0, v, pq);
   // WY factors for the register back-transformation (n <= 256); the stored
   // reflectors must be visible to the whole block first
-  if (n <= 256 && n > 2) {
+  if (n > 2) {
     __syncthreads();
     wy_factors<0>(A, n, Tall + wy_offset(t, s), rowpart);
   }
