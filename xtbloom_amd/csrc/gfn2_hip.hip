@@ -386,7 +386,6 @@ struct Device {
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
   hipEvent_t round_ev[2] = {nullptr, nullptr};  // end of the SCC rounds of each parity
   std::vector<hipEvent_t> probe_pool;  // per-launch timing events, grow-only
-  size_t lds_limit = 65536;            // dynamic LDS granted to the back-transformation
   // grow-only pinned staging: [0, 256) the per-round active count, then the
   // call's host-to-device uploads (pinned, so each copy is a plain async DMA)
   char* pinned = nullptr;
@@ -452,15 +451,6 @@ Device* device_create(int device_id, void* stream, std::string& error) {
   for (int i = 0; i < 4 && ok; ++i) ok = hipEventCreate(&d->ev[i]) == hipSuccess;
   for (int i = 0; i < 2 && ok; ++i)
     ok = hipEventCreateWithFlags(&d->round_ev[i], hipEventDisableTiming) == hipSuccess;
-  // gfx950 grants up to 160 KB of LDS to one workgroup; opt the back-transformations in
-  int lds = 0;
-  if (ok && hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device_id) == hipSuccess &&
-      lds > 65536 &&
-      hipFuncSetAttribute((const void*)k_backtransform, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          lds - (int)kBackStaticLds) == hipSuccess &&
-      hipFuncSetAttribute((const void*)k_backtransform_wy<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          lds) == hipSuccess)
-    d->lds_limit = (size_t)lds;
   if (!ok) {
     error = "failed to allocate or upload the device parameter tables";
     device_destroy(d);
@@ -617,10 +607,11 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
   std::vector<BackTask> back;
   std::vector<FockTile> chunks;
   std::vector<int64_t> part_off(B + 1, 0);
-  size_t back_lds = 0, back_lds_xl = 0;  // dynamic LDS of k_backtransform_wy, <false> and <true>
   int n_large = 0;  // systems above 256 AOs (a prefix of the size order)
   int n_xl = 0;     // systems above kMaxAO AOs (a prefix of that prefix)
-  size_t n_back_large = 0, n_back_xl = 0;  // their back-transformation tasks (prefixes of `back`)
+  // back-transformation tasks of the systems above 2048, 1024, 512 and 256 AOs
+  // (prefixes of `back`)
+  size_t n_back[4] = {0, 0, 0, 0};
   for (int i = 0; i < B; ++i) {
     const int s = T.order[i];
     const int n = T.ao_off[s + 1] - T.ao_off[s];
@@ -632,23 +623,15 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
         full.push_back({s, a, b});
         if (a >= b) lower.push_back({s, a, b});
       }
-    int cw = 64;  // columns per task: register path (n <= 256), WY path in place (n > kMaxAO)
-    if (n > 256 && n <= kMaxAO) {
-      while (cw > 4 && backtransform_wy_lds(n, cw, false) > dev->lds_limit) cw /= 2;
-      if (backtransform_wy_lds(n, cw, false) > dev->lds_limit) {
-        error = "the device grants too little LDS for the back-transformation";
-        return 6;
-      }
-      back_lds = std::max(back_lds, backtransform_wy_lds(n, cw, false));
-    } else if (n > kMaxAO) {
-      back_lds_xl = backtransform_wy_lds(n, cw, true);
-    }
-    for (int j0 = 0; j0 < n; j0 += cw) back.push_back({s, j0, cw, 0});
-    if (n > kMaxAO) n_back_xl = back.size();
-    if (n > 256) n_back_large = back.size();
+    for (int j0 = 0; j0 < n; j0 += n > 256 ? kWyCols : kBackCols) back.push_back({s, j0});
+    for (int c = 0; c < 4; ++c)
+      if (n > 2048 >> c) n_back[c] = back.size();
     for (int r0 = 0; r0 < n; r0 += kFockTile)
       for (int c0 = r0; c0 < n; c0 += kFockTile) chunks.push_back({s, r0, c0});
   }
+  // WY blocks of the largest system, in groups of eight (k_wy_factors)
+  const unsigned wy_groups =
+      n_large > 0 ? (unsigned)((T.ao_off[T.order[0] + 1] - T.ao_off[T.order[0]] - 2 + 8 * kWyBlock - 1) / (8 * kWyBlock)) : 0;
   // systems split by whether any shell is a d shell: [0] s/p only, [1] with d;
   // per class the prefix of ordered shell pairs and of ordered atom pairs
   std::vector<int> cls_sys[2];
@@ -715,7 +698,7 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
   addd(3 * (size_t)N); addd(6 * (size_t)N);
   for (int k = 0; k < 5; ++k) addd(NAO);  // eps fa fb occ fe
   addd(NAO); addd(NAO);                   // tridiagonal d and e
-  addd((size_t)kBackChunk * NAO + (size_t)kBackChunk * kBackChunk * B);  // WY factors (wy_offset)
+  addd((size_t)kWyPerAO * NAO + (size_t)kWyPerSys * B);  // WY factors (wy_offset)
   addd(B);                                // per-system eigenvalue change of the last round
   addd(NAO);                              // eigenvector normalization factors
   addd((size_t)NAO * 10);      // mulliken column partials
@@ -946,7 +929,7 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
   double* d_shift = cv.take<double>(B);
   double* d_zscale = cv.take<double>(NAO);
   double* d_td = cv.take<double>(NAO);
-  double* d_wyT = cv.take<double>((size_t)kBackChunk * NAO + (size_t)kBackChunk * kBackChunk * B);
+  double* d_wyT = cv.take<double>((size_t)kWyPerAO * NAO + (size_t)kWyPerSys * B);
   double* d_te = cv.take<double>(NAO);
   double* d_colsum = cv.take<double>((size_t)NAO * 10);
   MixerArrays mx{};
@@ -1263,24 +1246,23 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
                        EigenScratch{dT, dH, dC, dP, dW}, d_zscale, co);
     HIP_TRY(probe_end(kKTridiagEigen, 0.0, 0.0));
     HIP_TRY(probe_begin(kKBacktransform));
-    // systems above 256 AOs: the WY factors of their reflectors, then the WY
-    // back-transformation (in place in Y above kMaxAO); the rest: registers
-    if (n_xl > 0)
-      hipLaunchKernelGGL(k_wy_factors<true>, dim3(n_xl), dim3(512), 0, sm, t, d_order, dA, d_wyT, d_active,
-                         d_xl);
-    if (n_large > n_xl)
-      hipLaunchKernelGGL(k_wy_factors<false>, dim3(n_large - n_xl), dim3(512), 0, sm, t, d_order + n_xl, dA,
-                         d_wyT, d_active, d_xl);
-    if (n_back_xl > 0)
-      hipLaunchKernelGGL(k_backtransform_wy<true>, dim3((unsigned)n_back_xl), dim3(kWyThreads), back_lds_xl, sm,
-                         t, d_back, dA, dZ, d_wyT, dY, d_kocc, d_zscale, d_active);
-    if (n_back_large > n_back_xl)
-      hipLaunchKernelGGL(k_backtransform_wy<false>, dim3((unsigned)(n_back_large - n_back_xl)),
-                         dim3(kWyThreads), back_lds, sm, t, d_back + n_back_xl, dA, dZ, d_wyT, dY, d_kocc,
-                         d_zscale, d_active);
-    if (back.size() > n_back_large)
-      hipLaunchKernelGGL(k_backtransform, dim3((unsigned)(back.size() - n_back_large)), dim3(kBackThreads), 0,
-                         sm, t, d_back + n_back_large, dA, dZ, d_wyT, dY, d_kocc, d_zscale, d_active);
+    // systems above 256 AOs: the WY factors of their reflectors, then one
+    // launch per number of row tiles a wavefront holds
+    if (n_large > 0)
+      hipLaunchKernelGGL(k_wy_factors, dim3(n_large, wy_groups), dim3(512), 0, sm, t, d_order, dA, d_wyT,
+                         d_active);
+    auto back_wy = [&](auto* kernel, size_t first, size_t end) {
+      if (end > first)
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(end - first)), dim3(kWyThreads), 0, sm, t, d_back + first, dA,
+                           dZ, d_wyT, dY, d_kocc, d_zscale, d_active);
+    };
+    back_wy(k_backtransform_wy<0>, 0, n_back[0]);
+    back_wy(k_backtransform_wy<16>, n_back[0], n_back[1]);
+    back_wy(k_backtransform_wy<8>, n_back[1], n_back[2]);
+    back_wy(k_backtransform_wy<4>, n_back[2], n_back[3]);
+    if (back.size() > n_back[3])
+      hipLaunchKernelGGL(k_backtransform, dim3((unsigned)(back.size() - n_back[3])), dim3(kBackThreads), 0, sm, t,
+                         d_back + n_back[3], dA, dZ, d_wyT, dY, d_kocc, d_zscale, d_active);
     HIP_TRY(probe_end(kKBacktransform, 0.0, 0.0));
     if (rp) rp->bt = last_probe();
     // C = X Y (the kocc leading columns), P = C diag(f) C^T

@@ -323,8 +323,8 @@ __device__ void cholesky_global(const double* Sm, double* L, double* Xm, int n, 
 //                     tridiagonal LU (one thread per cluster of close eigenvalues,
 //                     modified Gram-Schmidt inside a cluster).  Eigenvalues are
 //                     ranked ascending (ties by index).
-//   k_backtransform   Y = Q Z on column blocks staged in LDS, many blocks per
-//                     system; column j of Z lands in column rank[j] of Y.
+//   k_backtransform   Y = Q Z on column blocks, many blocks per system, on the
+//                     matrix cores (k_backtransform_wy above 256 AOs).
 // Layouts: Z and Y are row-major (row i = component i, column j = vector j).
 // ---------------------------------------------------------------------------
 constexpr double kEps = 2.220446049250313e-16;
@@ -1148,75 +1148,59 @@ __device__ __forceinline__ void tridiag_full(double* A, int64_t ld, int n, doubl
 }
 
 // The back-transformation applies the reflectors in compact WY blocks of
-// kBackChunk:  H_{k_7} ... H_{k_0} = I - V T V^T,  V = [v_{k_0} .. v_{k_7}],
-// k_u = n-3 - ch kBackChunk - u, T lower triangular with
-//   T_mm = 2,  T_mi = -2 sum_{l=i}^{m-1} (v_m . v_l) T_li  (i < m),
-// which follows from H_m (I - V T V^T) = I - [V v_m] [[T, 0], [-2 v_m^T V T, 2]] [V v_m]^T.
-// T_mi of block ch sits at Tall[wy_offset + 64 ch + 8 m + i]; a system holds
-// ceil((n-2)/8) blocks of 64 entries, at most 8 n + 40.
-constexpr int kBackChunk = 8;  // reflectors per WY block
+// kWyBlock:  H_{k_15} ... H_{k_0} = I - V T V^T,  V = [v_{k_0} .. v_{k_15}],
+// k_u = n-3 - 16 ch - u, unit v, T lower triangular with
+//   T_mm = 2,  T_mc = -2 sum_{l=c}^{m-1} (v_m . v_l) T_lc  (c < m),
+// the inverse of 1/2 on the diagonal and the inner products below it.  Block
+// ch's entries below the diagonal sit packed by rows at wy_offset + 120 ch
+// (row m at m (m - 1) / 2); the last block holds the rows it has.  A system
+// needs at most 7.5 n doubles.
+constexpr int kWyBlock = 16;  // reflectors per WY block, one matrix-core tile
+constexpr int kWyPacked = kWyBlock * (kWyBlock - 1) / 2;
+constexpr int kWyPerAO = 8, kWyPerSys = 64;  // doubles reserved
 __device__ __forceinline__ int64_t wy_offset(const Topo& t, int s) {
-  return (int64_t)kBackChunk * t.ao_off[s] + (int64_t)kBackChunk * kBackChunk * s;
+  return (int64_t)kWyPerAO * t.ao_off[s] + (int64_t)kWyPerSys * s;
 }
 
-// T factors of all WY blocks of one system from its stored reflectors (A's
-// strict lower part, column k = reflector k), by the whole block: one thread
-// per (block, pair) inner product over rows > k_i (where both reflectors live),
-// then one thread per block runs the recurrence.  gsh holds 28 doubles per block.
-// (Each caller takes its own instance: a second caller of one instance changes
-// the register kernel's register allocation.)
-template <int INSTANCE>
-__device__ __forceinline__ void wy_factors(const double* A, int n, double* Ts, double* gsh) {
-  constexpr int kPairs = kBackChunk * (kBackChunk - 1) / 2;  // 28
-  const int tid = threadIdx.x, nt = blockDim.x;
-  const int nref = n - 2, nch = (nref + kBackChunk - 1) / kBackChunk;
-  for (int task = tid; task < nch * kPairs; task += nt) {
-    const int ch = task / kPairs;
-    int p = task - ch * kPairs, m = 1, i = 0;
-    while (p > 0) {
-      --p;
-      if (++i == m) { ++m; i = 0; }
-    }
-    const int kb = n - 3 - ch * kBackChunk, km = kb - m, ki = kb - i;
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    if (km >= 0) {
-      const double* vm = A + (int64_t)km * n;
-      const double* vi = A + (int64_t)ki * n;
-      int r = ki + 1;
-      for (; r + 3 < n; r += 4) {
+// T factor of block ch by one wavefront: the inner products V^T V on the matrix
+// cores (both operands of a step are the same registers), then lane c < 16 runs
+// the recurrence of column c.  g: 256 doubles of LDS of this wavefront's own.
+__device__ __forceinline__ void wy_factor(const double* A, int n, int ch, double* Ts, double* g) {
+  const int lane = threadIdx.x & 63, l16 = lane & 15, lk = lane >> 4;
+  const int kb = n - 3 - kWyBlock * ch, cnt = min(kWyBlock, kb + 1);
+  const int ku = kb - l16;  // this lane's reflector
+  const double* v = A + (int64_t)max(ku, 0) * n;
+  mfma_d4 acc[2] = {mfma_d4{0.0, 0.0, 0.0, 0.0}, mfma_d4{0.0, 0.0, 0.0, 0.0}};
+  for (int r0 = max(kb - (kWyBlock - 1), 0) + 1; r0 < n; r0 += 32) {
+    double x[8];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) acc[u] = fma(vm[r + u], vi[r + u], acc[u]);
-      }
-      for (; r < n; ++r) acc[0] = fma(vm[r], vi[r], acc[0]);
+    for (int q = 0; q < 8; ++q) x[q] = v[min(r0 + 4 * q + lk, n - 1)];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int r = r0 + 4 * q + lk;
+      const double xm = (ku >= 0 && r > ku && r < n) ? x[q] : 0.0;
+      acc[q & 1] = mfma_16x16x4(xm, xm, acc[q & 1]);
     }
-    gsh[task] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
   }
-  __syncthreads();
-  for (int ch = tid; ch < nch; ch += nt) {
-    const int kb = n - 3 - ch * kBackChunk;
-    const double* g = gsh + ch * kPairs;  // (v_m . v_l) at m (m-1) / 2 + l
-    double T[kBackChunk][kBackChunk];
 #pragma unroll
-    for (int m = 0; m < kBackChunk; ++m) {
+  for (int r = 0; r < 4; ++r) g[(lk + 4 * r) * kWyBlock + l16] = acc[0][r] + acc[1][r];
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  if (lane < kWyBlock) {
+    double* To = Ts + (int64_t)kWyPacked * ch;
+    double tc[kWyBlock];
 #pragma unroll
-      for (int i = 0; i < kBackChunk; ++i) T[m][i] = 0.0;
-      if (kb - m < 0) continue;  // past the last reflector: zero row
-      T[m][m] = 2.0;
+    for (int m = 0; m < kWyBlock; ++m) {
+      double s0 = 0.0, s1 = 0.0;  // tc[l] = 0 for l < c
 #pragma unroll
-      for (int i = 0; i < m; ++i) {
-        double acc = 0.0;
-#pragma unroll
-        for (int l = i; l < m; ++l) acc = fma(g[m * (m - 1) / 2 + l], T[l][i], acc);
-        T[m][i] = -2.0 * acc;
+      for (int l = 0; l < m; ++l) {
+        if (l & 1) s1 = fma(g[m * kWyBlock + l], tc[l], s1);
+        else s0 = fma(g[m * kWyBlock + l], tc[l], s0);
       }
+      tc[m] = m == lane ? 2.0 : -2.0 * (s0 + s1);
+      if (m > lane && m < cnt) To[m * (m - 1) / 2 + lane] = tc[m];
     }
-    double* To = Ts + ch * kBackChunk * kBackChunk;
-#pragma unroll
-    for (int m = 0; m < kBackChunk; ++m)
-#pragma unroll
-      for (int i = 0; i < kBackChunk; ++i) To[m * kBackChunk + i] = T[m][i];
   }
-  __syncthreads();
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 }
 
 // n <= 256, 512 threads per system (two waves per SIMD, 256 VGPRs per thread):
@@ -1242,12 +1226,12 @@ __global__ __launch_bounds__(512) void k_tridiag(Topo t, const int* order, doubl
     k0 = n - kFullN;
   }
   tridiag_full(A + k0 + (int64_t)k0 * n, n, n - k0, d + k0, e + k0, v, pq);
-  // WY factors for the register back-transformation (n <= 256); the stored
-  // reflectors must be visible to the whole block first
-  if (n > 2) {
-    __syncthreads();
-    wy_factors<0>(A, n, Tall + wy_offset(t, s), rowpart);
-  }
+  // WY factors for the back-transformation; the stored reflectors must be
+  // visible to the whole block first
+  __syncthreads();
+  const int wv = threadIdx.x >> 6;
+  for (int ch = wv; kWyBlock * ch < n - 2; ch += 8)
+    wy_factor(A, n, ch, Tall + wy_offset(t, s), rowpart + 256 * wv);
 }
 
 // n > 256: the blocked reduction, one 512-thread block per system (the host
@@ -2910,247 +2894,48 @@ __global__ __launch_bounds__(256) void k_cluster_vectors(Topo t, const int* orde
 
 // One column block of one system: Y[:, j0 .. j0+cw) = Q Z[:, j0 .. j0+cw), for
 // the columns below the system's kocc (Z holds eigenvectors by ascending rank).
+// One block's columns of the back-transformation.
 struct BackTask {
   int sys;
   int j0;
-  int cw;
-  int pad;
 };
 
-// 512 threads.  n <= 256: the 64-column block lives in registers (thread
-// (c, rg) = (tid % 64, tid / 64) holds rows rg, rg + 8, ...) and the
-// reflectors are applied kBackChunk at a time in compact WY form,
-//   H_{k_7} ... H_{k_0} = I - V T V^T,   V = [v_{k_0} .. v_{k_7}],
-// with k_u = n-3 - ch kBackChunk - u and T lower triangular (wy_factors):
-// one LDS reduction (V^T z for the whole chunk) and two barriers per chunk.
-// Reflectors are staged in LDS zero-padded to absolute row indices, so every
-// thread applies every reflector without masks; the next chunk is fetched into
-// registers while the current one is applied.  n > 256: the column block lives
-// in dynamic LDS ((n cw + 2 n + 512) doubles) and reflectors are applied one at
-// a time.
-constexpr int kBackThreads = 512;
-constexpr int kBackRegRows = 32;  // rows per thread of the register path (n <= 256)
-constexpr size_t kBackStaticLds =
-    (2 * kBackChunk * 256 + kBackChunk * kBackThreads + kBackChunk * 64) * sizeof(double);
-
-__device__ __forceinline__ void backtransform_registers(const double* __restrict__ A,
-                                                        const double* __restrict__ Z,
-                                                        const double* __restrict__ Tf,
-                                                        double* __restrict__ Y, int kocc,
-                                                        const double* zscale, int n, int j0,
-                                                        double* ring, double* part, double* wf) {
-  // thread (w, cg, rl): wavefront w, column group cg = lane / 4 (columns
-  // j0 + 4 cg + j, j < 4), row lane rl = lane % 4; rows rgp + 32 q (q < 8) with
-  // rgp = 4 w + rl.  Each reflector entry read from LDS feeds four columns.
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int cg = lane >> 2, rl = lane & 3, rgp = 4 * w + rl;
-  constexpr int kRows = 8, kCols = 4;
-  double z[kRows][kCols];
-#pragma unroll
-  for (int j = 0; j < kCols; ++j) {
-    const int c = j0 + kCols * cg + j;
-    const bool ok = c < kocc;
-    const double f = ok ? zscale[c] : 0.0;
-#pragma unroll
-    for (int q = 0; q < kRows; ++q) {
-      const int i = rgp + 32 * q;
-      z[q][j] = (ok && i < n) ? f * Z[(int64_t)i * n + c] : 0.0;
-    }
-  }
-  // chunk ch holds k = n-3 - ch*kBackChunk - u at ring slot
-  // ((ch & 1) * kBackChunk + u) * 256, zero-padded to absolute rows; its T
-  // factor at Tf[64 ch].
-  constexpr int kVals = kBackChunk * 256 / kBackThreads;
-  constexpr int kTT = kBackChunk * kBackChunk;
-  auto fetch = [&](int ch, double (&r)[kVals]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int v = 0; v < kVals; ++v) {
-      const int x = tid + kBackThreads * v, u = x >> 8, i = x & 255;
-      const int k = n - 3 - ch * kBackChunk - u;
-      r[v] = (k >= 0 && i > k && i < n) ? A[i + (int64_t)k * n] : 0.0;
-    }
-  };
-  auto stage = [&](int ch, const double (&r)[kVals]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int v = 0; v < kVals; ++v) ring[(ch & 1) * kBackChunk * 256 + tid + kBackThreads * v] = r[v];
-  };
-  const int nref = n - 2;  // reflectors k = 0 .. n-3
-  double rn[kVals];
-  if (nref > 0) {
-    fetch(0, rn);
-    stage(0, rn);
-  }
-  __syncthreads();
-  for (int ch = 0; ch * kBackChunk < nref; ++ch) {
-    const bool more = (ch + 1) * kBackChunk < nref;
-    if (more) fetch(ch + 1, rn);  // in flight while this chunk is applied
-    const double* hv = ring + (ch & 1) * kBackChunk * 256;
-    // T is read-only and wave-uniform: the constant address space puts it in
-    // SGPRs through scalar loads
-    const __attribute__((address_space(4))) double* tt =
-        (const __attribute__((address_space(4))) double*)(Tf + ch * kTT);
-    // V^T z: per reflector, this thread's rows, summed over the four row lanes
-    // of the column group (DPP quad permutations), then over the wavefronts
-#pragma unroll
-    for (int u = 0; u < kBackChunk; ++u) {
-      double p[kCols] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int q = 0; q < kRows; ++q) {
-        const double h = hv[u * 256 + rgp + 32 * q];
-#pragma unroll
-        for (int j = 0; j < kCols; ++j) p[j] = fma(h, z[q][j], p[j]);
-      }
-#pragma unroll
-      for (int j = 0; j < kCols; ++j) {
-        p[j] += dpp_move<0xb1, 0xf>(p[j]);  // lanes 0<->1, 2<->3
-        p[j] += dpp_move<0x4e, 0xf>(p[j]);  // lanes 0<->2, 1<->3
-      }
-      if (rl == 0) {
-#pragma unroll
-        for (int j = 0; j < kCols; ++j) part[(u * 8 + w) * 64 + kCols * cg + j] = p[j];
-      }
-    }
-    __syncthreads();
-    // w = V^T z for reflector u, column c (thread (u, c))
-    const int ur = tid >> 6, cr = tid & 63;
-    {
-      double acc = 0.0;
-#pragma unroll
-      for (int g = 0; g < 8; ++g) acc += part[(ur * 8 + g) * 64 + cr];
-      wf[ur * 64 + cr] = acc;
-    }
-    __syncthreads();
-    // y = T w (T lower triangular), thread (u, c); y goes to part[u][0][c]
-    {
-      double acc = 0.0;
-      for (int i = 0; i <= ur; ++i) acc = fma(tt[ur * kBackChunk + i], wf[i * 64 + cr], acc);
-      part[ur * 8 * 64 + cr] = acc;
-    }
-    __syncthreads();
-    // z -= V y, one reflector at a time (only its four y values live)
-#pragma unroll
-    for (int u = 0; u < kBackChunk; ++u) {
-      double yj[kCols];
-#pragma unroll
-      for (int j = 0; j < kCols; ++j) yj[j] = part[u * 8 * 64 + kCols * cg + j];
-#pragma unroll
-      for (int q = 0; q < kRows; ++q) {
-        const double h = hv[u * 256 + rgp + 32 * q];
-#pragma unroll
-        for (int j = 0; j < kCols; ++j) z[q][j] = fma(-h, yj[j], z[q][j]);
-      }
-      // Empty asm with a memory clobber pins the program order, so that only
-      // this reflector's entries are in flight (hoisting all of them spills).
-#pragma unroll
-      for (int q = 0; q < kRows; ++q)
-        asm volatile("" : "+v"(z[q][0]), "+v"(z[q][1]), "+v"(z[q][2]), "+v"(z[q][3])::"memory");
-    }
-    if (more) stage(ch + 1, rn);
-    __syncthreads();
-  }
-#pragma unroll
-  for (int j = 0; j < kCols; ++j) {
-    const int c = j0 + kCols * cg + j;
-    if (c >= kocc) continue;
-#pragma unroll
-    for (int q = 0; q < kRows; ++q) {
-      const int i = rgp + 32 * q;
-      if (i < n) Y[(int64_t)i * n + c] = z[q][j];
-    }
-  }
+// T[m][u] of a WY block with the packed factor To (u, m < 16); rows past the
+// block's last reflector are never used (their column of V is zero)
+__device__ __forceinline__ double wy_entry(const double* To, int m, int u, int cnt) {
+  const bool low = u < m && m < cnt;
+  const double x = To[low ? m * (m - 1) / 2 + u : 0];
+  return low ? x : (m == u ? 2.0 : 0.0);
 }
 
-__device__ __forceinline__ void backtransform_lds(const double* __restrict__ A,
-                                                  const double* __restrict__ Z,
-                                                  double* __restrict__ Y, int kocc,
-                                                  const double* zscale, int n, int j0, int cw,
-                                                  double* lds) {
-  double* Zb = lds;                 // [n][cw]
-  double* hvb = lds + n * cw;       // [2][n]
-  double* part = hvb + 2 * n;       // [512]
-  const int tid = threadIdx.x, nt = blockDim.x;
-  for (int idx = tid; idx < n * cw; idx += nt) {
-    const int i = idx / cw, c = idx % cw;
-    Zb[idx] = (j0 + c < kocc) ? zscale[j0 + c] * Z[(int64_t)i * n + j0 + c] : 0.0;
-  }
-  const int c = tid % cw, rg = tid / cw, nrg = nt / cw;
-  // reflector k occupies A[k+1 .. n-1, k] (column-major); m = n - k - 1 <= 1023
-  int k = n - 3;
-  if (k >= 0) {
-    double* hv = hvb + (k & 1) * n;
-    for (int i = tid; i < n - k - 1; i += nt) hv[i] = A[(k + 1 + i) + (int64_t)k * n];
-  }
-  __syncthreads();
-  for (; k >= 0; --k) {
-    const int m = n - k - 1;
-    const double* hv = hvb + (k & 1) * n;
-    double r0 = 0.0, r1 = 0.0;
-    const bool more = k >= 1;
-    if (more) {
-      const int kn = k - 1;
-      if (tid < m + 1) r0 = A[(kn + 1 + tid) + (int64_t)kn * n];
-      if (tid + nt < m + 1) r1 = A[(kn + 1 + tid + nt) + (int64_t)kn * n];
-    }
-    double p = 0.0;
-    for (int i = rg; i < m; i += nrg) p += hv[i] * Zb[(k + 1 + i) * cw + c];
-    part[rg * cw + c] = p;
-    __syncthreads();
-    double dot = 0.0;
-    for (int w = 0; w < nrg; ++w) dot += part[w * cw + c];
-    dot *= 2.0;
-    for (int i = rg; i < m; i += nrg) Zb[(k + 1 + i) * cw + c] -= dot * hv[i];
-    if (more) {
-      double* hn = hvb + ((k - 1) & 1) * n;
-      if (tid < m + 1) hn[tid] = r0;
-      if (tid + nt < m + 1) hn[tid + nt] = r1;
-    }
-    __syncthreads();
-  }
-  for (int idx = tid; idx < n * cw; idx += nt) {
-    const int i = idx / cw, cc = idx % cw;
-    if (j0 + cc < kocc) Y[(int64_t)i * n + j0 + cc] = Zb[idx];
-  }
-}
+// Y = Q Z, n <= 256, the occupied columns.  256 threads; each wavefront holds
+// 16 columns whole in registers, tile t = rows 16 t .. 16 t + 15 in the
+// accumulator layout of v_mfma_f64_16x16x4f64 (lane: column lane % 16, rows
+// 16 t + lane / 16 + 4 r).  Register r of tile t is then exactly the B operand
+// of the K step over rows 16 t + 4 r .. + 3, so
+//   w = V^T z,  y = T w,  z -= V y
+// run on the matrix cores with no data moved between lanes or wavefronts.  The
+// block's four wavefronts share the WY block's reflectors, staged in LDS one
+// block ahead (zero on and above their subdiagonal; row stride 260: the 16 x 4
+// operand reads of w spread over all banks): one barrier per 16 reflectors.
+//
+// Bound: FP64 matrix cores (2 n^2 kocc flop, 16 x 16 tiles) for large batches,
+// the serial chain of a wavefront's products for small ones.  Measured against
+// blocks of eight reflectors on the vector units with four block barriers each:
+// 74 -> 34 us for one system of 122 AOs, 314 -> 160 us a round for 512 systems
+// of 14-235 AOs.
+constexpr int kBackThreads = 256;
+constexpr int kBackCols = 64;   // columns of one block
+constexpr int kBackTiles = 16;  // row tiles (n <= 256)
+constexpr int kBackLd = 260;
 
-// T factors of the WY blocks of the systems above 256 AOs (the register
-// reduction forms its own), one 512-thread block per system after the blocked
-// reduction.  BIG (n > kMaxAO): the Gram entries in the system's global slice.
-constexpr int kWyGram = kBackChunk * (kBackChunk - 1) / 2 * ((kMaxAO - 2 + kBackChunk - 1) / kBackChunk);
-template <bool BIG>
-__global__ __launch_bounds__(512) void k_wy_factors(Topo t, const int* order, const double* Aall,
-                                                    double* Tall, const unsigned char* active, double* big) {
-  const int s = order[blockIdx.x];
-  if (active && !active[s]) return;
-  const int n = t.ao_off[s + 1] - t.ao_off[s];
-  __shared__ double gram_l[BIG ? 1 : kWyGram];
-  double* gram = BIG ? big + big_offset(t, s) : gram_l;  // 28 ceil((n-2)/8) <= kBigPerAO n doubles
-  wy_factors<1>(Aall + t.mat_off[s], n, Tall + wy_offset(t, s), gram);
-}
-
-// n > 256: Y = Q Z on a block of cw columns (cw | 64), the reflectors applied
-// kBackChunk at a time in compact WY form with the T factors of k_wy_factors:
-//   w = V^T z, y = T w, z -= V y,
-// four barriers per block of eight reflectors.  Thread (c, g) = (tid % cw,
-// tid / cw) holds column j0 + c, rows i0 + g, i0 + g + 512 / cw, ... of the
-// rows the block touches (i0 = one past its lowest reflector); the dot
-// partials are summed over the row groups of a wavefront by lane exchanges,
-// then over the wavefronts in LDS.
-// Dynamic LDS (doubles): non-BIG, the column block [n][cw], the block's
-// reflectors [8][n] (zero-padded to absolute rows), partials [8][8][cw] and
-// y [8][cw]; BIG (n > kMaxAO), partials and y only: the column block is
-// updated in place in Y and the reflectors are read from A.
-constexpr int kWyThreads = 512;
-__host__ __device__ constexpr size_t backtransform_wy_lds(int n, int cw, bool big) {
-  return ((big ? 0 : (size_t)n * cw + (size_t)kBackChunk * n) + (size_t)kBackChunk * 9 * cw) * sizeof(double);
-}
-
-template <bool BIG>
-__global__ __launch_bounds__(kWyThreads) void k_backtransform_wy(Topo t, const BackTask* tasks,
-                                                                 const double* Aall, const double* Zall,
-                                                                 const double* Tall, double* Yall,
-                                                                 const int* kocc_all, const double* zscale_all,
-                                                                 const unsigned char* active) {
-  extern __shared__ double lds[];
+__global__ __launch_bounds__(kBackThreads, 2) void k_backtransform(Topo t, const BackTask* tasks,
+                                                                   const double* Aall, const double* Zall,
+                                                                   const double* Tall, double* Yall,
+                                                                   const int* kocc_all,
+                                                                   const double* zscale_all,
+                                                                   const unsigned char* active) {
+  __shared__ double vs[2][kWyBlock * kBackLd];
   const BackTask task = tasks[blockIdx.x];
   const int s = task.sys;
   if (active && !active[s]) return;
@@ -3161,117 +2946,276 @@ __global__ __launch_bounds__(kWyThreads) void k_backtransform_wy(Topo t, const B
   const double* __restrict__ A = Aall + mo;
   const double* __restrict__ Z = Zall + mo;
   double* __restrict__ Y = Yall + mo;
-  const double* zscale = zscale_all + t.ao_off[s];
-  const double* Tf = Tall + wy_offset(t, s);
-  const int cw = task.cw, j0 = task.j0;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int c = tid % cw, g = tid / cw, ng = kWyThreads / cw;
-  const int col = j0 + c;
-  const bool on = col < kocc;
-  double* zb = BIG ? Y + j0 : lds;  // z(i, c) at zb[i * ldz + c]
-  const int64_t ldz = BIG ? n : cw;
-  double* vs = lds + (BIG ? 0 : (int64_t)n * cw);          // [8][n]
-  double* part = vs + (BIG ? 0 : (int64_t)kBackChunk * n);  // [8][8][cw]
-  double* yv = part + kBackChunk * 8 * cw;                  // [8][cw]
-  for (int i = g; i < n; i += ng) {
-    const double zv = on ? zscale[col] * Z[(int64_t)i * n + col] : 0.0;
-    if (!BIG || on) zb[i * ldz + c] = zv;
+  const double* __restrict__ Tf = Tall + wy_offset(t, s);
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lk = lane >> 4;
+  const int col = task.j0 + 16 * w + l16;
+  const bool on = col < kocc, live = task.j0 + 16 * w < kocc;  // live: any column of the wavefront
+  const int nt = (n + 15) >> 4;
+  mfma_d4 z[kBackTiles];
+  const double f = on ? zscale_all[t.ao_off[s] + col] : 0.0;
+#pragma unroll
+  for (int i = 0; i < kBackTiles; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 16 * i + lk + 4 * r;
+      z[i][r] = (on && row < n) ? f * Z[(int64_t)row * n + col] : 0.0;
+      if (r == 3 && i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+  double fr[kWyBlock];  // the next block's reflectors, row tid
+  auto fetch = [&](int ch) __attribute__((always_inline)) {
+    const int kb = n - 3 - kWyBlock * ch;
+#pragma unroll
+    for (int u = 0; u < kWyBlock; ++u) {
+      const int k = kb - u;
+      fr[u] = (k >= 0 && tid > k && tid < n) ? A[tid + (int64_t)k * n] : 0.0;
+    }
+  };
+  auto stage = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < kWyBlock; ++u) vs[buf][u * kBackLd + tid] = fr[u];
+  };
+  const int nch = (n - 2 + kWyBlock - 1) / kWyBlock;  // n - 2 reflectors
+  if (nch > 0) {
+    fetch(0);
+    stage(0);
   }
   __syncthreads();
-  const int nref = n - 2;  // reflectors k = 0 .. n-3
-  for (int ch = 0; ch * kBackChunk < nref; ++ch) {
-    const int kb = n - 3 - ch * kBackChunk;  // k_0; k_u = kb - u
-    const int i0 = max(kb - (kBackChunk - 1), 0) + 1;
-    const int m = n - i0;
-    if constexpr (!BIG) {
-      for (int x = tid; x < kBackChunk * m; x += kWyThreads) {
-        const int u = x / m, i = i0 + (x - u * m), k = kb - u;
-        vs[u * n + i] = (k >= 0 && i > k) ? A[i + (int64_t)k * n] : 0.0;
+  for (int ch = 0; ch < nch; ++ch) {
+    const bool more = ch + 1 < nch;
+    if (more) fetch(ch + 1);  // in flight while this block is applied
+    if (live) {
+      const double* hv = vs[ch & 1];
+      const int kb = n - 3 - kWyBlock * ch, cnt = min(kWyBlock, kb + 1);
+      const int t0 = (max(kb - (kWyBlock - 1), 0) + 1) >> 4;  // first row tile the block touches
+      double tt[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) tt[q] = wy_entry(Tf + kWyPacked * ch, l16, 4 * q + lk, cnt);
+      mfma_d4 wa = mfma_d4{0.0, 0.0, 0.0, 0.0}, wb = wa;
+#pragma unroll
+      for (int i = 0; i < kBackTiles; ++i) {
+        if (i >= t0 && i < nt) {
+          double a[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) a[r] = hv[l16 * kBackLd + 16 * i + 4 * r + lk];
+          wa = mfma_16x16x4(a[0], z[i][0], wa);
+          wb = mfma_16x16x4(a[1], z[i][1], wb);
+          wa = mfma_16x16x4(a[2], z[i][2], wa);
+          wb = mfma_16x16x4(a[3], z[i][3], wb);
+        }
       }
-      __syncthreads();
+      mfma_d4 y = mfma_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int q = 0; q < 4; ++q) y = mfma_16x16x4(-tt[q], wa[q] + wb[q], y);
+#pragma unroll
+      for (int i = 0; i < kBackTiles; ++i) {
+        if (i >= t0 && i < nt) {
+          double a[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) a[q] = hv[(4 * q + lk) * kBackLd + 16 * i + l16];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) z[i] = mfma_16x16x4(a[q], y[q], z[i]);
+        }
+      }
     }
-    auto vat = [&](int i, int u) __attribute__((always_inline)) -> double {
-      if constexpr (BIG) {
-        const int k = kb - u;
-        return (k >= 0 && i > k) ? A[i + (int64_t)k * n] : 0.0;
-      } else {
-        return vs[u * n + i];
-      }
-    };
-    double p[kBackChunk];
-#pragma unroll
-    for (int u = 0; u < kBackChunk; ++u) p[u] = 0.0;
-    for (int i = i0 + g; i < n; i += ng) {
-      const double zv = (!BIG || on) ? zb[i * ldz + c] : 0.0;
-#pragma unroll
-      for (int u = 0; u < kBackChunk; ++u) p[u] = fma(vat(i, u), zv, p[u]);
-    }
-    for (int off = cw; off < 64; off <<= 1)
-#pragma unroll
-      for (int u = 0; u < kBackChunk; ++u) p[u] += __shfl_xor(p[u], off, 64);
-    if (lane < cw)
-#pragma unroll
-      for (int u = 0; u < kBackChunk; ++u) part[(u * 8 + w) * cw + c] = p[u];
-    __syncthreads();
-    // y = T w, T lower triangular (thread (u, c))
-    if (tid < kBackChunk * cw) {
-      const int u = tid / cw, cc = tid - u * cw;
-      double acc = 0.0;
-      for (int i = 0; i <= u; ++i) {
-        double wsum = 0.0;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) wsum += part[(i * 8 + q) * cw + cc];
-        acc = fma(Tf[ch * kBackChunk * kBackChunk + u * kBackChunk + i], wsum, acc);
-      }
-      yv[u * cw + cc] = acc;
-    }
-    __syncthreads();
-    double yc[kBackChunk];
-#pragma unroll
-    for (int u = 0; u < kBackChunk; ++u) yc[u] = yv[u * cw + c];
-    if (!BIG || on)
-      for (int i = i0 + g; i < n; i += ng) {
-        double zv = zb[i * ldz + c];
-#pragma unroll
-        for (int u = 0; u < kBackChunk; ++u) zv = fma(-vat(i, u), yc[u], zv);
-        zb[i * ldz + c] = zv;
-      }
+    if (more) stage((ch + 1) & 1);
     __syncthreads();
   }
-  if constexpr (!BIG) {
-    if (on)
-      for (int i = g; i < n; i += ng) Y[(int64_t)i * n + col] = zb[i * cw + c];
+  if (on) {
+#pragma unroll
+    for (int i = 0; i < kBackTiles; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 16 * i + lk + 4 * r;
+        if (row < n) Y[(int64_t)row * n + col] = z[i][r];
+      }
   }
 }
 
-// two blocks per CU (four wavefronts per SIMD): at most 128 VGPRs.  The host
-// sends the column blocks of systems of at most 256 AOs here (the register
-// path) and larger ones to k_backtransform_wy; the LDS branch stays as the
-// kernel's general form.
-__global__ __launch_bounds__(kBackThreads, 4) void k_backtransform(Topo t, const BackTask* tasks,
-                                                                const double* Aall,
-                                                                const double* Zall,
-                                                                const double* Tall, double* Yall,
-                                                                const int* kocc_all,
-                                                                const double* zscale_all,
-                                                                const unsigned char* active) {
-  extern __shared__ double lds[];
-  __shared__ double ring[2 * kBackChunk * 256];
-  __shared__ double part[kBackChunk * kBackThreads];
-  __shared__ double wf[kBackChunk * 64];
+// T factors of the systems above 256 AOs (the register reduction forms its
+// own) after the blocked reduction: blockIdx.y covers eight WY blocks, one per
+// wavefront.
+__global__ __launch_bounds__(512) void k_wy_factors(Topo t, const int* order, const double* Aall,
+                                                    double* Tall, const unsigned char* active) {
+  __shared__ double g[8][kWyBlock * kWyBlock];
+  const int s = order[blockIdx.x];
+  if (active && !active[s]) return;
+  const int n = t.ao_off[s + 1] - t.ao_off[s];
+  const int wv = threadIdx.x >> 6, ch = 8 * blockIdx.y + wv;
+  if (kWyBlock * ch < n - 2) wy_factor(Aall + t.mat_off[s], n, ch, Tall + wy_offset(t, s), g[wv]);
+}
+
+// Y = Q Z, n > 256: the same products on 16 columns, whose row tiles are dealt
+// to the block's eight wavefronts (tile w + 8 q).  The wavefronts' partial w
+// meet in LDS: two barriers per WY block; y is formed redundantly.  Each
+// wavefront reads only the reflector rows of its own tiles, straight from A
+// (issued before the barriers, so that L2's latency overlaps the products).
+// MT row tiles per wavefront in registers (n <= 128 MT); MT = 0 keeps the
+// columns in Y.  Measured against eight reflectors at a time on the vector
+// units: 10.6 -> 0.70 ms at 1142 AOs, 375 -> 81 us for 14 systems of 258-482 AOs.
+constexpr int kWyThreads = 512;
+constexpr int kWyCols = 16;
+
+template <int MT>
+__global__ __launch_bounds__(kWyThreads) void k_backtransform_wy(Topo t, const BackTask* tasks,
+                                                                 const double* Aall, const double* Zall,
+                                                                 const double* Tall, double* Yall,
+                                                                 const int* kocc_all, const double* zscale_all,
+                                                                 const unsigned char* active) {
+  __shared__ double part[8][kWyBlock * kWyCols];
+  __shared__ double wsum[kWyBlock * kWyCols];
   const BackTask task = tasks[blockIdx.x];
   const int s = task.sys;
   if (active && !active[s]) return;
   const int n = t.ao_off[s + 1] - t.ao_off[s];
-  const int64_t mo = t.mat_off[s];
   const int kocc = kocc_all[s];
   if (task.j0 >= kocc) return;
-  const double* zscale = zscale_all + t.ao_off[s];
-  if (n <= 256)
-    backtransform_registers(Aall + mo, Zall + mo, Tall + wy_offset(t, s),
-                            Yall + mo, kocc, zscale, n, task.j0, ring, part, wf);
-  else
-    backtransform_lds(Aall + mo, Zall + mo, Yall + mo, kocc, zscale, n, task.j0, task.cw, lds);
+  const int64_t mo = t.mat_off[s];
+  const double* __restrict__ A = Aall + mo;
+  const double* __restrict__ Z = Zall + mo;
+  double* Y = Yall + mo;
+  const double* __restrict__ Tf = Tall + wy_offset(t, s);
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, lk = lane >> 4;
+  const int col = task.j0 + l16;
+  const bool on = col < kocc;
+  const int nt = (n + 15) >> 4;
+  const double f = on ? zscale_all[t.ao_off[s] + col] : 0.0;
+  constexpr int kQ = MT > 0 ? MT : 1;
+  mfma_d4 z[kQ];
+  auto at = [&](int i, int r) __attribute__((always_inline)) { return (int64_t)(16 * i + lk + 4 * r) * n + col; };
+  if constexpr (MT > 0) {
+#pragma unroll
+    for (int q = 0; q < MT; ++q)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        z[q][r] = (on && 16 * (w + 8 * q) + lk + 4 * r < n) ? f * Z[at(w + 8 * q, r)] : 0.0;
+        if (MT > 8 && r == 3 && q % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      }
+  } else {
+    if (on)
+      for (int i = w; i < nt; i += 8)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (16 * i + lk + 4 * r < n) Y[at(i, r)] = f * Z[at(i, r)];
+  }
+  const int nch = (n - 2 + kWyBlock - 1) / kWyBlock;
+  for (int ch = 0; ch < nch; ++ch) {
+    const int kb = n - 3 - kWyBlock * ch, cnt = min(kWyBlock, kb + 1);
+    const int t0 = (max(kb - (kWyBlock - 1), 0) + 1) >> 4;
+    // operand of w: V[row 16 i + 4 r + lk][u = l16]; of the update:
+    // V[row 16 i + l16][u = 4 q + lk].  Addresses are clamped into A, values masked.
+    const int ku = kb - l16;
+    const double* vu = A + (int64_t)max(ku, 0) * n;
+    auto w_op = [&](int i, double (&a)[4]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) a[r] = vu[min(16 * i + 4 * r + lk, n - 1)];
+    };
+    auto w_mask = [&](int i, double (&a)[4]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 16 * i + 4 * r + lk;
+        a[r] = (ku >= 0 && row > ku && row < n) ? a[r] : 0.0;
+      }
+    };
+    auto u_op = [&](int i, double (&a)[4]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) a[q] = A[min(16 * i + l16, n - 1) + (int64_t)max(kb - (4 * q + lk), 0) * n];
+    };
+    auto u_mask = [&](int i, double (&a)[4]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int k = kb - (4 * q + lk), row = 16 * i + l16;
+        a[q] = (k >= 0 && row > k && row < n) ? a[q] : 0.0;
+      }
+    };
+    double tt[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) tt[q] = wy_entry(Tf + (int64_t)kWyPacked * ch, l16, 4 * q + lk, cnt);
+    mfma_d4 wa = mfma_d4{0.0, 0.0, 0.0, 0.0}, wb = wa;
+    if constexpr (MT > 0) {
+#pragma unroll
+      for (int q = 0; q < MT; ++q) {
+        const int i = w + 8 * q;
+        if (i >= t0 && i < nt) {
+          double a[4];
+          w_op(i, a);
+          w_mask(i, a);
+          wa = mfma_16x16x4(a[0], z[q][0], wa);
+          wb = mfma_16x16x4(a[1], z[q][1], wb);
+          wa = mfma_16x16x4(a[2], z[q][2], wa);
+          wb = mfma_16x16x4(a[3], z[q][3], wb);
+        }
+        if constexpr (MT > 8) {  // loads of four tiles in flight
+          if (q % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    } else {
+      for (int i = t0 + ((w - t0) & 7); i < nt; i += 8) {
+        double a[4], zz[4];
+        w_op(i, a);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) zz[r] = (on && 16 * i + lk + 4 * r < n) ? Y[at(i, r)] : 0.0;
+        w_mask(i, a);
+        wa = mfma_16x16x4(a[0], zz[0], wa);
+        wb = mfma_16x16x4(a[1], zz[1], wb);
+        wa = mfma_16x16x4(a[2], zz[2], wa);
+        wb = mfma_16x16x4(a[3], zz[3], wb);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) part[w][(lk + 4 * r) * kWyCols + l16] = wa[r] + wb[r];
+    __syncthreads();
+    if (tid < kWyBlock * kWyCols) {
+      double x = 0.0;
+#pragma unroll
+      for (int g = 0; g < 8; ++g) x += part[g][tid];
+      wsum[tid] = x;
+    }
+    __syncthreads();
+    mfma_d4 y = mfma_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) y = mfma_16x16x4(-tt[q], wsum[(4 * q + lk) * kWyCols + l16], y);
+    if constexpr (MT > 0) {
+#pragma unroll
+      for (int q = 0; q < MT; ++q) {
+        const int i = w + 8 * q;
+        if (i >= t0 && i < nt) {
+          double a[4];
+          u_op(i, a);
+          u_mask(i, a);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) z[q] = mfma_16x16x4(a[r], y[r], z[q]);
+        }
+        if constexpr (MT > 8) {
+          if (q % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    } else {
+      for (int i = t0 + ((w - t0) & 7); i < nt; i += 8) {
+        double a[4];
+        mfma_d4 zz;
+        u_op(i, a);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) zz[r] = (on && 16 * i + lk + 4 * r < n) ? Y[at(i, r)] : 0.0;
+        u_mask(i, a);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) zz = mfma_16x16x4(a[r], y[r], zz);
+        if (on)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (16 * i + lk + 4 * r < n) Y[at(i, r)] = zz[r];
+      }
+    }
+  }
+  if constexpr (MT > 0) {
+    if (on)
+#pragma unroll
+      for (int q = 0; q < MT; ++q)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (16 * (w + 8 * q) + lk + 4 * r < n) Y[at(w + 8 * q, r)] = z[q][r];
+  }
 }
 
 }  // namespace xtb
