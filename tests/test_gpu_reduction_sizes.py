@@ -40,9 +40,21 @@ def stack(n, rng):
     [127, 128, 129, 130, 175, 176, 177],
     [190, 191, 192, 193, 194, 195],           # the switch between the two forms
     [208, 223, 225, 240, 254, 255, 256],
-    [257, 258, 259, 272, 289],                # the blocked reduction
+    [257, 258, 259, 272, 288, 289],           # teams of nine and ten workgroups
+    [353, 448, 449, 513],                     # row tiles per wavefront of the back-transformation
 ], ids=lambda s: f"{s[0]}-{s[-1]}")
 def test_sizes_against_the_oracle(sizes):
+    check(sizes)
+
+
+def test_teams_that_leave_at_the_gate(monkeypatch):
+    """A closed gate: every team leaves before it writes anything and one workgroup
+    per system reduces the matrices instead."""
+    monkeypatch.setenv("XTBLOOM_AMD_TEAMS", "0")
+    check([258, 289, 353])
+
+
+def check(sizes):
     rng = np.random.default_rng(sizes[0])
     b = workloads.from_systems([stack(n, rng) for n in sizes])
     ctx = interface.Context("hip", 0)

@@ -1147,6 +1147,333 @@ __device__ __forceinline__ void tridiag_full(double* A, int64_t ld, int n, doubl
   }
 }
 
+// Householder reduction by a team of workgroups, one system of 257 .. kTeamN
+// AOs, down to its last kFullN columns (k_tridiag finishes those).
+//
+// The whole matrix, both triangles, sits in the team's registers: member g of G
+// holds the rows i = g (mod G), its wavefront w the rows (8 s + w) G + g, s <
+// kTeamRows, lane l the columns l + 64 t.  A step k on every member:
+//   pass     A -= u r^T + r u^T of step k - 1 and p = A u_k on the member's
+//            rows, one sweep over the registers (u, r from LDS); row sums stay
+//            inside a wavefront;
+//   exchange the rows' p_i, and row k + 1 of A from its owner, through a ring
+//            of buffers in global memory; every member reads all of both;
+//   vectors  r = beta (p - beta (u.p) u / 2) and the next column
+//            A_{k+1, :} - u_{k+1} r - r_{k+1} u, formed by every member for
+//            itself (bit-identical: same data, same order).
+// So a step has one exchange and two block barriers, no panels and no pass over
+// memory.
+//
+// The exchanged words validate themselves: a buffer starts out filled with
+// kTeamEmpty (a NaN no arithmetic produces) and a reader spins on each word
+// until it is something else.  Slot k % kTeamRing is emptied by its writers in
+// step k + 1, when every member has published that step and so has read slot k;
+// it is written again kTeamRing - 1 exchanges later.
+//
+// Waiting is safe: no member writes anything before all G have met at the gate,
+// so from then on every partner is resident and runs.  Members that do not all
+// arrive within kTeamWaitTicks (the chip is held by something else) close the
+// gate together and leave; the system then takes k_tridiag_blocked.  The spins
+// are bounded too; one that runs out fails the system (status 8).
+//
+// Bound: the latency of a step, 4.5 us at 482 AOs (16 members) and 5.5 us at
+// 1142 (36), most of it the exchange through memory.  Measured against one
+// workgroup per system with panels of 16 reflectors (k_tridiag_blocked): 9.0 ->
+// 1.3 + 0.4 ms a round for 14 systems of 258-482 AOs, 111 -> 5.3 ms at 1142.
+// Members on one XCD (every eighth block) were 10 % slower than neighbours.
+constexpr int kTeamRows = 4, kTeamTiles = 20, kTeamN = 64 * kTeamTiles;
+constexpr int kTeamRing = 8;
+constexpr int kTeamOwn = (kTeamN + 511) / 512;  // vector entries per thread
+constexpr unsigned long long kTeamEmpty = 0xfff7a5a5c3c3e1e1ull;
+constexpr long long kTeamWaitTicks = 20000000;  // 100 MHz counter: 0.2 s
+constexpr int kTeamSpins = 1 << 22;
+constexpr unsigned kTeamClosed = 1u << 30;
+// team size: at most 8 kTeamRows rows per member
+__host__ __device__ constexpr int team_size(int n) { return (n + 8 * kTeamRows - 1) / (8 * kTeamRows); }
+
+// A system's exchange area (in the eigenvector matrix, free until the
+// eigenvectors are written): p ring, row ring, then the gate and done words.
+__device__ __forceinline__ unsigned* team_words(double* Z, int n) {
+  return reinterpret_cast<unsigned*>(Z + 2 * kTeamRing * (int64_t)n);
+}
+
+__global__ __launch_bounds__(256) void k_team_init(Topo t, const int* order, const unsigned char* active,
+                                                   double* Zall, unsigned gate) {
+  const int s = order[blockIdx.x];
+  if (active && !active[s]) return;
+  const int n = t.ao_off[s + 1] - t.ao_off[s];
+  double* Z = Zall + t.mat_off[s];
+  for (int i = threadIdx.x; i < 2 * kTeamRing * n; i += 256) Z[i] = __longlong_as_double((long long)kTeamEmpty);
+  if (threadIdx.x < 2) team_words(Z, n)[threadIdx.x] = threadIdx.x == 0 ? gate : 0u;
+}
+
+__device__ __forceinline__ void team_put(double* p, double x) {
+  unsigned long long b = (unsigned long long)__double_as_longlong(x);
+  if (b == kTeamEmpty) b = 0x7ff8000000000000ull;
+  __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void team_clear(double* p) {
+  __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), kTeamEmpty, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ unsigned long long team_peek(const double* p) {
+  return __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ __launch_bounds__(512) void k_tridiag_team(Topo t, const int* order, double* Aall, double* dall,
+                                                      double* eall, double* Zall, const unsigned char* active,
+                                                      SysState* st) {
+  const int s = order[blockIdx.y];
+  if (active && !active[s]) return;
+  const int n = t.ao_off[s + 1] - t.ao_off[s];
+  const int G = team_size(n), g = blockIdx.x;
+  if (g >= G) return;
+  double* A = Aall + t.mat_off[s];
+  double* d = dall + t.ao_off[s];
+  double* e = eall + t.ao_off[s];
+  double* ring_p = Zall + t.mat_off[s];
+  double* ring_r = ring_p + (int64_t)kTeamRing * n;
+  unsigned* gate = team_words(ring_p, n);
+  __shared__ double xb[2][kTeamN];  // u of this step and of the last one
+  __shared__ double rb[kTeamN];     // r of the last step
+  __shared__ double redn[8], redk[8];
+  __shared__ double sh_p;  // p at row k + 1
+  __shared__ int sh_bad;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int off = kTeamN - n;  // local index = global + off: the last tiles are always full
+  // the member's rows and column 0 (both read before the gate: from there on
+  // the owner of row k overwrites that row with its reflector)
+  double a[kTeamRows][kTeamTiles];
+#pragma unroll
+  for (int q = 0; q < kTeamRows; ++q) {
+    const int i = (8 * q + w) * G + g;
+    static_for<0, kTeamTiles>([&](auto CT) __attribute__((always_inline)) {
+      constexpr int T = decltype(CT)::value;
+      const int c = 64 * T + lane - off;
+      a[q][T] = 0.0;
+      if (i < n && c >= 0) a[q][T] = A[(int64_t)i * n + c];
+    });
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  double xo[kTeamOwn];  // this thread's entries L = tid + 512 q of the current column
+  {
+    double part = 0.0;
+#pragma unroll
+    for (int q = 0; q < kTeamOwn; ++q) {
+      const int L = tid + 512 * q;
+      double x = 0.0;
+      if (L >= off && L < kTeamN) x = A[L - off];
+      if (L == off && g == 0) d[0] = x;
+      xo[q] = L > off ? x : 0.0;
+      if (L > off + 1) part = fma(xo[q], xo[q], part);
+      if (L < kTeamN) {
+        xb[0][L] = xo[q];
+        xb[1][L] = 0.0;
+        rb[L] = 0.0;
+      }
+    }
+    part = wave_sum(part);
+    if (lane == 0) redn[w] = part;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  // the gate
+  if (tid == 0) {
+    unsigned old = __hip_atomic_fetch_add(gate, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    int closed = (old & kTeamClosed) != 0;
+    const long long t0 = wall_clock64();
+    old += 1;
+    while (!closed && (old & ~kTeamClosed) != (unsigned)G) {
+      __builtin_amdgcn_s_sleep(2);
+      old = __hip_atomic_load(gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      closed = (old & kTeamClosed) != 0;
+      if (!closed && (old & ~kTeamClosed) != (unsigned)G && wall_clock64() - t0 > kTeamWaitTicks) {
+        unsigned want = old;
+        if (__hip_atomic_compare_exchange_strong(gate, &want, old | kTeamClosed, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT))
+          closed = 1;
+      }
+    }
+    sh_bad = closed;
+  }
+  __syncthreads();
+  if (sh_bad) return;
+  const int kend = n - kFullN;  // columns reduced here
+  double v0 = 0.0;
+  int cur = 0;
+  int k = 0;
+  for (;; ++k) {
+    const int K = k + off, slot = k & (kTeamRing - 1);
+    double* pk = ring_p + (int64_t)slot * n;
+    double* rk = ring_r + (int64_t)slot * n;
+    const double tail = ((redn[0] + redn[1]) + (redn[2] + redn[3])) + ((redn[4] + redn[5]) + (redn[6] + redn[7]));
+    const double x0 = xb[cur][K + 1];
+    const double ss = fma(x0, x0, tail);
+    const bool noref = tail == 0.0 || ss < kTinyNorm;  // already reduced: inv = beta = 0
+    const double xn = ss * rsqrt_refined(fmax(ss, kTinyNorm));
+    const double alpha = x0 >= 0.0 ? -xn : xn;
+    v0 = x0 - alpha;
+    const double inv = noref ? 0.0 : rsqrt_refined(fmax(fma(v0, v0, tail), kTinyNorm));
+    const double beta = 2.0 * (inv * inv);
+    // one sweep over the registers: the pending update of step k - 1 (zero in
+    // step 0) and p = A u.  Finished rows ride along: their entries of u and r
+    // keep them finite, and the exchange hides them.
+    double p[kTeamRows], ur[kTeamRows], rr[kTeamRows];
+#pragma unroll
+    for (int q = 0; q < kTeamRows; ++q) {
+      const int L = min((8 * q + w) * G + g + off, kTeamN - 1);
+      ur[q] = xb[cur ^ 1][L];
+      rr[q] = rb[L];
+      p[q] = 0.0;
+    }
+    static_for<0, kTeamTiles>([&](auto CT) __attribute__((always_inline)) {
+      constexpr int T = decltype(CT)::value;
+      if (64 * T + 63 >= K) {  // a column tile with a live column
+        const int L = 64 * T + lane;
+        const double x = L == K + 1 ? v0 : xb[cur][L], u = xb[cur ^ 1][L], r = rb[L];
+#pragma unroll
+        for (int q = 0; q < kTeamRows; ++q) {
+          a[q][T] = fma(-ur[q], r, fma(-rr[q], u, a[q][T]));
+          p[q] = fma(a[q][T], x, p[q]);
+        }
+      }
+    });
+    if (k == kend) break;  // the last update is in: the trailing block is done
+    // publish row k + 1 and the rows' p.  The stores that emptied a slot were
+    // issued before the loads of the next exchange, whose return they precede,
+    // so they are long done when that slot comes round again.
+    // (opaque lane: addresses kept from step to step would live in scratch)
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    double* rl0 = rk + (ln - off);  // this lane's column of tile 0
+#pragma unroll
+    for (int q = 0; q < kTeamRows; ++q) {
+      if ((8 * q + w) * G + g == k + 1) {
+        static_for<0, kTeamTiles>([&](auto CT) __attribute__((always_inline)) {
+          constexpr int T = decltype(CT)::value;
+          if (64 * T + ln > K) team_put(rl0 + 64 * T, a[q][T]);
+        });
+      }
+    }
+    {
+      double r = row16_sums<kTeamRows>(p, lane & 15);
+      r += __shfl_xor(r, 16, 64);
+      r += __shfl_xor(r, 32, 64);
+      const int i = (8 * row16_index<kTeamRows>(lane & 15) + w) * G + g;
+      if (lane < 16 && (lane & 1) == 0 && i > k && i < n) team_put(pk + i, r);
+    }
+    if (g == k % G) {  // this member keeps column k's unit reflector (zero for no reflection)
+#pragma unroll
+      for (int q = 0; q < kTeamOwn; ++q) {
+        const int L = tid + 512 * q;
+        if (L > K && L < kTeamN) A[(L - off) + (int64_t)k * n] = (L == K + 1 ? v0 : xo[q]) * inv;
+      }
+      if (tid == 0) e[k] = noref ? x0 : alpha;
+    }
+    // everybody's p and the row
+    double po[kTeamOwn], ro[kTeamOwn];
+    {
+      int bad = 0;
+      unsigned long long bp[kTeamOwn], br[kTeamOwn];
+#pragma unroll
+      for (int q = 0; q < kTeamOwn; ++q) {
+        bp[q] = 0;
+        br[q] = 0;
+      }
+      for (int spin = 0;; ++spin) {
+        bool wait = false;
+#pragma unroll
+        for (int q = 0; q < kTeamOwn; ++q) {
+          const int L = tid + 512 * q;
+          if (L > K && L < kTeamN) {
+            bp[q] = team_peek(pk + (L - off));
+            br[q] = team_peek(rk + (L - off));
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < kTeamOwn; ++q) wait = wait || bp[q] == kTeamEmpty || br[q] == kTeamEmpty;
+        if (!wait) break;
+        if (spin >= kTeamSpins) {
+          bad = 1;
+          break;
+        }
+      }
+      if (bad) sh_bad = 1;
+      double kp = 0.0;
+#pragma unroll
+      for (int q = 0; q < kTeamOwn; ++q) {
+        const int L = tid + 512 * q;
+        po[q] = __longlong_as_double((long long)bp[q]);  // 0 where L <= K
+        ro[q] = __longlong_as_double((long long)br[q]);
+        if (L == K + 1) {
+          xo[q] = v0;
+          sh_p = po[q];
+        }
+        kp = fma(xo[q], po[q], kp);
+      }
+      kp = wave_sum(kp);
+      if (lane == 0) redk[w] = kp;
+    }
+    __syncthreads();
+    if (sh_bad) {
+      if (tid == 0) st[s].status = 8;
+      return;
+    }
+    {
+      const double hK = 0.5 * beta *
+                        (((redk[0] + redk[1]) + (redk[2] + redk[3])) + ((redk[4] + redk[5]) + (redk[6] + redk[7])));
+      const double r1 = beta * fma(-hK, v0, sh_p);
+      double part = 0.0;
+#pragma unroll
+      for (int q = 0; q < kTeamOwn; ++q) {
+        const int L = tid + 512 * q;
+        const double r = beta * fma(-hK, xo[q], po[q]);
+        const double x = fma(-v0, r, fma(-r1, xo[q], ro[q]));
+        if (L == K + 1) {
+          if (g == 0 && k + 1 < kend) d[k + 1] = x;
+          xb[cur][L] = v0;
+        }
+        xo[q] = L > K + 1 ? x : 0.0;
+        if (L > K + 2) part = fma(xo[q], xo[q], part);
+        if (L < kTeamN) {
+          rb[L] = r;
+          xb[cur ^ 1][L] = xo[q];
+        }
+      }
+      part = wave_sum(part);
+      if (lane == 0) redn[w] = part;
+    }
+    // every member has published step k, so it has read step k - 1: empty that slot
+    if (k > 0) {
+      double* pl = ring_p + (int64_t)((k - 1) & (kTeamRing - 1)) * n;
+      double* rl = ring_r + (int64_t)((k - 1) & (kTeamRing - 1)) * n;
+      if (lane < kTeamRows) {
+        const int i = (8 * lane + w) * G + g;
+        if (i >= k && i < n) team_clear(pl + i);
+      }
+      if (g == k % G && w == (k / G) % 8)
+        for (int c = k + lane; c < n; c += 64) team_clear(rl + c);
+    }
+    __syncthreads();
+    cur ^= 1;
+  }
+  // the trailing block, both triangles, for k_tridiag
+  int ln = lane;
+  asm volatile("" : "+v"(ln));
+#pragma unroll
+  for (int q = 0; q < kTeamRows; ++q) {
+    const int i = (8 * q + w) * G + g;
+    if (i >= kend && i < n)
+      static_for<0, kTeamTiles>([&](auto CT) __attribute__((always_inline)) {
+        constexpr int T = decltype(CT)::value;
+        // columns >= kend are the last kFullN local ones
+        if constexpr (64 * T >= kTeamN - kFullN) A[(int64_t)i * n + (64 * T + ln - off)] = a[q][T];
+      });
+  }
+  if (g == 0 && tid == 0) gate[1] = 1u;  // done
+}
+
 // The back-transformation applies the reflectors in compact WY blocks of
 // kWyBlock:  H_{k_15} ... H_{k_0} = I - V T V^T,  V = [v_{k_0} .. v_{k_15}],
 // k_u = n-3 - 16 ch - u, unit v, T lower triangular with
@@ -1205,9 +1532,10 @@ __device__ __forceinline__ void wy_factor(const double* A, int n, int ch, double
 
 // n <= 256, 512 threads per system (two waves per SIMD, 256 VGPRs per thread):
 // the columns before the last kFullN from the triangle in registers, the rest
-// with both triangles.
+// with both triangles.  n > 256: the last kFullN columns of the systems that
+// k_tridiag_team has reduced to them.
 __global__ __launch_bounds__(512) void k_tridiag(Topo t, const int* order, double* Aall, double* dall,
-                                                 double* eall, double* Tall,
+                                                 double* eall, double* Tall, double* Zall,
                                                  const unsigned char* active) {
   const int s = order[blockIdx.x];
   if (active && !active[s]) return;
@@ -1220,12 +1548,16 @@ __global__ __launch_bounds__(512) void k_tridiag(Topo t, const int* order, doubl
   __shared__ double col[512];  // published column of the triangle
   __shared__ double rowpart[32 * kTriPad];
   __shared__ double colpart[16 * kTriPad];
+  if (n > 256 && team_words(Zall + t.mat_off[s], n)[1] == 0u) return;
   int k0 = 0;
-  if (n > kFullN) {
+  if (n > 256) {
+    k0 = n - kFullN;
+  } else if (n > kFullN) {
     tridiag_registers<16>(A, n, d, e, v, col, pq, rowpart, colpart);
     k0 = n - kFullN;
   }
   tridiag_full(A + k0 + (int64_t)k0 * n, n, n - k0, d + k0, e + k0, v, pq);
+  if (n > 256) return;
   // WY factors for the back-transformation; the stored reflectors must be
   // visible to the whole block first
   __syncthreads();
@@ -1235,15 +1567,18 @@ __global__ __launch_bounds__(512) void k_tridiag(Topo t, const int* order, doubl
 }
 
 // n > 256: the blocked reduction, one 512-thread block per system (the host
-// launches the large systems only); W is per-system n x n scratch.  BIG: the
+// launches the large systems only; with Zteam the ones whose team left at the
+// gate); W is per-system n x n scratch.  BIG: the
 // systems above kMaxAO AOs, with the work vectors in their global slice of `big`.
 template <bool BIG>
 __global__ __launch_bounds__(512) void k_tridiag_blocked(Topo t, const int* order, double* Aall,
                                                          double* dall, double* eall, double* Wall,
-                                                         const unsigned char* active, double* big) {
+                                                         const unsigned char* active, double* big,
+                                                         double* Zteam) {
   const int s = order[blockIdx.x];
   if (active && !active[s]) return;
   const int n = t.ao_off[s + 1] - t.ao_off[s];
+  if (Zteam && team_words(Zteam + t.mat_off[s], n)[1] != 0u) return;  // reduced by its team
   __shared__ double v_l[BIG ? 1 : kMaxAO];
   __shared__ double pq_l[BIG ? 1 : kMaxAO];
   __shared__ double part_l[BIG ? 1 : 8 * kMaxAO];
@@ -3052,7 +3387,7 @@ __global__ __launch_bounds__(512) void k_wy_factors(Topo t, const int* order, co
 // (issued before the barriers, so that L2's latency overlaps the products).
 // MT row tiles per wavefront in registers (n <= 128 MT); MT = 0 keeps the
 // columns in Y.  Measured against eight reflectors at a time on the vector
-// units: 10.6 -> 0.70 ms at 1142 AOs, 375 -> 81 us for 14 systems of 258-482 AOs.
+// units: 10.6 -> 0.70 ms at 1142 AOs, 375 -> 96 us for 14 systems of 258-482 AOs.
 constexpr int kWyThreads = 512;
 constexpr int kWyCols = 16;
 
