@@ -304,6 +304,14 @@ __device__ __forceinline__ double wave_sum(double v) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
+// lane k's value (k uniform over the wavefront)
+__device__ __forceinline__ double lane_value(double v, int k) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)b, k);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), k);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
 // Block-wide sum for blockDim.x <= 1024; red must hold blockDim.x/64 doubles.
 __device__ __forceinline__ double block_sum(double v, double* red) {
   v = wave_sum(v);
