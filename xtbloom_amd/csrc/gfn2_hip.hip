@@ -609,6 +609,7 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
   std::vector<int64_t> part_off(B + 1, 0);
   int n_large = 0;  // systems above 256 AOs (a prefix of the size order)
   int n_xl = 0;     // systems above kMaxAO AOs (a prefix of that prefix)
+  int n_huge = 0;   // systems above kEigSplitAO AOs (a prefix of that one)
   // back-transformation tasks of the systems above 2048, 1024, 512 and 256 AOs
   // (prefixes of `back`)
   size_t n_back[4] = {0, 0, 0, 0};
@@ -617,6 +618,7 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
     const int n = T.ao_off[s + 1] - T.ao_off[s];
     n_large += n > 256;
     n_xl += n > kMaxAO;
+    n_huge += n > kEigSplitAO;
     const int nt = (n + kTile - 1) / kTile;
     for (int a = 0; a < nt; ++a)
       for (int b = 0; b < nt; ++b) {
@@ -1265,17 +1267,28 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
     if (rp) rp->tri = last_probe();
     HIP_TRY(probe_begin(kKTridiagEigen));
     // eigenvalues, occupations (kocc), eigenvectors of the kocc lowest levels
-    if (n_xl > 0)
-      hipLaunchKernelGGL(k_tridiag_eigen<true>, dim3(n_xl), dim3(256), 0, sm, t, d_order, d_active, d_td,
-                         d_te, dZ, EigenScratch{dT, dH, dC, dP, dW}, d_eps, d_shift, it, rptr, d_zscale,
-                         FermiOut{d_fa, d_fb, d_occ, d_fe, d_st, d_kocc, opt.kt}, d_xl, co);
-    if (n_xl < B)
-      hipLaunchKernelGGL(k_tridiag_eigen<false>, dim3(B - n_xl), dim3(256), 0, sm, t, d_order + n_xl,
-                         d_active, d_td, d_te, dZ, EigenScratch{dT, dH, dC, dP, dW}, d_eps, d_shift, it,
-                         rptr, d_zscale, FermiOut{d_fa, d_fb, d_occ, d_fe, d_st, d_kocc, opt.kt}, d_xl, co);
+    const EigenScratch scratch{dT, dH, dC, dP, dW};
+    const FermiOut fermi{d_fa, d_fb, d_occ, d_fe, d_st, d_kocc, opt.kt};
+    if (n_huge > 0)
+      hipLaunchKernelGGL(k_tridiag_eigen<true>, dim3(n_huge), dim3(256), 0, sm, t, d_order, d_active, d_td, d_te, dZ,
+                         scratch, d_eps, d_shift, it, rptr, d_zscale, fermi, d_xl, co);
+    if (n_large > n_huge) {  // spread over the chip, 64 eigenpairs a wavefront
+      const int nsys = n_large - n_huge;
+      const int* ord = d_order + n_huge;
+      const unsigned groups = (unsigned)((T.ao_off[T.order[n_huge] + 1] - T.ao_off[T.order[n_huge]] + 63) / 64);
+      hipLaunchKernelGGL(k_eig_values, dim3(groups, nsys), dim3(64), 0, sm, t, ord, d_active, d_td, d_te, d_eps,
+                         d_shift, it, rptr, dY);
+      hipLaunchKernelGGL(k_eig_occupations, dim3(nsys), dim3(256), 0, sm, t, ord, d_active, d_td, d_te, d_eps, d_shift,
+                         it, rptr, dY, fermi, co);
+      hipLaunchKernelGGL(k_eig_vectors, dim3(groups, nsys), dim3(64), 0, sm, t, ord, d_active, d_td, d_te, dY, dZ,
+                         scratch, d_zscale, d_kocc, co);
+    }
+    if (n_large < B)
+      hipLaunchKernelGGL(k_tridiag_eigen<false>, dim3(B - n_large), dim3(256), 0, sm, t, d_order + n_large, d_active,
+                         d_td, d_te, dZ, scratch, d_eps, d_shift, it, rptr, d_zscale, fermi, d_xl, co);
     // clusters of more than kSerialCluster eigenvalues (rare: near-dependent bases)
     hipLaunchKernelGGL(k_cluster_vectors, dim3(B), dim3(256), 0, sm, t, d_order, d_active, d_td, d_te, dZ,
-                       EigenScratch{dT, dH, dC, dP, dW}, d_zscale, co);
+                       scratch, d_zscale, co);
     HIP_TRY(probe_end(kKTridiagEigen, 0.0, 0.0));
     HIP_TRY(probe_begin(kKBacktransform));
     // systems above 256 AOs: the WY factors of their reflectors, then one

@@ -2643,152 +2643,90 @@ struct FermiOut {
 // above kMaxAO AOs, with d, e, e^2, the eigenvalues and their ranks in their
 // global slice of `big`.  Clusters of more than kSerialCluster close
 // eigenvalues are left to k_cluster_vectors through `co`.
-template <bool BIG>
-__global__ __launch_bounds__(256) void k_tridiag_eigen(Topo t, const int* order,
-                                                       const unsigned char* active,
-                                                       const double* dall, const double* eall,
-                                                       double* Zall, EigenScratch sc,
-                                                       double* wall, double* shift, int round_arg,
-                                                       const int* round_ptr,
-                                                       double* zscale_all, FermiOut fo, double* big,
-                                                       ClusterOut co) {
-  const int s = order[blockIdx.x];
-  if (active && !active[s]) return;
-  const int n = t.ao_off[s + 1] - t.ao_off[s];
-  const int64_t mo = t.mat_off[s];
-  double* __restrict__ Z = Zall + mo;
-  double* __restrict__ F0 = sc.u0 + mo;
-  double* __restrict__ F1 = sc.u1 + mo;
-  double* __restrict__ F2 = sc.u2 + mo;
-  double* __restrict__ FM = sc.mult + mo;
-  double* __restrict__ FP = sc.piv + mo;
-  double* zscale = zscale_all + t.ao_off[s];
-  __shared__ double d_l[BIG ? 1 : kMaxAO];
-  __shared__ double e_l[BIG ? 1 : kMaxAO];   // split off-diagonal (negligible entries zeroed)
-  __shared__ double e2_l[BIG ? 1 : kMaxAO];
-  __shared__ double lam_l[BIG ? 1 : kMaxAO];
-  double *d = d_l, *e = e_l, *e2 = e2_l, *lam = lam_l;
-  if constexpr (BIG) {
-    d = big + big_offset(t, s);  // d, e, e2, lam, rnk: 5 n <= kBigPerAO n doubles
-    e = d + n;
-    e2 = e + n;
-    lam = e2 + n;
-  }
-  __shared__ double red[16];
+// T of one system into d, e and e2 = e^2 with the negligible off-diagonals
+// zeroed, by the whole block; the pivot floor, and whether T did not split.
+__device__ __forceinline__ bool eig_load(const double* dg, const double* eg, int n, double* d, double* e, double* e2,
+                                         double* red, int& nsplit, double& pivmin) {
   const int tid = threadIdx.x, nt = blockDim.x;
-  if (tid == 0) co.flag[s] = 0;
   double emax2 = 0.0;
   for (int i = tid; i < n; i += nt) {
-    d[i] = dall[t.ao_off[s] + i];
-    double ei = i + 1 < n ? eall[t.ao_off[s] + i] : 0.0;
-    e[i] = ei;
+    d[i] = dg[i];
+    e[i] = i + 1 < n ? eg[i] : 0.0;
   }
+  if (tid == 0) nsplit = 0;
   __syncthreads();
+  int cut = 0;
   for (int i = tid; i < n; i += nt) {
     double ei = e[i];
     if (i + 1 < n && ei * ei <= kEps * kEps * fabs(d[i] * d[i + 1]) + kSafeMin) ei = 0.0;
+    if (i + 1 < n && ei == 0.0) ++cut;
     e2[i] = ei * ei;
     emax2 = fmax(emax2, ei * ei);
   }
+  if (cut) atomicAdd(&nsplit, cut);
   __syncthreads();
   for (int i = tid; i < n; i += nt)
     if (e2[i] == 0.0) e[i] = 0.0;
-  // block-wide max of e^2 for the pivot floor
-  {
-    double m2 = emax2;
-    for (int off = 32; off > 0; off >>= 1) m2 = fmax(m2, __shfl_xor(m2, off, 64));
-    __syncthreads();
-    if ((tid & 63) == 0) red[tid >> 6] = m2;
-    __syncthreads();
-    m2 = 0.0;
-    for (int w = 0; w < (nt >> 6); ++w) m2 = fmax(m2, red[w]);
-    emax2 = m2;
-    __syncthreads();
-  }
-  const double pivmin = kSafeMin * fmax(1.0, emax2);
+  for (int off = 32; off > 0; off >>= 1) emax2 = fmax(emax2, __shfl_xor(emax2, off, 64));
+  if ((tid & 63) == 0) red[tid >> 6] = emax2;
+  __syncthreads();
+  emax2 = 0.0;
+  for (int w = 0; w < (nt >> 6); ++w) emax2 = fmax(emax2, red[w]);
+  __syncthreads();
+  pivmin = kSafeMin * fmax(1.0, emax2);
+  return nsplit == 0;
+}
 
-  // ---- eigenvalues: lanes draw indices from a shared counter ----
-  // the previous round's eigenvalues are guesses when T did not split
-  __shared__ int nsplit, next_j;
-  if (tid == 0) { nsplit = 0; next_j = 0; }
-  __syncthreads();
-  for (int i = tid; i + 1 < n; i += nt)
-    if (e[i] == 0.0) atomicAdd(&nsplit, 1);
-  __syncthreads();
-  const bool unsplit = nsplit == 0;
-  // the SCC round: the launch argument, or the device-resident counter of
-  // rounds enqueued ahead of the host (graph-captured rounds)
-  const int round = round_ptr ? *round_ptr : round_arg;
-  const bool have_old = round >= 1 && unsplit;
-  const bool guess_ok = round >= 2 && unsplit;
-  const double delta = guess_ok ? 2.0 * shift[s] : 0.0;
-  // whole-matrix Gershgorin bounds (used when T is unsplit)
-  __shared__ double gbound[3];
-  if (unsplit) {
-    double gl = 1e300, gu = -1e300;
-    for (int i = tid; i < n; i += nt) {
-      const double off = (i > 0 ? fabs(e[i - 1]) : 0.0) + (i + 1 < n ? fabs(e[i]) : 0.0);
-      gl = fmin(gl, d[i] - off);
-      gu = fmax(gu, d[i] + off);
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-      gl = fmin(gl, __shfl_xor(gl, off, 64));
-      gu = fmax(gu, __shfl_xor(gu, off, 64));
-    }
-    if ((tid & 63) == 0) { red[tid >> 6] = gl; red[8 + (tid >> 6)] = gu; }
-    __syncthreads();
-    if (tid == 0) {
-      for (int w = 1; w < (nt >> 6); ++w) { gl = fmin(gl, red[w]); gu = fmax(gu, red[8 + w]); }
-      const double tnorm = fmax(fabs(gl), fabs(gu));
-      const double fudge = 2.0 * kEps * tnorm * n + 4.0 * pivmin;
-      gbound[0] = gl - fudge;
-      gbound[1] = gu + fudge;
-      gbound[2] = 2.0 * kEps * tnorm + pivmin;
-    }
-    __syncthreads();
+// Whole-matrix Gershgorin bounds and tolerance of an unsplit T: gbound = lo, hi, tol
+__device__ __forceinline__ void eig_bounds(const double* d, const double* e, int n, double pivmin, double* red,
+                                           double* gbound) {
+  const int tid = threadIdx.x, nt = blockDim.x;
+  double gl = 1e300, gu = -1e300;
+  for (int i = tid; i < n; i += nt) {
+    const double off = (i > 0 ? fabs(e[i - 1]) : 0.0) + (i + 1 < n ? fabs(e[i]) : 0.0);
+    gl = fmin(gl, d[i] - off);
+    gu = fmax(gu, d[i] + off);
   }
-  double dmax = 0.0;
-  {
-    EigState st;
-    bool busy = false;
-    for (;;) {
-      if (!busy) {
-        const int j = atomicAdd(&next_j, 1);
-        if (j >= n) break;
-        const double* wo = wall + t.ao_off[s];
-        const double g = have_old ? wo[j] : 0.0;
-        const double gp = (have_old && j > 0) ? wo[j - 1] : -1e300;
-        const double gn = (have_old && j + 1 < n) ? wo[j + 1] : 1e300;
-        busy = eig_start(st, j, d, e, n, pivmin, unsplit, gbound[0], gbound[1], gbound[2], guess_ok,
-                         g, gp, gn, delta, lam);
-        if (!busy) continue;
-      }
-      double x;
-      if (eig_step(st, d, e2, x)) {
-        lam[st.j] = x;
-        if (have_old) dmax = fmax(dmax, fabs(x - wall[t.ao_off[s] + st.j]));
-        busy = false;
-      }
-    }
+  for (int off = 32; off > 0; off >>= 1) {
+    gl = fmin(gl, __shfl_xor(gl, off, 64));
+    gu = fmax(gu, __shfl_xor(gu, off, 64));
   }
-  // largest eigenvalue change of this round (block max), for the next round's brackets
-  for (int off = 32; off > 0; off >>= 1) dmax = fmax(dmax, __shfl_xor(dmax, off, 64));
-  __syncthreads();
-  if ((tid & 63) == 0) red[tid >> 6] = dmax;
+  if ((tid & 63) == 0) { red[tid >> 6] = gl; red[8 + (tid >> 6)] = gu; }
   __syncthreads();
   if (tid == 0) {
-    double m = 0.0;
-    for (int w = 0; w < (nt >> 6); ++w) m = fmax(m, red[w]);
-    // first round: no change measured yet, take a generous bracket
-    shift[s] = have_old ? m : 1.0;
+    for (int w = 1; w < (nt >> 6); ++w) { gl = fmin(gl, red[w]); gu = fmax(gu, red[8 + w]); }
+    const double tnorm = fmax(fabs(gl), fabs(gu));
+    const double fudge = 2.0 * kEps * tnorm * n + 4.0 * pivmin;
+    gbound[0] = gl - fudge;
+    gbound[1] = gu + fudge;
+    gbound[2] = 2.0 * kEps * tnorm + pivmin;
   }
   __syncthreads();
+}
 
+// 1-norm of T
+__device__ __forceinline__ void eig_norm1(const double* d, const double* e, int n, double* red, double& tnorm1) {
+  const int tid = threadIdx.x, nt = blockDim.x;
+  double m = 0.0;
+  for (int i = tid; i < n; i += nt)
+    m = fmax(m, fabs(d[i]) + (i > 0 ? fabs(e[i - 1]) : 0.0) + (i + 1 < n ? fabs(e[i]) : 0.0));
+  for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, 64));
+  if ((tid & 63) == 0) red[tid >> 6] = m;
+  __syncthreads();
+  if (tid == 0) {
+    for (int w = 1; w < (nt >> 6); ++w) m = fmax(m, red[w]);
+    tnorm1 = m;
+  }
+  __syncthreads();
+}
+
+// Ascending ranks of the eigenvalues lam, the sorted spectrum (srt, w_out), the
+// Fermi occupations and kocc, by a block of at least 128 threads; returns kocc.
+__device__ __forceinline__ int eig_occupations(const Topo& t, int s, int n, const double* lam, int* rnk, double* srt,
+                                               double* w_out, const FermiOut& fo) {
+  const int tid = threadIdx.x, nt = blockDim.x;
   // ---- ascending rank (stable on ties) and the sorted spectrum ----
-  __shared__ int rnk_l[BIG ? 1 : kMaxAO];
-  int* rnk = BIG ? reinterpret_cast<int*>(lam + n) : rnk_l;
   __shared__ int kocc_sh;
-  double* srt = e2;  // e2 is not needed after the eigenvalues
   for (int j = tid; j < n; j += nt) {
     const double lj = lam[j];
     int r = 0;
@@ -2798,7 +2736,7 @@ __global__ __launch_bounds__(256) void k_tridiag_eigen(Topo t, const int* order,
     }
     rnk[j] = r;
     srt[r] = lj;
-    wall[t.ao_off[s] + r] = lj;
+    w_out[r] = lj;
   }
   __syncthreads();
   // ---- occupations: alpha on the first wavefront, beta on the second (a
@@ -2851,168 +2789,251 @@ __global__ __launch_bounds__(256) void k_tridiag_eigen(Topo t, const int* order,
     }
   }
   __syncthreads();
-  const int kocc = kocc_sh;
+  return kocc_sh;
+}
 
-  // ---- eigenvectors: thread per cluster start ----
-  // A cluster is needed when its first (lowest) member is below kocc; every
-  // member of a needed cluster is computed so the cluster stays orthogonal.
-  // an unsplit T is one block [0, n) whose 1-norm is the block-wide maximum
-  // row sum; split blocks are found and measured by the thread that needs them
-  __shared__ double tnorm1;
+// Eigenvector of eigenvalue j below kocc, or of the cluster that j starts, by
+// one thread.  A cluster is needed when its first (lowest) member is below
+// kocc; every member of a needed cluster is computed so the cluster stays
+// orthogonal.  An unsplit T is one block [0, n) of 1-norm tnorm1; split blocks
+// are found and measured by the thread that needs them.
+__device__ __forceinline__ void eig_vector(int j, int n, int kocc, const double* d, const double* e, const double* lam,
+                                           const int* rnk, bool unsplit, double tnorm1, double pivmin,
+                                           const EigenScratch& sc, int64_t mo, double* __restrict__ Z, double* zscale,
+                                           const ClusterOut& co, int s, int o) {
+  double* __restrict__ F0 = sc.u0 + mo;
+  double* __restrict__ F1 = sc.u1 + mo;
+  double* __restrict__ F2 = sc.u2 + mo;
+  double* __restrict__ FM = sc.mult + mo;
+  double* __restrict__ FP = sc.piv + mo;
+  if (rnk[j] >= kocc) return;
+  int b0 = j, b1 = j + 1;
+  double onenrm = 0.0;
   if (unsplit) {
-    double m = 0.0;
-    for (int i = tid; i < n; i += nt)
-      m = fmax(m, fabs(d[i]) + (i > 0 ? fabs(e[i - 1]) : 0.0) + (i + 1 < n ? fabs(e[i]) : 0.0));
-    for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, 64));
-    if ((tid & 63) == 0) red[tid >> 6] = m;
-    __syncthreads();
-    if (tid == 0) {
-      for (int w = 1; w < (nt >> 6); ++w) m = fmax(m, red[w]);
-      tnorm1 = m;
-    }
-    __syncthreads();
+    b0 = 0;
+    b1 = n;
+    onenrm = tnorm1;
+  } else {
+    while (b0 > 0 && e[b0 - 1] != 0.0) --b0;
+    while (b1 < n && e[b1 - 1] != 0.0) ++b1;
+    for (int i = b0; i < b1; ++i)
+      onenrm = fmax(onenrm, fabs(d[i]) + (i > b0 ? fabs(e[i - 1]) : 0.0) + (i + 1 < b1 ? fabs(e[i]) : 0.0));
   }
-  for (int j = tid; j < n; j += nt) {
-    if (rnk[j] >= kocc) continue;
-    int b0 = j, b1 = j + 1;
-    double onenrm = 0.0;
-    if (unsplit) {
-      b0 = 0;
-      b1 = n;
-      onenrm = tnorm1;
-    } else {
-      while (b0 > 0 && e[b0 - 1] != 0.0) --b0;
-      while (b1 < n && e[b1 - 1] != 0.0) ++b1;
-      for (int i = b0; i < b1; ++i)
-        onenrm = fmax(onenrm, fabs(d[i]) + (i > b0 ? fabs(e[i - 1]) : 0.0) + (i + 1 < b1 ? fabs(e[i]) : 0.0));
+  const int bn = b1 - b0;
+  const double gtol = kClusterTol * fmax(onenrm, kSafeMin);
+  if (j > b0 && lam[j] - lam[j - 1] <= gtol) return;  // not a cluster start
+  int g1 = j + 1;
+  while (g1 < b1 && lam[g1] - lam[g1 - 1] <= gtol) ++g1;
+  if (g1 - j > kSerialCluster) {  // the whole block orthogonalizes it (k_cluster_vectors)
+    for (int jj = j; jj < g1; ++jj) {
+      co.lam[o + jj] = lam[jj];
+      co.rank[o + jj] = rnk[jj];
     }
-    const int bn = b1 - b0;
-    const double gtol = kClusterTol * fmax(onenrm, kSafeMin);
-    if (j > b0 && lam[j] - lam[j - 1] <= gtol) continue;  // not a cluster start
-    int g1 = j + 1;
-    while (g1 < b1 && lam[g1] - lam[g1 - 1] <= gtol) ++g1;
-    if (g1 - j > kSerialCluster) {  // the whole block orthogonalizes it (k_cluster_vectors)
-      const int o = t.ao_off[s];
-      for (int jj = j; jj < g1; ++jj) {
-        co.lam[o + jj] = lam[jj];
-        co.rank[o + jj] = rnk[jj];
-      }
-      co.end[o + j] = g1;
-      co.flag[s] = 1;
+    co.end[o + j] = g1;
+    co.flag[s] = 1;
+    return;
+  }
+  const double ptol = kEps * fmax(onenrm, kSafeMin);       // smallest admissible pivot
+  const double pertol = 10.0 * kEps * fmax(onenrm, kSafeMin);
+  double xprev = 0.0;
+  for (int jj = j; jj < g1; ++jj) {
+    const int cj = rnk[jj];  // Z column of eigenvalue jj
+    // rows outside the block are zero
+    for (int i = 0; i < b0; ++i) Z[(int64_t)i * n + cj] = 0.0;
+    for (int i = b1; i < n; ++i) Z[(int64_t)i * n + cj] = 0.0;
+    zscale[cj] = 1.0;
+    if (bn == 1) {
+      Z[(int64_t)b0 * n + cj] = 1.0;
       continue;
     }
-    const double ptol = kEps * fmax(onenrm, kSafeMin);       // smallest admissible pivot
-    const double pertol = 10.0 * kEps * fmax(onenrm, kSafeMin);
-    double xprev = 0.0;
-    for (int jj = j; jj < g1; ++jj) {
-      const int cj = rnk[jj];  // Z column of eigenvalue jj
-      // rows outside the block are zero
-      for (int i = 0; i < b0; ++i) Z[(int64_t)i * n + cj] = 0.0;
-      for (int i = b1; i < n; ++i) Z[(int64_t)i * n + cj] = 0.0;
-      zscale[cj] = 1.0;
-      if (bn == 1) {
-        Z[(int64_t)b0 * n + cj] = 1.0;
+    double x = lam[jj];
+    if (jj > j && x - xprev < pertol) x = xprev + pertol;
+    xprev = x;
+    if (g1 - j == 1) {
+      double f;
+      if (twisted_vector(d, e, b0, b1, x, pivmin, n, cj, F0, F1, Z, f)) {
+        zscale[cj] = f;
         continue;
       }
-      double x = lam[jj];
-      if (jj > j && x - xprev < pertol) x = xprev + pertol;
-      xprev = x;
-      if (g1 - j == 1) {
-        double f;
-        if (twisted_vector(d, e, b0, b1, x, pivmin, n, cj, F0, F1, Z, f)) {
-          zscale[cj] = f;
-          continue;
-        }
+    }
+    // LU with partial pivoting of T_b - x I
+    double c0 = d[b0] - x, c1 = e[b0], c2 = 0.0;
+    for (int k = 0; k < bn - 1; ++k) {
+      const int gi = b0 + k;
+      const double n0 = e[gi], n1 = d[gi + 1] - x, n2 = (k + 2 < bn) ? e[gi + 1] : 0.0;
+      const int64_t at = (int64_t)gi * n + cj;
+      if (fabs(c0) >= fabs(n0)) {
+        const double m = c0 != 0.0 ? n0 / c0 : 0.0;
+        F0[at] = c0; F1[at] = c1; F2[at] = c2; FM[at] = m; FP[at] = 0.0;
+        c0 = n1 - m * c1;
+        c1 = n2 - m * c2;
+      } else {
+        const double m = c0 / n0;
+        F0[at] = n0; F1[at] = n1; F2[at] = n2; FM[at] = m; FP[at] = 1.0;
+        const double t0 = c1 - m * n1, t1 = c2 - m * n2;
+        c0 = t0;
+        c1 = t1;
       }
-      // LU with partial pivoting of T_b - x I
-      double c0 = d[b0] - x, c1 = e[b0], c2 = 0.0;
-      for (int k = 0; k < bn - 1; ++k) {
-        const int gi = b0 + k;
-        const double n0 = e[gi], n1 = d[gi + 1] - x, n2 = (k + 2 < bn) ? e[gi + 1] : 0.0;
-        const int64_t at = (int64_t)gi * n + cj;
-        if (fabs(c0) >= fabs(n0)) {
-          const double m = c0 != 0.0 ? n0 / c0 : 0.0;
-          F0[at] = c0; F1[at] = c1; F2[at] = c2; FM[at] = m; FP[at] = 0.0;
-          c0 = n1 - m * c1;
-          c1 = n2 - m * c2;
-        } else {
-          const double m = c0 / n0;
-          F0[at] = n0; F1[at] = n1; F2[at] = n2; FM[at] = m; FP[at] = 1.0;
-          const double t0 = c1 - m * n1, t1 = c2 - m * n2;
-          c0 = t0;
-          c1 = t1;
-        }
-        c2 = 0.0;
+      c2 = 0.0;
+    }
+    {
+      const int64_t at = (int64_t)(b1 - 1) * n + cj;
+      F0[at] = c0; F1[at] = 0.0; F2[at] = 0.0; FM[at] = 0.0; FP[at] = 0.0;
+    }
+    for (int i = b0; i < b1; ++i) Z[(int64_t)i * n + cj] = start_component(jj, i - b0);
+    for (int it = 0; it <= kInverseIterations; ++it) {
+      // orthogonalize against the cluster members already finished
+      for (int p = j; p < jj; ++p) {
+        double dot = 0.0;
+        for (int i = b0; i < b1; ++i) dot += Z[(int64_t)i * n + rnk[p]] * Z[(int64_t)i * n + cj];
+        for (int i = b0; i < b1; ++i) Z[(int64_t)i * n + cj] -= dot * Z[(int64_t)i * n + rnk[p]];
       }
+      if (it == kInverseIterations) break;
+      // scale to unit max-norm, then solve (T_b - x I) y = r
+      double rmax = 0.0;
+      for (int i = b0; i < b1; ++i) rmax = fmax(rmax, fabs(Z[(int64_t)i * n + cj]));
+      const double rs = rmax > 0.0 ? 1.0 / rmax : 1.0;
+      for (int i = b0; i < b1; ++i) Z[(int64_t)i * n + cj] *= rs;
+      // forward elimination; the running entry stays in a register (it is
+      // the one stored one row earlier), so only independent loads remain
       {
-        const int64_t at = (int64_t)(b1 - 1) * n + cj;
-        F0[at] = c0; F1[at] = 0.0; F2[at] = 0.0; FM[at] = 0.0; FP[at] = 0.0;
+        double cur = Z[(int64_t)b0 * n + cj];
+        for (int k = 0; k < bn - 1; ++k) {
+          const int64_t at = (int64_t)(b0 + k) * n + cj;
+          double rk = cur, rn = Z[at + n];
+          if (FP[at] != 0.0) { const double tmp = rk; rk = rn; rn = tmp; }
+          Z[at] = rk;
+          cur = rn - FM[at] * rk;
+        }
+        Z[(int64_t)(b1 - 1) * n + cj] = cur;
       }
-      for (int i = b0; i < b1; ++i) Z[(int64_t)i * n + cj] = start_component(jj, i - b0);
-      for (int it = 0; it <= kInverseIterations; ++it) {
-        // orthogonalize against the cluster members already finished
-        for (int p = j; p < jj; ++p) {
-          double dot = 0.0;
-          for (int i = b0; i < b1; ++i) dot += Z[(int64_t)i * n + rnk[p]] * Z[(int64_t)i * n + cj];
-          for (int i = b0; i < b1; ++i) Z[(int64_t)i * n + cj] -= dot * Z[(int64_t)i * n + rnk[p]];
+      // back substitution with the two entries below in registers
+      {
+        double z1 = 0.0, z2 = 0.0;  // solution entries k + 1, k + 2
+        for (int k = bn - 1; k >= 0; --k) {
+          const int64_t at = (int64_t)(b0 + k) * n + cj;
+          double r = Z[at];
+          if (k + 1 < bn) r -= F1[at] * z1;
+          if (k + 2 < bn) r -= F2[at] * z2;
+          double u = F0[at];
+          if (fabs(u) < ptol) u = u < 0.0 ? -ptol : ptol;
+          const double zk = r / u;
+          Z[at] = zk;
+          z2 = z1;
+          z1 = zk;
         }
-        if (it == kInverseIterations) break;
-        // scale to unit max-norm, then solve (T_b - x I) y = r
-        double rmax = 0.0;
-        for (int i = b0; i < b1; ++i) rmax = fmax(rmax, fabs(Z[(int64_t)i * n + cj]));
-        const double rs = rmax > 0.0 ? 1.0 / rmax : 1.0;
-        for (int i = b0; i < b1; ++i) Z[(int64_t)i * n + cj] *= rs;
-        // forward elimination; the running entry stays in a register (it is
-        // the one stored one row earlier), so only independent loads remain
-        {
-          double cur = Z[(int64_t)b0 * n + cj];
-          for (int k = 0; k < bn - 1; ++k) {
-            const int64_t at = (int64_t)(b0 + k) * n + cj;
-            double rk = cur, rn = Z[at + n];
-            if (FP[at] != 0.0) { const double tmp = rk; rk = rn; rn = tmp; }
-            Z[at] = rk;
-            cur = rn - FM[at] * rk;
-          }
-          Z[(int64_t)(b1 - 1) * n + cj] = cur;
-        }
-        // back substitution with the two entries below in registers
-        {
-          double z1 = 0.0, z2 = 0.0;  // solution entries k + 1, k + 2
-          for (int k = bn - 1; k >= 0; --k) {
-            const int64_t at = (int64_t)(b0 + k) * n + cj;
-            double r = Z[at];
-            if (k + 1 < bn) r -= F1[at] * z1;
-            if (k + 2 < bn) r -= F2[at] * z2;
-            double u = F0[at];
-            if (fabs(u) < ptol) u = u < 0.0 ? -ptol : ptol;
-            const double zk = r / u;
-            Z[at] = zk;
-            z2 = z1;
-            z1 = zk;
-          }
-        }
-        // normalize
-        double nrm = 0.0, ymax = 0.0;
-        for (int i = b0; i < b1; ++i) ymax = fmax(ymax, fabs(Z[(int64_t)i * n + cj]));
-        const double ys = ymax > 0.0 ? 1.0 / ymax : 1.0;
-        for (int i = b0; i < b1; ++i) {
-          const double y = Z[(int64_t)i * n + cj] * ys;
-          nrm += y * y;
-        }
-        const double sc2 = ys / sqrt(nrm);
-        for (int i = b0; i < b1; ++i) Z[(int64_t)i * n + cj] *= sc2;
       }
-      // final normalization; sign: largest-magnitude component positive
-      double nrm = 0.0, big = 0.0;
+      // normalize
+      double nrm = 0.0, ymax = 0.0;
+      for (int i = b0; i < b1; ++i) ymax = fmax(ymax, fabs(Z[(int64_t)i * n + cj]));
+      const double ys = ymax > 0.0 ? 1.0 / ymax : 1.0;
       for (int i = b0; i < b1; ++i) {
-        const double y = Z[(int64_t)i * n + cj];
+        const double y = Z[(int64_t)i * n + cj] * ys;
         nrm += y * y;
-        if (fabs(y) > fabs(big)) big = y;
       }
-      const double f = (big < 0.0 ? -1.0 : 1.0) / sqrt(nrm);
-      for (int i = b0; i < b1; ++i) Z[(int64_t)i * n + cj] *= f;
+      const double sc2 = ys / sqrt(nrm);
+      for (int i = b0; i < b1; ++i) Z[(int64_t)i * n + cj] *= sc2;
+    }
+    // final normalization; sign: largest-magnitude component positive
+    double nrm = 0.0, big = 0.0;
+    for (int i = b0; i < b1; ++i) {
+      const double y = Z[(int64_t)i * n + cj];
+      nrm += y * y;
+      if (fabs(y) > fabs(big)) big = y;
+    }
+    const double f = (big < 0.0 ? -1.0 : 1.0) / sqrt(nrm);
+    for (int i = b0; i < b1; ++i) Z[(int64_t)i * n + cj] *= f;
+  }
+}
+
+template <bool BIG>
+__global__ __launch_bounds__(256) void k_tridiag_eigen(Topo t, const int* order,
+                                                       const unsigned char* active,
+                                                       const double* dall, const double* eall,
+                                                       double* Zall, EigenScratch sc,
+                                                       double* wall, double* shift, int round_arg,
+                                                       const int* round_ptr,
+                                                       double* zscale_all, FermiOut fo, double* big,
+                                                       ClusterOut co) {
+  const int s = order[blockIdx.x];
+  if (active && !active[s]) return;
+  const int n = t.ao_off[s + 1] - t.ao_off[s];
+  const int64_t mo = t.mat_off[s];
+  double* zscale = zscale_all + t.ao_off[s];
+  __shared__ double d_l[BIG ? 1 : kMaxAO];
+  __shared__ double e_l[BIG ? 1 : kMaxAO];   // split off-diagonal (negligible entries zeroed)
+  __shared__ double e2_l[BIG ? 1 : kMaxAO];
+  __shared__ double lam_l[BIG ? 1 : kMaxAO];
+  double *d = d_l, *e = e_l, *e2 = e2_l, *lam = lam_l;
+  if constexpr (BIG) {
+    d = big + big_offset(t, s);  // d, e, e2, lam, rnk: 5 n <= kBigPerAO n doubles
+    e = d + n;
+    e2 = e + n;
+    lam = e2 + n;
+  }
+  __shared__ double red[16];
+  const int tid = threadIdx.x, nt = blockDim.x;
+  if (tid == 0) co.flag[s] = 0;
+  __shared__ int nsplit, next_j;
+  if (tid == 0) next_j = 0;
+  double pivmin;
+  const bool unsplit = eig_load(dall + t.ao_off[s], eall + t.ao_off[s], n, d, e, e2, red, nsplit, pivmin);
+  // the SCC round: the launch argument, or the device-resident counter of
+  // rounds enqueued ahead of the host (graph-captured rounds)
+  const int round = round_ptr ? *round_ptr : round_arg;
+  const bool have_old = round >= 1 && unsplit;
+  const bool guess_ok = round >= 2 && unsplit;
+  const double delta = guess_ok ? 2.0 * shift[s] : 0.0;
+  // whole-matrix Gershgorin bounds (used when T is unsplit)
+  __shared__ double gbound[3];
+  if (unsplit) eig_bounds(d, e, n, pivmin, red, gbound);
+  double dmax = 0.0;
+  {
+    EigState st;
+    bool busy = false;
+    for (;;) {
+      if (!busy) {
+        const int j = atomicAdd(&next_j, 1);
+        if (j >= n) break;
+        const double* wo = wall + t.ao_off[s];
+        const double g = have_old ? wo[j] : 0.0;
+        const double gp = (have_old && j > 0) ? wo[j - 1] : -1e300;
+        const double gn = (have_old && j + 1 < n) ? wo[j + 1] : 1e300;
+        busy = eig_start(st, j, d, e, n, pivmin, unsplit, gbound[0], gbound[1], gbound[2], guess_ok,
+                         g, gp, gn, delta, lam);
+        if (!busy) continue;
+      }
+      double x;
+      if (eig_step(st, d, e2, x)) {
+        lam[st.j] = x;
+        if (have_old) dmax = fmax(dmax, fabs(x - wall[t.ao_off[s] + st.j]));
+        busy = false;
+      }
     }
   }
+  // largest eigenvalue change of this round (block max), for the next round's brackets
+  for (int off = 32; off > 0; off >>= 1) dmax = fmax(dmax, __shfl_xor(dmax, off, 64));
+  __syncthreads();
+  if ((tid & 63) == 0) red[tid >> 6] = dmax;
+  __syncthreads();
+  if (tid == 0) {
+    double m = 0.0;
+    for (int w = 0; w < (nt >> 6); ++w) m = fmax(m, red[w]);
+    // first round: no change measured yet, take a generous bracket
+    shift[s] = have_old ? m : 1.0;
+  }
+  __syncthreads();
+
+  __shared__ int rnk_l[BIG ? 1 : kMaxAO];
+  int* rnk = BIG ? reinterpret_cast<int*>(lam + n) : rnk_l;
+  double* srt = e2;  // e2 is not needed after the eigenvalues
+  const int kocc = eig_occupations(t, s, n, lam, rnk, srt, wall + t.ao_off[s], fo);
+
+  // ---- eigenvectors: thread per cluster start ----
+  __shared__ double tnorm1;
+  if (unsplit) eig_norm1(d, e, n, red, tnorm1);
+  for (int j = tid; j < n; j += nt)
+    eig_vector(j, n, kocc, d, e, lam, rnk, unsplit, tnorm1, pivmin, sc, mo, Zall + mo, zscale, co, s, t.ao_off[s]);
 }
 
 // Block-wide maximum (blockDim.x <= 1024; red holds blockDim.x / 64 doubles).
@@ -3026,6 +3047,115 @@ __device__ __forceinline__ double block_max(double v, double* red) {
   for (int i = 1; i < nw; ++i) m = fmax(m, red[i]);
   __syncthreads();
   return m;
+}
+
+// 256 < n <= kEigSplitAO: the same three stages as launches of their own, so that
+// a system's eigenvalues and vectors spread over the chip: one wavefront per 64
+// eigenvalues, one block per system for ranks and occupations, one wavefront per
+// 64 vectors.  Between the launches the eigenvalues (in T's order) and ranks sit
+// in the system's slot of `lam_all` (the Y matrix, free until the
+// back-transformation).  Larger systems run k_tridiag_eigen<true>.
+//
+// Bound: the serial chains of a lane (about nine Sturm passes, four recurrences
+// of n rows).  Measured against one 256-thread block per system: 7.8 -> 1.5 ms
+// a launch at 1142 AOs (eigenvalues 0.82, occupations 0.16, vectors 0.49; a
+// geometry whose close eigenvalues need inverse iteration takes 3.1 for the
+// vectors), 0.74 -> 0.45 ms for 14 systems of 258-482 AOs.
+constexpr int kEigSplitAO = 2048;
+
+__global__ __launch_bounds__(64) void k_eig_values(Topo t, const int* order, const unsigned char* active,
+                                                   const double* dall, const double* eall, const double* wall,
+                                                   const double* shift, int round_arg, const int* round_ptr,
+                                                   double* lam_all) {
+  const int s = order[blockIdx.y];
+  if (active && !active[s]) return;
+  const int n = t.ao_off[s + 1] - t.ao_off[s];
+  if (64 * (int)blockIdx.x >= n) return;
+  __shared__ double d[kEigSplitAO], e[kEigSplitAO], e2[kEigSplitAO];
+  __shared__ double red[16], gbound[3];
+  __shared__ int nsplit;
+  double pivmin;
+  const bool unsplit = eig_load(dall + t.ao_off[s], eall + t.ao_off[s], n, d, e, e2, red, nsplit, pivmin);
+  if (unsplit) eig_bounds(d, e, n, pivmin, red, gbound);
+  const int round = round_ptr ? *round_ptr : round_arg;
+  const bool have_old = round >= 1 && unsplit, guess_ok = round >= 2 && unsplit;
+  const double delta = guess_ok ? 2.0 * shift[s] : 0.0;
+  double* lam = lam_all + t.mat_off[s];
+  const int j = 64 * blockIdx.x + threadIdx.x;
+  if (j >= n) return;
+  const double* wo = wall + t.ao_off[s];
+  EigState st;
+  if (!eig_start(st, j, d, e, n, pivmin, unsplit, gbound[0], gbound[1], gbound[2], guess_ok, have_old ? wo[j] : 0.0,
+                 have_old && j > 0 ? wo[j - 1] : -1e300, have_old && j + 1 < n ? wo[j + 1] : 1e300, delta, lam))
+    return;
+  double x;
+  while (!eig_step(st, d, e2, x)) {}
+  lam[j] = x;
+}
+
+__global__ __launch_bounds__(256) void k_eig_occupations(Topo t, const int* order, const unsigned char* active,
+                                                         const double* dall, const double* eall, double* wall,
+                                                         double* shift, int round_arg, const int* round_ptr,
+                                                         double* lam_all, FermiOut fo, ClusterOut co) {
+  const int s = order[blockIdx.x];
+  if (active && !active[s]) return;
+  const int n = t.ao_off[s + 1] - t.ao_off[s];
+  const int tid = threadIdx.x, nt = blockDim.x;
+  __shared__ double lam[kEigSplitAO], srt[kEigSplitAO];
+  __shared__ int rnk[kEigSplitAO];
+  __shared__ double red[16];
+  double* lam_g = lam_all + t.mat_off[s];
+  double* w = wall + t.ao_off[s];
+  const double* dg = dall + t.ao_off[s];
+  const double* eg = eall + t.ao_off[s];
+  if (tid == 0) co.flag[s] = 0;
+  const int round = round_ptr ? *round_ptr : round_arg;
+  // the largest eigenvalue change of this round, for the next round's brackets;
+  // a T that split gives none (its eigenvalues are not in ascending order)
+  double dmax = 0.0;
+  int cut = 0;
+  for (int i = tid; i < n; i += nt) {
+    lam[i] = lam_g[i];
+    if (round >= 1) dmax = fmax(dmax, fabs(lam[i] - w[i]));
+    if (i + 1 < n && eg[i] * eg[i] <= kEps * kEps * fabs(dg[i] * dg[i + 1]) + kSafeMin) cut = 1;
+  }
+  dmax = block_max(dmax, red);
+  const bool unsplit = !__syncthreads_or(cut);
+  if (tid == 0) shift[s] = round >= 1 && unsplit ? dmax : 1.0;
+  __syncthreads();
+  eig_occupations(t, s, n, lam, rnk, srt, w, fo);
+  int* rnk_g = reinterpret_cast<int*>(lam_g + n);
+  for (int i = tid; i < n; i += nt) rnk_g[i] = rnk[i];
+}
+
+__global__ __launch_bounds__(64) void k_eig_vectors(Topo t, const int* order, const unsigned char* active,
+                                                    const double* dall, const double* eall, const double* lam_all,
+                                                    double* Zall, EigenScratch sc, double* zscale_all,
+                                                    const int* kocc_all, ClusterOut co) {
+  const int s = order[blockIdx.y];
+  if (active && !active[s]) return;
+  const int n = t.ao_off[s + 1] - t.ao_off[s];
+  if (64 * (int)blockIdx.x >= n) return;
+  const int kocc = kocc_all[s];
+  __shared__ double d[kEigSplitAO], e[kEigSplitAO], lam[kEigSplitAO];  // lam holds e^2 first
+  __shared__ int rnk[kEigSplitAO];
+  __shared__ double red[16], tnorm1;
+  __shared__ int nsplit;
+  double pivmin;
+  const bool unsplit = eig_load(dall + t.ao_off[s], eall + t.ao_off[s], n, d, e, lam, red, nsplit, pivmin);
+  if (unsplit) eig_norm1(d, e, n, red, tnorm1);
+  const int64_t mo = t.mat_off[s];
+  const double* lam_g = lam_all + mo;
+  const int* rnk_g = reinterpret_cast<const int*>(lam_g + n);
+  for (int i = threadIdx.x; i < n; i += 64) {
+    lam[i] = lam_g[i];
+    rnk[i] = rnk_g[i];
+  }
+  __syncthreads();
+  const int j = 64 * blockIdx.x + threadIdx.x;
+  if (j < n)
+    eig_vector(j, n, kocc, d, e, lam, rnk, unsplit, tnorm1, pivmin, sc, mo, Zall + mo, zscale_all + t.ao_off[s], co, s,
+               t.ao_off[s]);
 }
 
 // Eigenvectors of the clusters k_tridiag_eigen hands over (more than
