@@ -1,0 +1,87 @@
+"""Atom-level gradients of systems above 32 atoms, a wavefront per atom.
+
+Sizes around the switch and around 64 atoms (one lane more than a wavefront), with
+point charges, against the oracle at the package's bars; reproducible mode against
+the default to its resolution; and, above 1024 atoms, where a block's sums of the
+three-body term no longer fit LDS, copies of one cluster too far apart to interact:
+each copy's forces are the single cluster's.
+"""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from xtbloom_amd import interface, library, workloads
+
+pytestmark = pytest.mark.gpu
+
+E_TOL, F_TOL = 1e-7, 1e-6
+
+
+def chain(n, rng):
+    """n atoms, hydrogen molecules 4 bohr apart on a square grid, one He when n is odd."""
+    z, xyz = [], []
+    for m in range(n // 2):
+        c = 4.0 * np.array([m % 4, (m // 4) % 4, m // 16]) + rng.normal(0.0, 0.1, 3)
+        u = rng.normal(size=3)
+        u *= 0.7 / np.linalg.norm(u)
+        z += [1, 1]
+        xyz += [c - u, c + u]
+    if n % 2:
+        z.append(2)
+        xyz.append(np.array([-4.0, -4.0, 0.0]))
+    return dict(Z=np.array(z, np.int32), xyz=np.array(xyz), charge=0.0, uhf=0)
+
+
+def run(batch, points=False, **kw):
+    ctx = interface.Context("hip", 0)
+    try:
+        if points:
+            kw.update(point_offsets=batch.point_offsets, point_positions=batch.point_positions,
+                      point_values=batch.point_charges, point_gammas=batch.point_gammas,
+                      flags=library.COMPUTE_ENERGY | library.COMPUTE_FORCES | library.COMPUTE_POINT_CHARGE_FORCES)
+        return interface.compute_arrays(ctx, batch.atom_offsets, batch.atomic_numbers, batch.positions,
+                                        batch.molecular_charges, batch.unpaired_electrons, **kw)
+    finally:
+        ctx.close()
+
+
+def test_switch_and_wavefront_edges_with_point_charges():
+    rng = np.random.default_rng(7)
+    systems = []
+    for n, m in [(32, 3), (33, 1), (34, 17), (63, 40), (64, 0), (65, 5), (130, 33)]:
+        s = chain(n, rng)
+        if m:
+            s.update(workloads.point_charges(s["xyz"], rng, m, 5.0, 7.0, gamma=0.5))
+        systems.append(s)
+    b = workloads.from_systems(systems)
+    print("case wide forces: 32..130 atoms with point charges", flush=True)
+    out = run(b, points=True)
+    ref = O.batch(b.atom_offsets, b.atomic_numbers, b.positions, b.molecular_charges, b.unpaired_electrons,
+                  point_offsets=b.point_offsets, pc_xyz=b.point_positions, pc_q=b.point_charges,
+                  pc_gamma=b.point_gammas, threads=4, want_point_gradient=True)
+    assert np.all(out.per_system_status == 0) and np.all(ref["status"] == 0)
+    assert np.abs(out.energies - ref["energies"]).max() <= E_TOL
+    assert np.abs(out.forces + ref["gradient"]).max() <= F_TOL
+    assert np.abs(out.point_charge_forces + ref["pc_gradient"]).max() <= F_TOL
+    # reproducible: up to 130^2 / 2 contributions to an atom, each within 2^-41
+    fixed = [run(b, points=True, determinism=library.DETERMINISM_REPRODUCIBLE) for _ in range(2)]
+    assert np.array_equal(fixed[0].forces, fixed[1].forces)
+    assert np.abs(fixed[0].forces - out.forces).max() <= 1e-7
+
+
+@pytest.mark.parametrize("reproducible", [False, True])
+def test_more_atoms_than_the_block_sums_hold(reproducible):
+    one = chain(40, np.random.default_rng(3))
+    copies = 26  # 1040 atoms
+    many = dict(Z=np.tile(one["Z"], copies), charge=0.0, uhf=0,
+                xyz=np.concatenate([one["xyz"] + np.array([0.0, 0.0, 150.0 * k]) for k in range(copies)]))
+    b = workloads.from_systems([many, one])
+    kw = dict(charge_tolerance=1e-8, energy_tolerance=1e-10)
+    if reproducible:
+        kw["determinism"] = library.DETERMINISM_REPRODUCIBLE
+    print("case wide forces: 1040 atoms, reproducible", reproducible, flush=True)
+    out = run(b, **kw)
+    assert np.all(out.per_system_status == 0)
+    # what is left between copies: quadrupoles 150 bohr apart, below 1e-9 in all
+    assert abs(out.energies[0] - copies * out.energies[1]) <= copies * E_TOL
+    assert np.abs(out.forces[:1040].reshape(copies, 40, 3) - out.forces[1040:]).max() <= F_TOL

@@ -610,6 +610,9 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
   int n_large = 0;  // systems above 256 AOs (a prefix of the size order)
   int n_xl = 0;     // systems above kMaxAO AOs (a prefix of that prefix)
   int n_huge = 0;   // systems above kEigSplitAO AOs (a prefix of that one)
+  // systems above kWideAtoms atoms are among the first n_wide of the size order
+  int n_wide = 0, wide_top = 0;
+  bool any_narrow = false;
   // back-transformation tasks of the systems above 2048, 1024, 512 and 256 AOs
   // (prefixes of `back`)
   size_t n_back[4] = {0, 0, 0, 0};
@@ -619,6 +622,12 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
     n_large += n > 256;
     n_xl += n > kMaxAO;
     n_huge += n > kEigSplitAO;
+    const int atoms = T.atom_off[s + 1] - T.atom_off[s];
+    if (atoms > kWideAtoms)
+      n_wide = i + 1;
+    else
+      any_narrow = true;
+    wide_top = std::max(wide_top, atoms);
     const int nt = (n + kTile - 1) / kTile;
     for (int a = 0; a < nt; ++a)
       for (int b = 0; b < nt; ++b) {
@@ -1520,26 +1529,46 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
       HIP_TRY(probe_end(kKForcePairs, 0.0, 24.0 * v2));  // reads P, W, S
     }
   }
+  const dim3 wide_atoms(n_wide, std::min((wide_top + 3) / 4, 8192));
   HIP_TRY(probe_begin(kKForceAtoms));
-  hipLaunchKernelGGL(k_force_atoms, dim3(B), dim3(512), 0, sm, t, d_order, d_valid, mx.x, d_qat,
-                     d_cnd4, d_mrad, d_dmrad, d_gam, d_w4, d_dw4, d_dedcn, d_dedcn4, d_grad,
-                     d_erep, d_pcgrad, d_dedq);
+  if (n_wide > 0) {
+    auto stage = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, wide_atoms, dim3(256), 0, sm, t, d_order, d_valid, mx.x, d_qat, d_cnd4, d_mrad,
+                         d_dmrad, d_gam, d_w4, d_dw4, d_dedcn, d_dedcn4, d_grad, d_c6pair, d_pcgrad, d_dedq);
+    };
+    stage(k_wide_atoms<1>);
+    stage(k_wide_atoms<2>);
+    stage(k_wide_atoms<3>);
+  }
+  if (any_narrow)
+    hipLaunchKernelGGL(k_force_atoms, dim3(B), dim3(512), 0, sm, t, d_order, d_valid, mx.x, d_qat,
+                       d_cnd4, d_mrad, d_dmrad, d_gam, d_w4, d_dw4, d_dedcn, d_dedcn4, d_grad,
+                       d_erep, d_pcgrad, d_dedq);
   HIP_TRY(probe_end(kKForceAtoms, 0.0, 0.0));
   HIP_TRY(probe_begin(kKForceAtm));
-  if (opt.reproducible) {
-    if (n_xl > 0)
-      hipLaunchKernelGGL((k_force_atm<true, true>), dim3(n_xl), dim3(512), 0, sm, t, d_order, d_valid, d_cnd4,
-                         d_w4, d_dw4, d_c6pair, d_dedcn4, d_grad, d_eatm, d_xl);
-    if (n_xl < B)
-      hipLaunchKernelGGL((k_force_atm<true, false>), dim3(B - n_xl), dim3(512), 0, sm, t, d_order + n_xl,
-                         d_valid, d_cnd4, d_w4, d_dw4, d_c6pair, d_dedcn4, d_grad, d_eatm, d_xl);
-  } else {
-    if (n_xl > 0)
-      hipLaunchKernelGGL((k_force_atm<false, true>), dim3(n_xl), dim3(512), 0, sm, t, d_order, d_valid, d_cnd4,
-                         d_w4, d_dw4, d_c6pair, d_dedcn4, d_grad, d_eatm, d_xl);
-    if (n_xl < B)
-      hipLaunchKernelGGL((k_force_atm<false, false>), dim3(B - n_xl), dim3(512), 0, sm, t, d_order + n_xl,
-                         d_valid, d_cnd4, d_w4, d_dw4, d_c6pair, d_dedcn4, d_grad, d_eatm, d_xl);
+  if (n_wide > 0) {
+    const int64_t wide_pairs = (int64_t)wide_top * wide_top;
+    hipLaunchKernelGGL(k_wide_pairs, dim3(n_wide, (int)std::min<int64_t>((wide_pairs + 255) / 256, 8192)), dim3(256),
+                       0, sm, t, d_order, d_valid, d_w4, d_dw4, d_c6pair, d_erep);
+    // one block per part: the blocks' energies have slots of their own
+    const dim3 parts(n_wide, wide_parts(wide_top));
+    if (opt.reproducible) {
+      hipLaunchKernelGGL(k_wide_triples<true>, parts, dim3(256), 0, sm, t, d_order, d_valid, d_c6pair);
+      hipLaunchKernelGGL(k_wide_atm<true>, wide_atoms, dim3(256), 0, sm, t, d_order, d_valid, d_c6pair, d_dedcn4,
+                         d_grad, d_eatm);
+    } else {
+      hipLaunchKernelGGL(k_wide_triples<false>, parts, dim3(256), 0, sm, t, d_order, d_valid, d_c6pair);
+      hipLaunchKernelGGL(k_wide_atm<false>, wide_atoms, dim3(256), 0, sm, t, d_order, d_valid, d_c6pair, d_dedcn4,
+                         d_grad, d_eatm);
+    }
+  }
+  if (any_narrow) {
+    if (opt.reproducible)
+      hipLaunchKernelGGL(k_force_atm<true>, dim3(B), dim3(512), 0, sm, t, d_order, d_valid, d_cnd4, d_w4, d_dw4,
+                         d_c6pair, d_dedcn4, d_grad, d_eatm);
+    else
+      hipLaunchKernelGGL(k_force_atm<false>, dim3(B), dim3(512), 0, sm, t, d_order, d_valid, d_cnd4, d_w4, d_dw4,
+                         d_c6pair, d_dedcn4, d_grad, d_eatm);
   }
   HIP_TRY(probe_end(kKForceAtm, 0.0, 0.0));
   HIP_TRY(hipGetLastError());

@@ -632,6 +632,136 @@ __device__ void aes2_pair_vjp(const Topo& t, int i, int j, const double* mrad, c
   dcn_j = 0.5 * dE_drho * dmrad[j];
 }
 
+// Atom-level gradient terms of atom a from partners b = a0 + lb, a0 + lb + step, ...
+// below a0 + le.  g: dE/dR_a.
+
+// AES2 VJP (both pair orders); dc: dE/dCN_a
+__device__ __forceinline__ void force_aes2(const Topo& t, int a, int a0, int lb, int le, int step, const double* qat,
+                                           const double* mrad, const double* dmrad, const double* dip,
+                                           const double* quad, double (&g)[3], double& dc) {
+  for (int b = a0 + lb; b < a0 + le; b += step) {
+    if (b == a) continue;
+    const int i = min(a, b), j = max(a, b);
+    double gi[3], dci, dcj;
+    aes2_pair_vjp(t, i, j, mrad, dmrad, qat, dip, quad, a0, gi, dci, dcj);
+    const double sg = (a == i) ? 1.0 : -1.0;
+    for (int c = 0; c < 3; ++c) g[c] += sg * gi[c];
+    dc += (a == i) ? dci : dcj;
+  }
+}
+
+// D4 two-body explicit gradient; d4cn: D4-CN adjoint of a
+__device__ __forceinline__ void force_d4(const Topo& t, int a, int a0, int lb, int le, int step, const double* w4,
+                                         const double* dw4c, double (&g)[3], double& d4cn) {
+  const double* ra = t.xyz + 3 * a;
+  for (int b = a0 + lb; b < a0 + le; b += step) {
+    if (b == a) continue;
+    const double* rb = t.xyz + 3 * b;
+    const double r[3] = {ra[0] - rb[0], ra[1] - rb[1], ra[2] - rb[2]};
+    const double r2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
+    double damp, ddamp;
+    d4_damping(t, a, b, r2, damp, ddamp);
+    if (damp == 0.0) continue;
+    const double c6 = d4_contract(t, a, b, w4 + kD4MaxRef * a, w4 + kD4MaxRef * b);
+    const double dc6 = d4_contract(t, a, b, dw4c + kD4MaxRef * a, w4 + kD4MaxRef * b);
+    for (int c = 0; c < 3; ++c) g[c] += -c6 * ddamp * r[c];
+    d4cn -= dc6 * damp;
+  }
+}
+
+// CN chains and repulsion (symmetric pair formulas); erp: repulsion energy of a < b
+__device__ __forceinline__ void force_cn_rep(const Topo& t, int a, int a0, int lb, int le, int step,
+                                             const double* dedcn, const double* dedcn4, double (&g)[3],
+                                             double& erp) {
+  const double* ra = t.xyz + 3 * a;
+  for (int b = a0 + lb; b < a0 + le; b += step) {
+    if (b == a) continue;
+    const double* rb = t.xyz + 3 * b;
+    const double r[3] = {ra[0] - rb[0], ra[1] - rb[1], ra[2] - rb[2]};
+    const double r2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
+    const double rr = sqrt(r2);
+    double sc = 0.0;
+    if (r2 <= 625.0) {
+      double val, der;
+      dexp_count(rr, t.at_cnrad[a] + t.at_cnrad[b], val, der);
+      sc += (dedcn[a] + dedcn[b]) * der / rr;
+      // repulsion (reference repulsion.cpp:127-176)
+      const bool light = t.Z[a] <= 2 && t.Z[b] <= 2;
+      const double k = light ? 1.0 : 1.5;
+      const double rk = light ? rr : rr * sqrt(rr);
+      const double al = t.at_sqrt_arep[a] * t.at_sqrt_arep[b];
+      const double pe = t.at_zeff[a] * t.at_zeff[b] * exp(-al * rk) / rr;
+      if (a < b) erp += pe;
+      sc -= (al * k * rk + 1.0) * pe / r2;
+    }
+    if (r2 <= 900.0) {
+      double val, der;
+      d4_cn_count(t, a, b, rr, val, der);
+      sc += (dedcn4[a] + dedcn4[b]) * der / rr;
+    }
+    for (int c = 0; c < 3; ++c) g[c] += sc * r[c];
+  }
+}
+
+// ES2 at fixed q: -q_s q_t Gamma^3 (R_A - R_C) per shell pair on different atoms,
+// over the shells s0 + lb, ...
+__device__ __forceinline__ void force_es2(const Topo& t, int a, int s0, int ns, int lb, int le, int step,
+                                          const double* qsh, const double* Gm, double (&g)[3]) {
+  const double* ra = t.xyz + 3 * a;
+  for (int si = t.atom_sh0[a]; si < t.atom_sh0[a + 1]; ++si) {
+    for (int sj = s0 + lb; sj < s0 + le; sj += step) {
+      const int C = t.sh_atom[sj];
+      if (C == a) continue;
+      const double gm = Gm[(int64_t)(si - s0) * ns + (sj - s0)];
+      const double f = -qsh[si - s0] * qsh[sj - s0] * gm * gm * gm;
+      for (int c = 0; c < 3; ++c) g[c] += f * (ra[c] - t.xyz[3 * C + c]);
+    }
+  }
+}
+
+// External point charges p0 + first, p0 + first + step, ... on atom a
+// (reference external_point_charges.cpp:389-491)
+__device__ __forceinline__ void force_pc_atom(const Topo& t, int a, int s0, int p0, int p1, int first, int step,
+                                              const double* qsh, double (&g)[3]) {
+  for (int sh = t.atom_sh0[a]; sh < t.atom_sh0[a + 1]; ++sh) {
+    const double qs = qsh[sh - s0];
+    for (int p = p0 + first; p < p1; p += step) {
+      const double d[3] = {t.xyz[3 * a] - t.pc_xyz[3 * p], t.xyz[3 * a + 1] - t.pc_xyz[3 * p + 1],
+                           t.xyz[3 * a + 2] - t.pc_xyz[3 * p + 2]};
+      if (d[0] == 0.0 && d[1] == 0.0 && d[2] == 0.0) continue;
+      const double ia = 2.0 / (t.sh_eta[sh] + t.pc_gam[p]);
+      const double rs2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2] + ia * ia;
+      const double rs = sqrt(rs2);
+      const double fs = qs * t.pc_q[p] / (rs2 * rs);
+      for (int c = 0; c < 3; ++c) g[c] -= fs * d[c];
+    }
+  }
+}
+
+// the shells sb, sb + step, ... < s1 on point charge p; dq: dE/dq_p
+__device__ __forceinline__ void force_pc(const Topo& t, int p, int s0, int sb, int s1, int step, const double* qsh,
+                                         double (&g)[3], double& dq) {
+  for (int sh = sb; sh < s1; sh += step) {
+    const int a = t.sh_atom[sh];
+    const double d[3] = {t.xyz[3 * a] - t.pc_xyz[3 * p], t.xyz[3 * a + 1] - t.pc_xyz[3 * p + 1],
+                         t.xyz[3 * a + 2] - t.pc_xyz[3 * p + 2]};
+    const double ia = 2.0 / (t.sh_eta[sh] + t.pc_gam[p]);
+    const double rs2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2] + ia * ia;
+    const double rs = sqrt(rs2);
+    dq += qsh[sh - s0] / rs;
+    if (d[0] == 0.0 && d[1] == 0.0 && d[2] == 0.0) continue;
+    const double fs = qsh[sh - s0] * t.pc_q[p] / (rs2 * rs);
+    for (int c = 0; c < 3; ++c) g[c] += fs * d[c];
+  }
+}
+
+// Systems of more than kWideAtoms atoms take their atom-level gradients from the
+// kernels k_wide_* (a wavefront per atom, blocks over slices of a system); the
+// others from k_force_atoms and k_force_atm (one block per system), where the
+// two launches cost less than the seven of the wide path.
+constexpr int kWideAtoms = 32;
+constexpr int kAtmFields = 5;  // pair tables of the three-body term (k_force_atm)
+
 // Per-system atom-level gradients: AES2 VJP, GFN2-CN chain (H0 + AES2 adjoints),
 // ES2, D4 two-body (+ D4-CN chain), repulsion energy/gradient and point charges.
 __global__ __launch_bounds__(512) void k_force_atoms(Topo t, const int* order,
@@ -645,6 +775,7 @@ __global__ __launch_bounds__(512) void k_force_atoms(Topo t, const int* order,
   const int s = order[blockIdx.x];
   if (!valid[s]) return;
   const int a0 = t.atom_off[s], a1 = t.atom_off[s + 1], N = a1 - a0;
+  if (N > kWideAtoms) return;
   const int s0 = t.shell_off[s], s1 = t.shell_off[s + 1], ns = s1 - s0;
   const double* x = xstate + t.vec_off[s];
   const double* qsh = x;
@@ -656,26 +787,17 @@ __global__ __launch_bounds__(512) void k_force_atoms(Topo t, const int* order,
   // the potentials), partial results combined with xor shuffles.
   const int G = pair_lanes(N, nt), gl = tid & (G - 1), per = nt / G;
   const int L = (N + G - 1) / G, Ls = (ns + G - 1) / G;
+  const int lb = gl * L, le = min(N, (gl + 1) * L);
   auto lanes_sum = [&](double& v) __attribute__((always_inline)) {
     for (int off = G >> 1; off > 0; off >>= 1) v += __shfl_xor(v, off);
   };
-  // phase 1: AES2 VJP (per atom, both pair orders) and D4 weights at the converged charges
+  // phase 1: AES2 VJP and D4 weights at the converged charges
   for (int base = 0; base < N; base += per) {
     const int la = base + tid / G;
     const bool act = la < N;
     const int a = a0 + (act ? la : 0);
     double g[3] = {0, 0, 0}, dc = 0.0;
-    if (act) {
-      for (int b = a0 + gl * L; b < a0 + min(N, (gl + 1) * L); ++b) {
-        if (b == a) continue;
-        const int i = min(a, b), j = max(a, b);
-        double gi[3], dci, dcj;
-        aes2_pair_vjp(t, i, j, mrad, dmrad, qat, dip, quad, a0, gi, dci, dcj);
-        const double sg = (a == i) ? 1.0 : -1.0;
-        for (int c = 0; c < 3; ++c) g[c] += sg * gi[c];
-        dc += (a == i) ? dci : dcj;
-      }
-    }
+    if (act) force_aes2(t, a, a0, lb, le, 1, qat, mrad, dmrad, dip, quad, g, dc);
     for (int c = 0; c < 3; ++c) lanes_sum(g[c]);
     lanes_sum(dc);
     if (act && gl == 0) {
@@ -685,28 +807,13 @@ __global__ __launch_bounds__(512) void k_force_atoms(Topo t, const int* order,
     }
   }
   __syncthreads();
-  // phase 2: D4 two-body explicit gradient and D4-CN adjoint
+  // phase 2: D4 two-body
   for (int base = 0; base < N; base += per) {
     const int la = base + tid / G;
     const bool act = la < N;
     const int a = a0 + (act ? la : 0);
-    const double* ra = t.xyz + 3 * a;
     double g[3] = {0, 0, 0}, d4cn = 0.0;
-    if (act) {
-      for (int b = a0 + gl * L; b < a0 + min(N, (gl + 1) * L); ++b) {
-        if (b == a) continue;
-        const double* rb = t.xyz + 3 * b;
-        const double r[3] = {ra[0] - rb[0], ra[1] - rb[1], ra[2] - rb[2]};
-        const double r2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
-        double damp, ddamp;
-        d4_damping(t, a, b, r2, damp, ddamp);
-        if (damp == 0.0) continue;
-        const double c6 = d4_contract(t, a, b, w4 + kD4MaxRef * a, w4 + kD4MaxRef * b);
-        const double dc6 = d4_contract(t, a, b, dw4c + kD4MaxRef * a, w4 + kD4MaxRef * b);
-        for (int c = 0; c < 3; ++c) g[c] += -c6 * ddamp * r[c];
-        d4cn -= dc6 * damp;
-      }
-    }
+    if (act) force_d4(t, a, a0, lb, le, 1, w4, dw4c, g, d4cn);
     for (int c = 0; c < 3; ++c) lanes_sum(g[c]);
     lanes_sum(d4cn);
     if (act && gl == 0) {
@@ -715,53 +822,17 @@ __global__ __launch_bounds__(512) void k_force_atoms(Topo t, const int* order,
     }
   }
   __syncthreads();
-  // phase 3: CN chains, ES2, repulsion (per atom, symmetric pair formulas)
+  // phase 3: CN chains, ES2, repulsion
   double erp = 0.0;
   const double* Gm = gam + t.gam_off[s];
   for (int base = 0; base < N; base += per) {
     const int la = base + tid / G;
     const bool act = la < N;
     const int a = a0 + (act ? la : 0);
-    const double* ra = t.xyz + 3 * a;
     double g[3] = {0, 0, 0};
     if (act) {
-      for (int b = a0 + gl * L; b < a0 + min(N, (gl + 1) * L); ++b) {
-        if (b == a) continue;
-        const double* rb = t.xyz + 3 * b;
-        const double r[3] = {ra[0] - rb[0], ra[1] - rb[1], ra[2] - rb[2]};
-        const double r2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
-        const double rr = sqrt(r2);
-        double sc = 0.0;
-        if (r2 <= 625.0) {
-          double val, der;
-          dexp_count(rr, t.at_cnrad[a] + t.at_cnrad[b], val, der);
-          sc += (dedcn[a] + dedcn[b]) * der / rr;
-          // repulsion (reference repulsion.cpp:127-176)
-          const bool light = t.Z[a] <= 2 && t.Z[b] <= 2;
-          const double k = light ? 1.0 : 1.5;
-          const double rk = light ? rr : rr * sqrt(rr);
-          const double al = t.at_sqrt_arep[a] * t.at_sqrt_arep[b];
-          const double pe = t.at_zeff[a] * t.at_zeff[b] * exp(-al * rk) / rr;
-          if (a < b) erp += pe;
-          sc -= (al * k * rk + 1.0) * pe / r2;
-        }
-        if (r2 <= 900.0) {
-          double val, der;
-          d4_cn_count(t, a, b, rr, val, der);
-          sc += (dedcn4[a] + dedcn4[b]) * der / rr;
-        }
-        for (int c = 0; c < 3; ++c) g[c] += sc * r[c];
-      }
-      // ES2 at fixed q: -q_s q_t Gamma^3 (R_A - R_C) per shell pair on different atoms
-      for (int si = t.atom_sh0[a]; si < t.atom_sh0[a + 1]; ++si) {
-        for (int sj = s0 + gl * Ls; sj < s0 + min(ns, (gl + 1) * Ls); ++sj) {
-          const int C = t.sh_atom[sj];
-          if (C == a) continue;
-          const double gm = Gm[(si - s0) * ns + (sj - s0)];
-          const double f = -qsh[si - s0] * qsh[sj - s0] * gm * gm * gm;
-          for (int c = 0; c < 3; ++c) g[c] += f * (ra[c] - t.xyz[3 * C + c]);
-        }
-      }
+      force_cn_rep(t, a, a0, lb, le, 1, dedcn, dedcn4, g, erp);
+      force_es2(t, a, s0, ns, gl * Ls, min(ns, (gl + 1) * Ls), 1, qsh, Gm, g);
     }
     for (int c = 0; c < 3; ++c) lanes_sum(g[c]);
     if (act && gl == 0)
@@ -769,40 +840,17 @@ __global__ __launch_bounds__(512) void k_force_atoms(Topo t, const int* order,
   }
   erp = block_sum(erp, red);
   if (tid == 0) erep[s] = erp;
-  // phase 4: external point charges (reference external_point_charges.cpp:389-491)
+  // phase 4: external point charges
   const int p0 = t.pc_off[s], p1 = t.pc_off[s + 1];
   if (p1 > p0) {
     for (int a = a0 + tid; a < a1; a += nt) {
       double g[3] = {0, 0, 0};
-      for (int sh = t.atom_sh0[a]; sh < t.atom_sh0[a + 1]; ++sh) {
-        const double qs = qsh[sh - s0];
-        for (int p = p0; p < p1; ++p) {
-          const double d[3] = {t.xyz[3 * a] - t.pc_xyz[3 * p], t.xyz[3 * a + 1] - t.pc_xyz[3 * p + 1],
-                               t.xyz[3 * a + 2] - t.pc_xyz[3 * p + 2]};
-          if (d[0] == 0.0 && d[1] == 0.0 && d[2] == 0.0) continue;
-          const double ia = 2.0 / (t.sh_eta[sh] + t.pc_gam[p]);
-          const double rs2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2] + ia * ia;
-          const double rs = sqrt(rs2);
-          const double fs = qs * t.pc_q[p] / (rs2 * rs);
-          for (int c = 0; c < 3; ++c) g[c] -= fs * d[c];
-        }
-      }
+      force_pc_atom(t, a, s0, p0, p1, 0, 1, qsh, g);
       for (int c = 0; c < 3; ++c) grad[3 * a + c] += g[c];
     }
     for (int p = p0 + tid; p < p1; p += nt) {
       double g[3] = {0, 0, 0}, dq = 0.0;
-      for (int sh = s0; sh < s1; ++sh) {
-        const int a = t.sh_atom[sh];
-        const double d[3] = {t.xyz[3 * a] - t.pc_xyz[3 * p], t.xyz[3 * a + 1] - t.pc_xyz[3 * p + 1],
-                             t.xyz[3 * a + 2] - t.pc_xyz[3 * p + 2]};
-        const double ia = 2.0 / (t.sh_eta[sh] + t.pc_gam[p]);
-        const double rs2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2] + ia * ia;
-        const double rs = sqrt(rs2);
-        dq += qsh[sh - s0] / rs;
-        if (d[0] == 0.0 && d[1] == 0.0 && d[2] == 0.0) continue;
-        const double fs = qsh[sh - s0] * t.pc_q[p] / (rs2 * rs);
-        for (int c = 0; c < 3; ++c) g[c] += fs * d[c];
-      }
+      force_pc(t, p, s0, s0, s1, 1, qsh, g, dq);
       for (int c = 0; c < 3; ++c) pc_grad[3 * p + c] = g[c];
       dedq[p] = dq;
     }
@@ -816,6 +864,83 @@ __global__ __launch_bounds__(512) void k_force_atoms(Topo t, const int* order,
   }
 }
 
+// The same terms for systems of more than kWideAtoms atoms, a wavefront per atom
+// and four atoms per block: STAGE 1 is phase 1 above, 2 is phase 2, 3 the rest.
+// The stages are launches because each needs every atom's result of the one
+// before.  STAGE 3 also leaves the D4 weights at zero charge for the three-body
+// term, and clears the diagonals of its pair tables (see k_wide_pairs).
+// Bound: the latency of a lane's partner loop (exp, erf, the reference table),
+// one to four partners long up to 256 atoms.  k_force_atoms took 149 us for 62
+// atoms and 5.0 ms for 572, the stages take 25, 15 and 21 us for 62.
+template <int STAGE>
+__global__ __launch_bounds__(256) void k_wide_atoms(Topo t, const int* order, const unsigned char* valid,
+                                                    const double* xstate, const double* qat, const double* cnd4,
+                                                    const double* mrad, const double* dmrad, const double* gam,
+                                                    double* w4, double* dw4c, double* dedcn, double* dedcn4,
+                                                    double* grad, double* pairbuf, double* pc_grad, double* dedq) {
+  const int s = order[blockIdx.x];
+  if (!valid[s]) return;
+  const int a0 = t.atom_off[s], N = t.atom_off[s + 1] - a0;
+  if (N <= kWideAtoms) return;
+  const int s0 = t.shell_off[s], s1 = t.shell_off[s + 1], ns = s1 - s0;
+  const double* qsh = xstate + t.vec_off[s];
+  const double* dip = qsh + ns;
+  const double* quad = dip + 3 * N;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t NN = (int64_t)N * N;
+  const int p0 = t.pc_off[s], p1 = t.pc_off[s + 1];
+  for (int la = blockIdx.y * 4 + wv; la < N; la += gridDim.y * 4) {
+    const int a = a0 + la;
+    double g[3] = {0, 0, 0};
+    if constexpr (STAGE == 1) {
+      double dc = 0.0;
+      force_aes2(t, a, a0, lane, N, 64, qat, mrad, dmrad, dip, quad, g, dc);
+      dc = wave_sum(dc);
+      if (lane == 0) {
+        dedcn[a] += dc;
+        d4_weights(t, a, cnd4[a], qat[a], w4 + kD4MaxRef * a, dw4c + kD4MaxRef * a, nullptr);
+      }
+    } else if constexpr (STAGE == 2) {
+      double d4cn = 0.0;
+      force_d4(t, a, a0, lane, N, 64, w4, dw4c, g, d4cn);
+      d4cn = wave_sum(d4cn);
+      if (lane == 0) dedcn4[a] = d4cn;
+    } else {
+      double erp = 0.0;
+      force_cn_rep(t, a, a0, lane, N, 64, dedcn, dedcn4, g, erp);
+      force_es2(t, a, s0, ns, lane, ns, 64, qsh, gam + t.gam_off[s], g);
+      if (p1 > p0) force_pc_atom(t, a, s0, p0, p1, lane, 64, qsh, g);
+      erp = wave_sum(erp);
+      if (lane == 0) {
+        // explicit force of a uniform field on the atomic charges, dE/dR_A = -q_A E
+        if (t.field)
+          for (int c = 0; c < 3; ++c) g[c] = fma(-qat[a], t.field[3 * s + c], g[c]);
+        d4_weights(t, a, cnd4[a], 0.0, w4 + kD4MaxRef * a, dw4c + kD4MaxRef * a, nullptr);
+      }
+      if (lane < 5) pairbuf[kAtmFields * t.apair_off[s] + lane * NN + (int64_t)la * N + la] = lane == 4 ? erp : 0.0;
+    }
+    for (int c = 0; c < 3; ++c) g[c] = wave_sum(g[c]);
+    if (lane == 0)
+      for (int c = 0; c < 3; ++c) grad[3 * a + c] += g[c];
+  }
+  if constexpr (STAGE == 3) {
+    // 16 lanes per point charge, 16 charges per block and trip
+    const int np = p1 - p0, l16 = threadIdx.x & 15;
+    for (int lp = blockIdx.y * 16 + (threadIdx.x >> 4); lp - (int)(threadIdx.x >> 4) < np; lp += gridDim.y * 16) {
+      const bool act = lp < np;
+      const int p = p0 + (act ? lp : 0);
+      double g[3] = {0, 0, 0}, dq = 0.0;
+      if (act) force_pc(t, p, s0, s0 + l16, s1, 16, qsh, g, dq);
+      for (int c = 0; c < 3; ++c) g[c] = row16_sum(g[c]);
+      dq = row16_sum(dq);
+      if (act && l16 == 0) {
+        for (int c = 0; c < 3; ++c) pc_grad[3 * p + c] = g[c];
+        dedq[p] = dq;
+      }
+    }
+  }
+}
+
 // D4 three-body ATM energy and gradient with zero-charge weights
 // (reference d4.cpp:1120-1362).  Every factor of a triple's term that belongs
 // to one pair is computed once per ordered pair and staged (structure of
@@ -826,34 +951,75 @@ __global__ __launch_bounds__(512) void k_force_atoms(Topo t, const int* order,
 // and sqrt|C6_ij C6_ik C6_jk| = sc_ij sc_ik sc_jk: a triple needs no power,
 // square root or division except the damping's reciprocal.  One thread per pair
 // (j, k), j > k, loops over i > j, so the lanes of a wavefront share the loop
-// length; gradient and CN adjoint of i go to LDS atomics (one system per block,
-// at most kMaxAO atoms), those of j and k stay in registers.  The D4-CN chain
-// finishes the kernel.
+// length; gradient and CN adjoint of i go to LDS atomics (one system of at most
+// kWideAtoms atoms per block), those of j and k stay in registers.  The D4-CN
+// chain finishes the kernel.
 // FIX: the LDS sums of the i-atom adjoints run in fixed point (reproducible
-// mode), so their value does not depend on the order of the LDS atomics.
-// BIG: systems above kMaxAO AOs (and so possibly above kMaxAO atoms), with the
-// per-atom sums and coordinates in their global slice of `big`.
-constexpr int kAtmFields = 5;
+// mode), so their value does not depend on the order of the LDS atom// one ordered pair's entries of the tables, NN apart
+__device__ __forceinline__ void atm_pair(const Topo& t, int a0, int lx, int ly, const double* w4, const double* dw4c,
+                                         double* tab, int64_t NN) {
+  const int x = a0 + lx, y = a0 + ly;
+  const double d0 = t.xyz[3 * y] - t.xyz[3 * x], d1 = t.xyz[3 * y + 1] - t.xyz[3 * x + 1],
+               d2 = t.xyz[3 * y + 2] - t.xyz[3 * x + 2];
+  const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
+  const double r = sqrt(r2);
+  const double c6 = d4_contract(t, x, y, w4 + kD4MaxRef * x, w4 + kD4MaxRef * y);
+  const double dc6 = d4_contract(t, x, y, dw4c + kD4MaxRef * x, w4 + kD4MaxRef * y);
+  tab[0] = r2;
+  tab[NN] = 1.0 / r;
+  tab[2 * NN] = pow(d4_r0(t, x, y) / r, 16.0 / 3.0);
+  tab[3 * NN] = sqrt(fabs(c6));
+  tab[4 * NN] = dc6 / c6;
+}
 
-template <bool FIX, bool BIG>
+// One triple's term (minus its energy) from its pair factors; rp: product of the
+// three q, sc: of the three sc; dg: pair gradients along ij, ik, jk.
+__device__ __forceinline__ double atm_triple(double r2ij, double r2ik, double r2jk, double irij, double irik,
+                                             double irjk, double rp, double sc, const double* xi, const double* xj,
+                                             const double* xk, double (&dg)[3][3]) {
+  const double ir1 = irij * irik * irjk;
+  const double ir3 = ir1 * ir1 * ir1, ir5 = ir3 * ir1 * ir1;
+  const double damp = 1.0 / (1.0 + 6.0 * rp);
+  const double ang = 0.375 * (r2ij + r2jk - r2ik) * (r2ij - r2jk + r2ik) * (-r2ij + r2jk + r2ik) * ir5 + ir3;
+  const double c9 = -5.0 * sc;
+  const double de = ang * damp * c9;
+  const double ddamp = -2.0 * 16.0 * rp * damp * damp;
+  const double tg[3] = {r2ij, r2ik, r2jk}, o1[3] = {r2jk, r2jk, r2ik}, o2[3] = {r2ik, r2ij, r2ij};
+  const double irr[3] = {irij, irik, irjk};
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    const double T = tg[q], a = o1[q], b = o2[q];
+    const double dang = -0.375 * (T * T * T + T * T * (a + b) + T * (3.0 * a * a + 2.0 * a * b + 3.0 * b * b) -
+                                  5.0 * (a - b) * (a - b) * (a + b)) * ir5;
+    const double scq = c9 * (-dang * damp + ang * ddamp) * (irr[q] * irr[q]);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) dg[q][c] = scq * (q == 0 ? xj[c] - xi[c] : q == 1 ? xk[c] - xi[c] : xk[c] - xj[c]);
+  }
+  return de;
+}
+
+// pair (j, k), j > k, at p = j (j-1)/2 + k
+__device__ __forceinline__ void triangle_pair(int64_t p, int& lj, int& lk) {
+  lj = (int)((1.0 + sqrt(1.0 + 8.0 * (double)p)) * 0.5);
+  while ((int64_t)lj * (lj - 1) / 2 > p) --lj;
+  while ((int64_t)(lj + 1) * lj / 2 <= p) ++lj;
+  lk = (int)(p - (int64_t)lj * (lj - 1) / 2);
+}
+
+template <bool FIX>
 __global__ __launch_bounds__(512) void k_force_atm(Topo t, const int* order, const unsigned char* valid,
                                                    const double* cnd4, double* w4, double* dw4c,
                                                    double* pairbuf, double* dedcn4, double* grad,
-                                                   double* eatm, double* big) {
+                                                   double* eatm) {
   const int s = order[blockIdx.x];
   if (!valid[s]) return;
   const int a0 = t.atom_off[s], a1 = t.atom_off[s + 1], N = a1 - a0;
+  if (N > kWideAtoms) return;
   const int tid = threadIdx.x, nt = blockDim.x;
   __shared__ double red[16];
-  __shared__ double gsh_l[BIG ? 1 : 3 * kMaxAO];
-  __shared__ double csh_l[BIG ? 1 : kMaxAO];
-  __shared__ double xs_l[BIG ? 1 : 3 * kMaxAO];
-  double *gsh = gsh_l, *csh = csh_l, *xs = xs_l;
-  if constexpr (BIG) {
-    gsh = big + big_offset(t, s);  // 7 N <= kBigPerAO n doubles
-    csh = gsh + 3 * N;
-    xs = csh + N;
-  }
+  __shared__ double gsh[3 * kWideAtoms];
+  __shared__ double csh[kWideAtoms];
+  __shared__ double xs[3 * kWideAtoms];
   const int64_t NN = (int64_t)N * N;
   double* pr2 = pairbuf + kAtmFields * t.apair_off[s];
   double* pir = pr2 + NN;
@@ -870,22 +1036,10 @@ __global__ __launch_bounds__(512) void k_force_atm(Topo t, const int* order, con
     csh[la] = 0.0;
   }
   __syncthreads();
-  const double ex3 = 16.0 / 3.0;
   for (int64_t idx = tid; idx < NN; idx += nt) {
     const int lx = (int)(idx / N), ly = (int)(idx % N);
     if (lx == ly) continue;
-    const int x = a0 + lx, y = a0 + ly;
-    const double d0 = xs[3 * ly] - xs[3 * lx], d1 = xs[3 * ly + 1] - xs[3 * lx + 1],
-                 d2 = xs[3 * ly + 2] - xs[3 * lx + 2];
-    const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
-    const double r = sqrt(r2);
-    const double c6 = d4_contract(t, x, y, w4 + kD4MaxRef * x, w4 + kD4MaxRef * y);
-    const double dc6 = d4_contract(t, x, y, dw4c + kD4MaxRef * x, w4 + kD4MaxRef * y);
-    pr2[idx] = r2;
-    pir[idx] = 1.0 / r;
-    pq[idx] = pow(d4_r0(t, x, y) / r, ex3);
-    psc[idx] = sqrt(fabs(c6));
-    pdc[idx] = dc6 / c6;
+    atm_pair(t, a0, lx, ly, w4, dw4c, pr2 + idx, NN);
   }
   __syncthreads();
   double e = 0.0;
@@ -893,48 +1047,22 @@ __global__ __launch_bounds__(512) void k_force_atm(Topo t, const int* order, con
   // busy, and consecutive lanes share j and with it the length of the i loop
   const int64_t ntri = (int64_t)N * (N - 1) / 2;
   for (int64_t p = tid; p < ntri; p += nt) {
-    int lj = (int)((1.0 + sqrt(1.0 + 8.0 * (double)p)) * 0.5);
-    while ((int64_t)lj * (lj - 1) / 2 > p) --lj;
-    while ((int64_t)(lj + 1) * lj / 2 <= p) ++lj;
-    const int lk = (int)(p - (int64_t)lj * (lj - 1) / 2);
+    int lj, lk;
+    triangle_pair(p, lj, lk);
     const int64_t jk = (int64_t)lj * N + lk;
     const double r2jk = pr2[jk];
     if (r2jk > 625.0) continue;
     const double irjk = pir[jk], qjk = pq[jk], scjk = psc[jk];
     const double dcjk_j = pdc[jk], dcjk_k = pdc[(int64_t)lk * N + lj];
-    const double vjk[3] = {xs[3 * lk] - xs[3 * lj], xs[3 * lk + 1] - xs[3 * lj + 1],
-                           xs[3 * lk + 2] - xs[3 * lj + 2]};
     double gj[3] = {0, 0, 0}, gk[3] = {0, 0, 0}, dcj = 0.0, dck = 0.0;
     for (int li = lj + 1; li < N; ++li) {
       const int64_t ij = (int64_t)li * N + lj, ik = (int64_t)li * N + lk;
       const double r2ij = pr2[ij], r2ik = pr2[ik];
       if (r2ij > 625.0 || r2ik > 625.0) continue;
-      const double ir1 = pir[ij] * pir[ik] * irjk;
-      const double ir3 = ir1 * ir1 * ir1, ir5 = ir3 * ir1 * ir1;
-      const double rp = pq[ij] * pq[ik] * qjk;
-      const double damp = 1.0 / (1.0 + 6.0 * rp);
-      const double ang = 0.375 * (r2ij + r2jk - r2ik) * (r2ij - r2jk + r2ik) * (-r2ij + r2jk + r2ik) * ir5 + ir3;
-      const double c9 = -5.0 * psc[ij] * psc[ik] * scjk;
-      const double de = ang * damp * c9;
-      e -= de;
-      const double ddamp = -2.0 * 16.0 * rp * damp * damp;
-      const double vij[3] = {xs[3 * lj] - xs[3 * li], xs[3 * lj + 1] - xs[3 * li + 1],
-                             xs[3 * lj + 2] - xs[3 * li + 2]};
-      const double vik[3] = {xs[3 * lk] - xs[3 * li], xs[3 * lk + 1] - xs[3 * li + 1],
-                             xs[3 * lk + 2] - xs[3 * li + 2]};
-      const double tg[3] = {r2ij, r2ik, r2jk}, o1[3] = {r2jk, r2jk, r2ik}, o2[3] = {r2ik, r2ij, r2ij};
-      const double irr[3] = {pir[ij], pir[ik], irjk};
-      const double* vv[3] = {vij, vik, vjk};
       double dg[3][3];
-#pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        const double T = tg[q], a = o1[q], b = o2[q];
-        const double dang = -0.375 * (T * T * T + T * T * (a + b) + T * (3.0 * a * a + 2.0 * a * b + 3.0 * b * b) -
-                                      5.0 * (a - b) * (a - b) * (a + b)) * ir5;
-        const double scq = c9 * (-dang * damp + ang * ddamp) * (irr[q] * irr[q]);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) dg[q][c] = scq * vv[q][c];
-      }
+      const double de = atm_triple(r2ij, r2ik, r2jk, pir[ij], pir[ik], irjk, pq[ij] * pq[ik] * qjk,
+                                   psc[ij] * psc[ik] * scjk, xs + 3 * li, xs + 3 * lj, xs + 3 * lk, dg);
+      e -= de;
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
         acc_add<FIX>(&gsh[3 * li + c], -(dg[0][c] + dg[1][c]));
@@ -985,5 +1113,214 @@ __global__ __launch_bounds__(512) void k_force_atm(Topo t, const int* order, con
     dedcn4[a] = csh[la];
   }
 }
+
+// The three-body term of systems above kWideAtoms atoms.  k_wide_pairs fills the
+// tables, one thread per ordered pair.  k_wide_triples runs the triples, a
+// thread per pair (j, k): the lanes of a wavefront run over the same i, so the
+// adjoints of i are summed over the 16 lanes of a row before the LDS atomics (a
+// row's four sums are exchanged together: five permutes instead of sixteen), and
+// a block's sums go to the tables' unused diagonals, x y z of the gradient and the
+// CN adjoint in the first four.  The fifth holds the repulsion energies of
+// k_wide_atoms until k_wide_pairs has summed them, then the blocks' energies.
+// k_wide_atm adds the sums and the D4-CN chain, a wavefront per atom.
+// Bound: FP64 issue of the triples (about 300 instructions each).  One block per
+// system with an LDS atomic of 64 lanes on one address per adjoint took 208 us
+// for 62 atoms and 24.4 ms for 572; k_wide_triples takes 53 and 208 us.
+constexpr int kAtmLdsAtoms = 1024;
+
+__global__ __launch_bounds__(256) void k_wide_pairs(Topo t, const int* order, const unsigned char* valid,
+                                                    const double* w4, const double* dw4c, double* pairbuf,
+                                                    double* erep) {
+  const int s = order[blockIdx.x];
+  if (!valid[s]) return;
+  const int a0 = t.atom_off[s], N = t.atom_off[s + 1] - a0;
+  if (N <= kWideAtoms) return;
+  const int64_t NN = (int64_t)N * N;
+  double* tab = pairbuf + kAtmFields * t.apair_off[s];
+  for (int64_t idx = (int64_t)blockIdx.y * 256 + threadIdx.x; idx < NN; idx += (int64_t)gridDim.y * 256) {
+    const int lx = (int)(idx / N), ly = (int)(idx % N);
+    if (lx != ly) atm_pair(t, a0, lx, ly, w4, dw4c, tab + idx, NN);
+  }
+  if (blockIdx.y == 0 && threadIdx.x < 64) {
+    double e = 0.0;
+    double* diag = tab + 4 * NN;
+    for (int la = threadIdx.x; la < N; la += 64) {
+      e += diag[(int64_t)la * N + la];
+      diag[(int64_t)la * N + la] = 0.0;
+    }
+    e = wave_sum(e);
+    if (threadIdx.x == 0) erep[s] = e;
+  }
+}
+
+// blocks of k_wide_triples that a system of N atoms takes (no more than its diagonal has slots)
+__host__ __device__ inline int wide_parts(int N) {
+  const int64_t p = ((int64_t)N * (N - 1) / 2 + 255) / 256;
+  return p < N ? (int)p : N;
+}
+
+template <bool FIX>
+__global__ __launch_bounds__(256) void k_wide_triples(Topo t, const int* order, const unsigned char* valid,
+                                                      double* pairbuf) {
+  const int s = order[blockIdx.x];
+  if (!valid[s]) return;
+  const int a0 = t.atom_off[s], N = t.atom_off[s + 1] - a0;
+  if (N <= kWideAtoms) return;
+  const int parts = wide_parts(N), tid = threadIdx.x, lane = tid & 63;
+  if ((int)blockIdx.y >= parts) return;
+  __shared__ double red[16];
+  __shared__ double acc[4 * kAtmLdsAtoms];  // field c of atom l at c kAtmLdsAtoms + l
+  const bool lds = N <= kAtmLdsAtoms;
+  const int64_t NN = (int64_t)N * N;
+  double* pr2 = pairbuf + kAtmFields * t.apair_off[s];
+  const double* pir = pr2 + NN;
+  const double* pq = pr2 + 2 * NN;
+  const double* psc = pr2 + 3 * NN;
+  const double* pdc = pr2 + 4 * NN;
+  const double* xs = t.xyz + 3 * (int64_t)a0;
+  auto add = [&](int c, int l, double v) __attribute__((always_inline)) {
+    if (lds)
+      acc_add<FIX>(&acc[c * kAtmLdsAtoms + l], v);
+    else
+      acc_add<FIX>(&pr2[c * NN + (int64_t)l * N + l], v);
+  };
+  // an encoded sum in FIX
+  auto add_sum = [&](int c, int l, double v) __attribute__((always_inline)) {
+    const auto bits = (unsigned long long)__double_as_longlong(v);
+    if constexpr (!FIX)
+      add(c, l, v);
+    else if (lds)
+      atomicAdd(reinterpret_cast<unsigned long long*>(&acc[c * kAtmLdsAtoms + l]), bits);
+    else
+      atomicAdd(reinterpret_cast<unsigned long long*>(&pr2[c * NN + (int64_t)l * N + l]), bits);
+  };
+  if (lds) {
+    for (int x = tid; x < 4 * N; x += 256) acc[(x & 3) * kAtmLdsAtoms + (x >> 2)] = 0.0;
+    __syncthreads();
+  }
+  double e = 0.0;
+  const int64_t ntri = (int64_t)N * (N - 1) / 2;
+  for (int64_t base = (int64_t)blockIdx.y * 256; base < ntri; base += (int64_t)parts * 256) {
+    const int64_t p = base + tid;
+    int lj, lk;
+    triangle_pair(p < ntri ? p : ntri - 1, lj, lk);
+    const int64_t jk = (int64_t)lj * N + lk;
+    const double r2jk = pr2[jk];
+    const bool act = p < ntri && !(r2jk > 625.0);
+    if (!__any(act)) continue;
+    const double irjk = pir[jk], qjk = pq[jk], scjk = psc[jk];
+    const double dcjk_j = pdc[jk], dcjk_k = pdc[(int64_t)lk * N + lj];
+    double gj[3] = {0, 0, 0}, gk[3] = {0, 0, 0}, dcj = 0.0, dck = 0.0;
+    // j does not fall along the lanes: the first lane's is the least
+    for (int li = __builtin_amdgcn_readfirstlane(lj) + 1; li < N; ++li) {
+      double v[4] = {0, 0, 0, 0};  // gradient and CN adjoint of i
+      bool on = act && li > lj;
+      if (on) {
+        const int64_t ij = (int64_t)li * N + lj, ik = (int64_t)li * N + lk;
+        const double r2ij = pr2[ij], r2ik = pr2[ik];
+        on = !(r2ij > 625.0 || r2ik > 625.0);
+        if (on) {
+          double dg[3][3];
+          const double de = atm_triple(r2ij, r2ik, r2jk, pir[ij], pir[ik], irjk, pq[ij] * pq[ik] * qjk,
+                                       psc[ij] * psc[ik] * scjk, xs + 3 * li, xs + 3 * lj, xs + 3 * lk, dg);
+          e -= de;
+#pragma unroll
+          for (int c = 0; c < 3; ++c) {
+            v[c] = -(dg[0][c] + dg[1][c]);
+            gj[c] += dg[0][c] - dg[2][c];
+            gk[c] += dg[1][c] + dg[2][c];
+          }
+          // dC6(x, y)/dCN_x / C6(x, y) sits at the ordered pair [x][y]
+          v[3] = -0.5 * de * (pdc[ij] + pdc[ik]);
+          dcj -= 0.5 * de * (pdc[(int64_t)lj * N + li] + dcjk_j);
+          dck -= 0.5 * de * (pdc[(int64_t)lk * N + li] + dcjk_k);
+        }
+      }
+      if (!__any(on)) continue;
+      // lane l keeps field l % 4: halves exchanged within the quad, then quads
+      // summed.  FIX: every triple's contribution is rounded by itself and the
+      // sums are integer sums, whatever their order.
+      if constexpr (FIX)
+        for (int c = 0; c < 4; ++c) v[c] = __longlong_as_double((long long)fix_encode(v[c]));
+      auto plus = [](double x, double y) __attribute__((always_inline)) {
+        if constexpr (FIX) return __longlong_as_double(__double_as_longlong(x) + __double_as_longlong(y));
+        return x + y;
+      };
+      const bool b0 = lane & 1, b1 = lane & 2;
+      const double u0 = plus(b0 ? v[1] : v[0], dpp_permute<0xb1>(b0 ? v[0] : v[1]));
+      const double u1 = plus(b0 ? v[3] : v[2], dpp_permute<0xb1>(b0 ? v[2] : v[3]));
+      double u = plus(b1 ? u1 : u0, dpp_permute<0x4e>(b1 ? u0 : u1));
+      u = plus(u, dpp_permute<0x124>(u));  // row_ror:4
+      u = plus(u, dpp_permute<0x128>(u));  // row_ror:8
+      if ((lane & 12) == 0) add_sum(lane & 3, li, u);
+    }
+    if (act) {
+      for (int c = 0; c < 3; ++c) {
+        add(c, lj, gj[c]);
+        add(c, lk, gk[c]);
+      }
+      add(3, lj, dcj);
+      add(3, lk, dck);
+    }
+  }
+  e = block_sum(e, red);  // its barriers end the block's LDS sums
+  if (tid == 0) pr2[4 * NN + (int64_t)blockIdx.y * N + blockIdx.y] = e;
+  if (lds)
+    for (int x = tid; x < 4 * N; x += 256) {
+      const int c = x & 3, l = x >> 2;
+      double* to = &pr2[c * NN + (int64_t)l * N + l];
+      const double v = acc[c * kAtmLdsAtoms + l];
+      if constexpr (FIX)
+        atomicAdd(reinterpret_cast<unsigned long long*>(to), (unsigned long long)__double_as_longlong(v));
+      else
+        atomicAdd(to, v);
+    }
+}
+
+template <bool FIX>
+__global__ __launch_bounds__(256) void k_wide_atm(Topo t, const int* order, const unsigned char* valid,
+                                                  const double* pairbuf, double* dedcn4, double* grad, double* eatm) {
+  const int s = order[blockIdx.x];
+  if (!valid[s]) return;
+  const int a0 = t.atom_off[s], N = t.atom_off[s + 1] - a0;
+  if (N <= kWideAtoms) return;
+  const int64_t NN = (int64_t)N * N;
+  const double* tab = pairbuf + kAtmFields * t.apair_off[s];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  auto sum = [&](int c, int l) __attribute__((always_inline)) {
+    const double v = tab[c * NN + (int64_t)l * N + l];
+    if constexpr (FIX) return fix_decode((unsigned long long)__double_as_longlong(v));
+    return v;
+  };
+  for (int la = blockIdx.y * 4 + wv; la < N; la += gridDim.y * 4) {
+    const double* ra = t.xyz + 3 * (int64_t)(a0 + la);
+    const double ca = sum(3, la);
+    double g[3] = {0, 0, 0};
+    for (int lb = lane; lb < N; lb += 64) {
+      if (lb == la) continue;
+      const double* rb = t.xyz + 3 * (int64_t)(a0 + lb);
+      const double r[3] = {ra[0] - rb[0], ra[1] - rb[1], ra[2] - rb[2]};
+      const double r2 = r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
+      if (r2 > 900.0) continue;
+      const double rr = sqrt(r2);
+      double val, der;
+      d4_cn_count(t, a0 + la, a0 + lb, rr, val, der);
+      const double sc = (ca + sum(3, lb)) * der / rr;
+      for (int c = 0; c < 3; ++c) g[c] += sc * r[c];
+    }
+    for (int c = 0; c < 3; ++c) g[c] = wave_sum(g[c]);
+    if (lane == 0) {
+      for (int c = 0; c < 3; ++c) grad[3 * (int64_t)(a0 + la) + c] += g[c] + sum(c, la);
+      dedcn4[a0 + la] = ca;
+    }
+  }
+  if (blockIdx.y == 0 && wv == 0) {
+    double e = 0.0;
+    for (int p = lane; p < wide_parts(N); p += 64) e += tab[4 * NN + (int64_t)p * N + p];
+    e = wave_sum(e);
+    if (lane == 0) eatm[s] = e;
+  }
+}
+
 
 }  // namespace xtb
