@@ -190,7 +190,9 @@ __device__ inline void d4_weights(const Topo& t, int a, double cn, double q, dou
   }
   const double inorm = fabs(norm) > 1.4916681462400413e-154 ? 1.0 / norm : 0.0;
   const double qmod = q + t.at_d4zeff[a], c = t.at_d4hard[a] * 2.0;
-  for (int r = 0; r < kD4MaxRef; ++r) {
+  // every entry is stored once: blocks that stage the same atoms write the same
+  // values over each other
+  for (int r = nref; r < kD4MaxRef; ++r) {
     w[r] = 0.0;
     if (dwdcn) dwdcn[r] = 0.0;
     if (dwdq) dwdq[r] = 0.0;

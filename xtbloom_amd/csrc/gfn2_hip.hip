@@ -1006,14 +1006,15 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
   HIP_TRY(up_topo(d_perm, T.perm));
   t.perm = d_perm;
   const bool big_systems = T.max_atoms > kPairStageAtoms;
+  const bool sliced = T.max_atoms > kSliceFrom;
+  const dim3 slices(B, sliced ? (T.max_atoms + kSliceAtoms - 1) / kSliceAtoms : 1);
   auto launch_potentials = [&](const unsigned char* mask) {
-    hipLaunchKernelGGL(k_potentials<true>, dim3(B), dim3(512), 0, sm, t, d_order, mask, mx.x,
-                       d_cnd4, d_mrad, d_gam, d_vpc, d_qat, d_w4, d_dw4, d_vat, d_vsh, d_vd, d_vqq,
-                       d_gstage, d_gstagei);
-    if (big_systems)
-      hipLaunchKernelGGL(k_potentials<false>, dim3(B), dim3(512), 0, sm, t, d_order, mask, mx.x,
-                         d_cnd4, d_mrad, d_gam, d_vpc, d_qat, d_w4, d_dw4, d_vat, d_vsh, d_vd,
-                         d_vqq, d_gstage, d_gstagei);
+    auto launch = [&](auto* kernel) {
+      hipLaunchKernelGGL(kernel, slices, dim3(512), 0, sm, t, d_order, mask, mx.x, d_cnd4, d_mrad, d_gam, d_vpc,
+                         d_qat, d_w4, d_dw4, d_vat, d_vsh, d_vd, d_vqq, d_gstage, d_gstagei);
+    };
+    launch(k_potentials<true>);
+    if (big_systems) launch(k_potentials<false>);
   };
 
   HIP_TRY(hipMemsetAsync(d_st, 0, sizeof(SysState) * B, sm));
@@ -1344,13 +1345,15 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
     HIP_TRY(probe_end(kKMulliken, 0.0, 0.0));
     if (rp) rp->mull = last_probe();
     HIP_TRY(probe_begin(kKEnergyMix));
-    hipLaunchKernelGGL(k_energy_mix<true>, dim3(B), dim3(512), 0, sm, t, d_order, d_active,
-                       d_cnd4, d_mrad, d_gam, d_vpc, d_qat, d_w4, mx, d_st, cnt, d_gstage,
-                       d_gstagei, rptr);
-    if (big_systems)
-      hipLaunchKernelGGL(k_energy_mix<false>, dim3(B), dim3(512), 0, sm, t, d_order, d_active,
-                         d_cnd4, d_mrad, d_gam, d_vpc, d_qat, d_w4, mx, d_st, cnt, d_gstage,
-                         d_gstagei, rptr);
+    auto energy = [&](auto* slices_kernel, auto* mix_kernel) {
+      if (sliced)
+        hipLaunchKernelGGL(slices_kernel, slices, dim3(512), 0, sm, t, d_order, d_active, d_cnd4, d_mrad, d_gam,
+                           d_vpc, d_qat, d_w4, mx.raw, d_gstage, d_gstagei, dY);
+      hipLaunchKernelGGL(mix_kernel, dim3(B), dim3(512), 0, sm, t, d_order, d_active, d_cnd4, d_mrad, d_gam, d_vpc,
+                         d_qat, d_w4, mx, d_st, cnt, d_gstage, d_gstagei, rptr, dY);
+    };
+    energy(k_energy_slices<true>, k_energy_mix<true>);
+    if (big_systems) energy(k_energy_slices<false>, k_energy_mix<false>);
     HIP_TRY(probe_end(kKEnergyMix, 0.0, 0.0));
     HIP_TRY(hipGetLastError());
     return 0;

@@ -5,44 +5,21 @@
 
 namespace xtb {
 
-// ---------------------------------------------------------------------------
-// SCC energy from the raw multipoles (reference scc_driver.cpp:2105-2286),
-// modified Broyden step (reference common/scc_mixer.cpp:559-745) and the
-// convergence gate rms < qtol and |dF| < etol (scc_driver.cpp:869-893).
-// One 512-thread block per active system; the pair energies come from the
-// shared pair sums (STAGED as for k_potentials).
-// ---------------------------------------------------------------------------
+// Energy terms at the raw state (es2 es3 pc aes2 d4), this thread's share, of the
+// atoms [pa0, pa1) in staging order; the terms that are not pair sums are
+// thread 0's and up of the slice that starts at atom 0.
 template <bool STAGED>
-__global__ __launch_bounds__(512) void k_energy_mix(Topo t, const int* order, unsigned char* active,
-                                                    const double* cnd4, const double* mrad,
-                                                    const double* gam, const double* vpc,
-                                                    double* qat_raw, double* w4, MixerArrays mx,
-                                                    SysState* st, int* active_count,
-                                                    double* gstage, int* gstagei,
-                                                    const int* round_ptr) {
-  const int s = order[blockIdx.x];
-  if (!active[s]) return;
-  // the beta copy of an unrestricted system has no state of its own: its
-  // alpha system mixes both channels and sets its flags
-  if (t.partner && t.partner[s] >= 0 && t.partner[s] < s) return;
-  const int a0 = t.atom_off[s], a1 = t.atom_off[s + 1], N = a1 - a0;
-  if (STAGED != (N <= kPairStageAtoms)) return;
+__device__ __forceinline__ void energy_terms(const Topo& t, int s, int pa0, int pa1, const double* raw,
+                                             const double* cnd4, const double* mrad, const double* gam,
+                                             const double* vpc, double* qat_raw, double* w4, double* buf, int* ibuf,
+                                             double (&e)[5]) {
+  const int a0 = t.atom_off[s], N = t.atom_off[s + 1] - a0;
   const int s0 = t.shell_off[s], ns = t.shell_off[s + 1] - s0;
-  const int vo = t.vec_off[s], dim = t.vec_off[s + 1] - vo;
-  const double* raw = mx.raw + vo;
+  const bool sliced = pa1 - pa0 < N;
   const double* qsh = raw;
   const double* dip = raw + ns;
   const double* quad = raw + ns + 3 * N;
   const int tid = threadIdx.x, nt = blockDim.x;
-  __shared__ double red[64];  // block_sum_n: K values per wavefront
-  // the atom staging area while the pair sums run, the Broyden beta matrix after
-  __shared__ double lbuf[STAGED ? kPairStageDoubles * kPairStageAtoms : 64 * 64];
-  __shared__ int libuf[STAGED ? kPairStageInts * kPairStageAtoms : 1];
-  __shared__ double coef[64];
-  __shared__ int slots[64];
-  __shared__ double sh_scalar[4];
-  double* buf = STAGED ? lbuf : gstage + (size_t)kPairStageDoubles * a0;
-  int* ibuf = STAGED ? libuf : gstagei + (size_t)kPairStageInts * a0;
   const PairStage S = pair_stage(buf, ibuf, N);
   for (int p = tid; p < N; p += nt) {
     const int a = t.perm[a0 + p];
@@ -54,24 +31,27 @@ __global__ __launch_bounds__(512) void k_energy_mix(Topo t, const int* order, un
   __syncthreads();
   // ES2 / ES3 / point charges (Gamma symmetric: coalesced column reads)
   const double* Gm = gam + t.gam_off[s];
-  double e[5] = {0.0, 0.0, 0.0, 0.0, 0.0};  // es2 es3 pc aes2 d4
   for (int i = tid; i < ns; i += nt) {
-    double v = 0.0;
-    for (int j = 0; j < ns; ++j) v += Gm[j * ns + i] * qsh[j];
     const int sh = s0 + i;
-    e[0] += 0.5 * qsh[i] * v;
-    e[1] += t.sh_gam3[sh] * qsh[i] * qsh[i] * qsh[i] / 3.0;
-    e[2] = fma(qsh[i], vpc[sh], e[2]);
+    if (!sliced) {
+      double v = 0.0;
+      for (int j = 0; j < ns; ++j) v += Gm[j * ns + i] * qsh[j];
+      e[0] += 0.5 * qsh[i] * v;
+    }
+    if (pa0 == 0) {
+      e[1] += t.sh_gam3[sh] * qsh[i] * qsh[i] * qsh[i] / 3.0;
+      e[2] = fma(qsh[i], vpc[sh], e[2]);
+    }
   }
   // a uniform field's dipole term -E.mu_A joins the external energy (its
   // charge term -q_A E.R_A is part of vpc)
-  if (t.field) {
+  if (pa0 == 0 && t.field) {
     const double* E = t.field + 3 * s;
     for (int i = tid; i < 3 * N; i += nt) e[2] -= E[i % 3] * dip[i];
   }
   // spin polarization m.W.m / 2 of the raw magnetization (reference
   // spin.cpp:135-172), kept with AES2 in e[3]
-  if (t.partner && t.partner[s] > s) {
+  if (pa0 == 0 && t.partner && t.partner[s] > s) {
     const double* m = raw + ns + 9 * N;
     for (int i = tid; i < ns; i += nt) {
       const int sh = s0 + i, f = t.atom_sh0[t.sh_atom[sh]] - s0;
@@ -83,7 +63,7 @@ __global__ __launch_bounds__(512) void k_energy_mix(Topo t, const int* order, un
   }
   // external charge operator q.b + q.(A q)/2 at the raw atomic charges
   // (reference periodic_embedding.cpp:352-434)
-  if (t.pshift || t.presp) {
+  if (pa0 == 0 && (t.pshift || t.presp)) {
     for (int la = tid; la < N; la += nt) {
       double r = 0.0;
       if (t.presp) {
@@ -98,11 +78,11 @@ __global__ __launch_bounds__(512) void k_energy_mix(Topo t, const int* order, un
   // energy equals q_a V_q + d_a.V_d + Q_a.V_Q of atom a in the field of b,
   // symmetric in (a, b).
   const double qscale[6] = {1.0, 2.0, 1.0, 2.0, 2.0, 1.0};
-  const int G = pair_lanes(N, nt), g = tid & (G - 1), per = nt / G;
+  const int G = pair_lanes(pa1 - pa0, nt), g = tid & (G - 1), per = nt / G;
   const int L = (N + G - 1) / G;
-  for (int base = 0; base < N; base += per) {
+  for (int base = pa0; base < pa1; base += per) {
     const int pa = base + tid / G;
-    if (pa < N) {
+    if (pa < pa1) {
       PairSums o;
       pair_sums(t, S, N, pa, min(N, g * L), min(N, (g + 1) * L), o);
       pair_sums_reduce(o, G);
@@ -123,7 +103,85 @@ __global__ __launch_bounds__(512) void k_energy_mix(Topo t, const int* order, un
         e[3] += t.at_dk[a] * d2 + t.at_qk[a] * q2 + 0.5 * pair;
         e[4] -= 0.5 * ew;
       }
+      if (sliced) {
+        const int a = t.perm[a0 + pa];
+        for (int sh = t.atom_sh0[a]; sh < t.atom_sh0[a + 1]; ++sh) {
+          const double v = gamma_row(Gm, sh - s0, ns, qsh, g, G);
+          if (g == 0) e[0] += 0.5 * qsh[sh - s0] * v;
+        }
+      }
     }
+  }
+}
+
+// The energy terms of systems of more than kSliceFrom atoms, a block per slice:
+// slice k's sums go to part + 8 k of the system's slot of the Y matrix, which is
+// free between the density and the next round's eigenvectors.
+template <bool STAGED>
+__global__ __launch_bounds__(512) void k_energy_slices(Topo t, const int* order, const unsigned char* active,
+                                                          const double* cnd4, const double* mrad, const double* gam,
+                                                          const double* vpc, double* qat_raw, double* w4,
+                                                          const double* raw, double* gstage, int* gstagei, double* part) {
+  const int s = order[blockIdx.x];
+  if (!active[s]) return;
+  if (t.partner && t.partner[s] >= 0 && t.partner[s] < s) return;
+  const int a0 = t.atom_off[s], N = t.atom_off[s + 1] - a0;
+  if (STAGED != (N <= kPairStageAtoms)) return;
+  const int pa0 = (int)blockIdx.y * kSliceAtoms;
+  if (N <= kSliceFrom || pa0 >= N) return;
+  __shared__ double red[64];
+  __shared__ double lbuf[STAGED ? kPairStageDoubles * kPairStageAtoms : 1];
+  __shared__ int libuf[STAGED ? kPairStageInts * kPairStageAtoms : 1];
+  double e[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  energy_terms<STAGED>(t, s, pa0, min(N, pa0 + kSliceAtoms), raw + t.vec_off[s], cnd4, mrad, gam, vpc, qat_raw, w4,
+                       STAGED ? lbuf : gstage + (size_t)kPairStageDoubles * a0,
+                       STAGED ? libuf : gstagei + (size_t)kPairStageInts * a0, e);
+  block_sum_n<5>(e, red);
+  if (threadIdx.x == 0)
+    for (int k = 0; k < 5; ++k) part[t.mat_off[s] + 8 * (int64_t)blockIdx.y + k] = e[k];
+}
+
+// ---------------------------------------------------------------------------
+// SCC energy from the raw multipoles (reference scc_driver.cpp:2105-2286),
+// modified Broyden step (reference common/scc_mixer.cpp:559-745) and the
+// convergence gate rms < qtol and |dF| < etol (scc_driver.cpp:869-893).
+// One 512-thread block per active system; the pair energies come from the
+// shared pair sums (STAGED as for k_potentials).
+// ---------------------------------------------------------------------------
+template <bool STAGED>
+__global__ __launch_bounds__(512) void k_energy_mix(Topo t, const int* order, unsigned char* active,
+                                                    const double* cnd4, const double* mrad,
+                                                    const double* gam, const double* vpc,
+                                                    double* qat_raw, double* w4, MixerArrays mx,
+                                                    SysState* st, int* active_count,
+                                                    double* gstage, int* gstagei,
+                                                    const int* round_ptr, const double* part) {
+  const int s = order[blockIdx.x];
+  if (!active[s]) return;
+  // the beta copy of an unrestricted system has no state of its own: its
+  // alpha system mixes both channels and sets its flags
+  if (t.partner && t.partner[s] >= 0 && t.partner[s] < s) return;
+  const int a0 = t.atom_off[s], a1 = t.atom_off[s + 1], N = a1 - a0;
+  if (STAGED != (N <= kPairStageAtoms)) return;
+  const int s0 = t.shell_off[s], ns = t.shell_off[s + 1] - s0;
+  const int vo = t.vec_off[s], dim = t.vec_off[s + 1] - vo;
+  const double* raw = mx.raw + vo;
+  const int tid = threadIdx.x, nt = blockDim.x;
+  __shared__ double red[64];  // block_sum_n: K values per wavefront
+  // the atom staging area while the pair sums run, the Broyden beta matrix after
+  __shared__ double lbuf[STAGED ? kPairStageDoubles * kPairStageAtoms : 64 * 64];
+  __shared__ int libuf[STAGED ? kPairStageInts * kPairStageAtoms : 1];
+  __shared__ double coef[64];
+  __shared__ int slots[64];
+  __shared__ double sh_scalar[4];
+  double e[5] = {0.0, 0.0, 0.0, 0.0, 0.0};  // es2 es3 pc aes2 d4
+  if (N > kSliceFrom) {  // summed by k_energy_slices
+    for (int k = tid; k * kSliceAtoms < N; k += nt)
+      for (int c = 0; c < 5; ++c) e[c] += part[t.mat_off[s] + 8 * (int64_t)k + c];
+  } else {
+    energy_terms<STAGED>(t, s, 0, N, raw, cnd4, mrad, gam, vpc, qat_raw, w4,
+                         STAGED ? lbuf : gstage + (size_t)kPairStageDoubles * a0,
+                         STAGED ? libuf : gstagei + (size_t)kPairStageInts * a0, e);
   }
   block_sum_n<5>(e, red);
   const double e2 = e[0], e3 = e[1], epc = e[2], eaes = e[3], ed4 = e[4];
