@@ -190,8 +190,6 @@ __device__ inline void d4_weights(const Topo& t, int a, double cn, double q, dou
   }
   const double inorm = fabs(norm) > 1.4916681462400413e-154 ? 1.0 / norm : 0.0;
   const double qmod = q + t.at_d4zeff[a], c = t.at_d4hard[a] * 2.0;
-  // every entry is stored once: blocks that stage the same atoms write the same
-  // values over each other
   for (int r = nref; r < kD4MaxRef; ++r) {
     w[r] = 0.0;
     if (dwdcn) dwdcn[r] = 0.0;
@@ -215,6 +213,35 @@ __device__ inline void d4_weights(const Topo& t, int a, double cn, double q, dou
     if (dwdcn) dwdcn[r] = dcw * z;
     if (dwdq) dwdq[r] = cw * zeta_scale_dq(c, qref, qmod);
   }
+}
+
+// The same weights by eight consecutive lanes, lane r = lane % 8 on reference r
+// (kD4MaxRef < 8): the exponentials of one reference a lane instead of all seven
+// in a chain.  Only lanes with r < kD4MaxRef hold a result.
+__device__ __forceinline__ void d4_weight_lane(const Topo& t, int a, double cn, double q, int r, double& w,
+                                               double& dwdq) {
+  const int off = t.at_d4ref[a], nref = t.at_d4nref[a];
+  const bool on = r < nref;
+  const double rc = on ? t.d4_refcn[off + r] : -1.0e300;
+  double num = 0.0;
+  if (on)
+    for (int k = 1; k <= t.d4_refng[off + r]; ++k) {
+      const double f = 6.0 * k, dl = cn - rc;
+      num += exp(-f * dl * dl);
+    }
+  double norm = num, maxcn = rc;
+#pragma unroll
+  for (int m = 1; m < 8; m *= 2) {
+    norm += __shfl_xor(norm, m);
+    maxcn = fmax(maxcn, __shfl_xor(maxcn, m));
+  }
+  const double inorm = fabs(norm) > 1.4916681462400413e-154 ? 1.0 / norm : 0.0;
+  const double qmod = q + t.at_d4zeff[a], c = t.at_d4hard[a] * 2.0;
+  double cw = num * inorm;
+  if (!isfinite(cw) || inorm == 0.0) cw = fabs(maxcn - rc) < 1e-12 ? 1.0 : 0.0;
+  const double qref = on ? t.d4_refq[off + r] + t.at_d4zeff[a] : 0.0;
+  w = on ? cw * zeta_scale(c, qref, qmod) : 0.0;
+  dwdq = on ? cw * zeta_scale_dq(c, qref, qmod) : 0.0;
 }
 
 // sum_rs wa_r wb_s C6ref[r][s]

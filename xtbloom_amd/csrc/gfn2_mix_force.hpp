@@ -21,13 +21,7 @@ __device__ __forceinline__ void energy_terms(const Topo& t, int s, int pa0, int 
   const double* quad = raw + ns + 3 * N;
   const int tid = threadIdx.x, nt = blockDim.x;
   const PairStage S = pair_stage(buf, ibuf, N);
-  for (int p = tid; p < N; p += nt) {
-    const int a = t.perm[a0 + p];
-    double q = 0.0;
-    for (int sh = t.atom_sh0[a]; sh < t.atom_sh0[a + 1]; ++sh) q += qsh[sh - s0];
-    qat_raw[a] = q;
-    pair_stage_atom(t, S, N, p, a, a - a0, dip, quad, q, cnd4, mrad, w4, nullptr);
-  }
+  pair_stage_system(t, s, S, qsh, dip, quad, cnd4, mrad, qat_raw, w4, nullptr);
   __syncthreads();
   // ES2 / ES3 / point charges (Gamma symmetric: coalesced column reads)
   const double* Gm = gam + t.gam_off[s];

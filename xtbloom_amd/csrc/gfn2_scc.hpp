@@ -339,22 +339,47 @@ __device__ __forceinline__ PairStage pair_stage(double* buf, int* ibuf, int N) {
 // dip / quad: the system's dipole and quadrupole blocks of the state vector;
 // la: the atom's index inside the system.
 __device__ __forceinline__ void pair_stage_atom(const Topo& t, const PairStage& S, int N, int p,
-                                                int a, int la, const double* dip,
+                                                int a, int la, int r, const double* dip,
                                                 const double* quad, double q, const double* cnd4,
                                                 const double* mrad, double* w4, double* dw4) {
-  for (int c = 0; c < 3; ++c) {
-    S.x[c * N + p] = t.xyz[3 * a + c];
-    S.dp[c * N + p] = dip[3 * la + c];
+  if (r < 3) {
+    S.x[r * N + p] = t.xyz[3 * a + r];
+    S.dp[r * N + p] = dip[3 * la + r];
   }
-  for (int c = 0; c < 6; ++c) S.qp[c * N + p] = quad[6 * la + c];
-  S.mr[p] = mrad[a];
-  S.q[p] = q;
-  S.r42[p] = t.at_d4r4r2[a];
-  S.ref[p] = t.at_d4ref[a];
-  S.nref[p] = t.at_d4nref[a];
-  d4_weights(t, a, cnd4[a], q, w4 + kD4MaxRef * a, nullptr,
-             dw4 ? dw4 + kD4MaxRef * a : nullptr);
-  for (int r = 0; r < kD4MaxRef; ++r) S.w[r * N + p] = w4[kD4MaxRef * a + r];
+  if (r < 6) S.qp[r * N + p] = quad[6 * la + r];
+  if (r == 6) {
+    S.mr[p] = mrad[a];
+    S.q[p] = q;
+  }
+  if (r == 7) {
+    S.r42[p] = t.at_d4r4r2[a];
+    S.ref[p] = t.at_d4ref[a];
+    S.nref[p] = t.at_d4nref[a];
+  }
+  double w, dw;
+  d4_weight_lane(t, a, cnd4[a], q, r, w, dw);
+  if (r < kD4MaxRef) {
+    w4[kD4MaxRef * a + r] = w;
+    if (dw4) dw4[kD4MaxRef * a + r] = dw;
+    S.w[r * N + p] = w;
+  }
+}
+
+// Stages all atoms of system s, eight lanes an atom, and their charges.  Every
+// value is stored once, so blocks that stage the same system write the same
+// values over each other.
+__device__ __forceinline__ void pair_stage_system(const Topo& t, int s, const PairStage& S, const double* qsh,
+                                                  const double* dip, const double* quad, const double* cnd4,
+                                                  const double* mrad, double* qat, double* w4, double* dw4) {
+  const int a0 = t.atom_off[s], N = t.atom_off[s + 1] - a0, s0 = t.shell_off[s];
+  for (int idx = threadIdx.x; idx < 8 * N; idx += blockDim.x) {
+    const int p = idx >> 3, r = idx & 7;
+    const int a = t.perm[a0 + p];
+    double q = 0.0;
+    for (int sh = t.atom_sh0[a]; sh < t.atom_sh0[a + 1]; ++sh) q += qsh[sh - s0];
+    if (r == 0) qat[a] = q;
+    pair_stage_atom(t, S, N, p, a, a - a0, r, dip, quad, q, cnd4, mrad, w4, dw4);
+  }
 }
 
 struct PairSums {
@@ -505,13 +530,7 @@ __global__ __launch_bounds__(512, 4) void k_potentials(Topo t, const int* order,
   double* buf = STAGED ? lbuf : gstage + (size_t)kPairStageDoubles * a0;
   int* ibuf = STAGED ? libuf : gstagei + (size_t)kPairStageInts * a0;
   const PairStage S = pair_stage(buf, ibuf, N);
-  for (int p = tid; p < N; p += nt) {
-    const int a = t.perm[a0 + p];
-    double q = 0.0;
-    for (int sh = t.atom_sh0[a]; sh < t.atom_sh0[a + 1]; ++sh) q += qsh[sh - s0];
-    qat[a] = q;
-    pair_stage_atom(t, S, N, p, a, a - a0, x + ns, x + ns + 3 * N, q, cnd4, mrad, w4, dw4);
-  }
+  pair_stage_system(t, s, S, qsh, x + ns, x + ns + 3 * N, cnd4, mrad, qat, w4, dw4);
   __syncthreads();
   // ES2 + ES3 + point charges; Gamma is symmetric, so column i is read
   // (coalesced across the block) in place of row i.
