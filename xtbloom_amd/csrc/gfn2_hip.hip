@@ -1146,9 +1146,22 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
   }
   HIP_TRY(probe_begin(kKCholesky));
   // systems are ordered largest first: the n_large above 256 AOs take the
-  // blocked factorization, the rest the register one
-  if (n_large > 0)
-    hipLaunchKernelGGL(k_cholesky_blocked, dim3(n_large), dim3(512), 0, sm, t, d_order, dS, dA, dX, d_st);
+  // factorization over the chip, the rest the register one
+  if (n_large > 0) {
+    const int top = T.ao_off[T.order[0] + 1] - T.ao_off[T.order[0]];
+    const unsigned blocks16 = (unsigned)((top + 15) / 16);
+    hipLaunchKernelGGL(k_chol_start, dim3(n_large, 64), dim3(256), 0, sm, t, d_order, dS, dA, dX);
+    for (int k0 = 0; k0 < top; k0 += kCholPanel) {
+      const int below = std::max(top - k0 - kCholPanel, 1);
+      const int64_t rows16 = (below + 15) / 16, tiles = rows16 * (rows16 + 1) / 2;
+      hipLaunchKernelGGL(k_chol_panel, dim3(n_large, (below + 255) / 256), dim3(256), 0, sm, t, d_order, dA, dX, d_st,
+                         k0);
+      hipLaunchKernelGGL(k_chol_trailing, dim3(n_large, (unsigned)std::min<int64_t>((tiles + 3) / 4, 4096)), dim3(256),
+                         0, sm, t, d_order, dA, dX, k0);
+    }
+    hipLaunchKernelGGL(k_chol_diagonal, dim3(n_large, (blocks16 + 3) / 4), dim3(64), 0, sm, t, d_order, dA, dX);
+    hipLaunchKernelGGL(k_chol_invert, dim3(n_large, blocks16), dim3(512), 0, sm, t, d_order, dA, dX);
+  }
   if (n_large < B)
     hipLaunchKernelGGL(k_cholesky_inverse, dim3(B - n_large), dim3(512), 0, sm, t, d_order + n_large, dS, dA,
                        dX, d_st);

@@ -1739,174 +1739,230 @@ __global__ __launch_bounds__(512) void k_cholesky_inverse(Topo t, const int* ord
   if (threadIdx.x == 0 && bad) status[s].status = 8;
 }
 
-// Overlap factorization for n > 256, 512 threads, X = L^{-T} as above (L in
-// `work`, column-major lower; X row-major upper with its strict lower part
-// zero).
-//   factorization  right-looking in panels of kCholPanel columns: inside a
-//                  panel column by column (the pivot row's panel entries go
-//                  through LDS, every thread owns rows); after the panel the
-//                  trailing lower triangle takes A -= L21 L21^T once, in
-//                  16 x 16 tiles on the FP64 matrix cores (K = the panel).
-//   inverse        L^{-1} by 16 x 16 blocks: the diagonal blocks by
-//                  substitution (a thread per block column), then block row
-//                  I from the rows above it,
-//                    Linv_IJ = -Linv_II sum_{K=J}^{I-1} L_IK Linv_KJ,
-//                  one block J per wavefront at a time (matrix cores, the sum
-//                  staged through the wavefront's LDS tile), one barrier per
-//                  block row.  Linv_ij is stored as X_ji.
+// Overlap factorization for n > 256, X = L^{-T} as above (L in `work`,
+// column-major lower; X row-major upper with its strict lower part zero), in
+// launches that spread each system over the chip:
+//   k_chol_start     L = S, X's strict lower part.
+//   per panel of kCholPanel columns:
+//   k_chol_panel     every block factors the diagonal block by itself (one
+//                    wavefront, a row per lane in registers) and takes 256 rows
+//                    below it, a row per thread, through the substitution.  Block
+//                    0 leaves the diagonal factor in X, because the others read
+//                    the unfactored one from L.
+//   k_chol_trailing  A -= L21 L21^T on the lower triangle, a 16 x 16 tile per
+//                    wavefront on the FP64 matrix cores; moves the diagonal
+//                    factor into L.
+//   k_chol_diagonal  the 16 x 16 diagonal blocks of L^{-1}, a thread per column.
+//   k_chol_invert    a block per 16 columns J of L^{-1}, down the block rows:
+//                      Linv_IJ = -Linv_II sum_{K=J}^{I-1} L_IK Linv_KJ,
+//                    the sum over K split over eight wavefronts.
+// Bound: two launches a panel (36 panels at 1142 AOs) and the chain of block rows
+// of the inverse.  One 512-thread block per system took 21.2 ms at 1142 AOs and
+// 2.5 ms for fourteen systems of 258 to 482; the launches take 1.5 and 0.6 ms.
 // Matrix-core lane mapping (v_mfma_f64_16x16x4f64): for D = P Q^T over k,
 // lane (l16, lk) supplies a = Q[l16][k], b = P[l16][k] for k = 4 q + lk and
 // receives D[l16][lk + 4 r], r < 4.
-constexpr int kCholPanel = 16;
+constexpr int kCholPanel = 32;
 
-__global__ __launch_bounds__(512) void k_cholesky_blocked(Topo t, const int* order, const double* S,
-                                                          double* work, double* X, SysState* status) {
+__global__ __launch_bounds__(256) void k_chol_start(Topo t, const int* order, const double* S, double* work,
+                                                    double* X) {
   const int s = order[blockIdx.x];
   const int n = t.ao_off[s + 1] - t.ao_off[s];
-  const int64_t mo = t.mat_off[s];
-  const double* __restrict__ Sm = S + mo;
-  double* __restrict__ L = work + mo;
-  double* __restrict__ Xm = X + mo;
-  const int tid = threadIdx.x, nt = blockDim.x;
-  const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), nw = nt >> 6;
-  const int l16 = lane & 15, lk = lane >> 4;
-  __shared__ double pl[kCholPanel];
-  __shared__ double sh_ipiv;
-  __shared__ double sS[8][16][17];
-  __shared__ int bad;
-  auto at = [n](int r, int c) __attribute__((always_inline)) { return (int64_t)r + (int64_t)c * n; };
-  if (tid == 0) bad = 0;
-  for (int64_t idx = tid; idx < (int64_t)n * n; idx += nt) L[idx] = Sm[idx];
-  __syncthreads();
-  for (int k0 = 0; k0 < n; k0 += kCholPanel) {
-    const int jn = min(kCholPanel, n - k0);
-    for (int j = k0; j < k0 + jn; ++j) {
-      if (tid == 0) {
-        double d = L[at(j, j)];
-        if (!(d > 0.0)) {
-          bad = 1;
-          d = 1.0;
-        }
-        const double piv = sqrt(d);
-        const double ipiv = 1.0 / piv;
-        L[at(j, j)] = piv;
-        for (int jj = j + 1; jj < k0 + jn; ++jj) pl[jj - k0] = L[at(jj, j)] * ipiv;
-        sh_ipiv = ipiv;
-      }
-      __syncthreads();
-      const double ipiv = sh_ipiv;
-      for (int i = j + 1 + tid; i < n; i += nt) {
-        const double v = L[at(i, j)] * ipiv;
-        L[at(i, j)] = v;
-        const int je = min(i, k0 + jn - 1);
-        for (int jj = j + 1; jj <= je; ++jj) L[at(i, jj)] -= v * pl[jj - k0];
-      }
-      __syncthreads();
-    }
-    // trailing lower triangle, rows and columns >= c0: A -= L21 L21^T
-    const int c0 = k0 + jn, mt = n - c0;
-    const int nb16 = (mt + 15) >> 4;
-    const int ntiles = nb16 * (nb16 + 1) / 2;
-    for (int tile = wv; tile < ntiles; tile += nw) {
-      int TI = (int)((sqrt(8.0 * tile + 1.0) - 1.0) * 0.5);
-      while (TI * (TI + 1) / 2 > tile) --TI;
-      while ((TI + 1) * (TI + 2) / 2 <= tile) ++TI;
-      const int TJ = tile - TI * (TI + 1) / 2;
-      const int rr = 16 * TI + l16, cc = 16 * TJ + l16;  // this lane's row of P (rows), of Q (columns)
-      const int rrc = c0 + min(rr, mt - 1), ccc = c0 + min(cc, mt - 1);
-      double xa[kCholPanel / 4], xb[kCholPanel / 4];
-#pragma unroll
-      for (int q = 0; q < kCholPanel / 4; ++q) {
-        const int ci = k0 + min(4 * q + lk, jn - 1);
-        xa[q] = L[at(ccc, ci)];
-        xb[q] = L[at(rrc, ci)];
-      }
-      mfma_d4 acc = mfma_d4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-      for (int q = 0; q < kCholPanel / 4; ++q) {
-        const bool on = 4 * q + lk < jn;
-        acc = mfma_16x16x4(on && cc < mt ? xa[q] : 0.0, on && rr < mt ? xb[q] : 0.0, acc);
-      }
-      // acc[r] = D[row = 16 TI + l16][col = 16 TJ + lk + 4 r]
-      const int row = 16 * TI + l16;
-      double old[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int col = 16 * TJ + lk + 4 * r;
-        old[r] = L[at(c0 + min(row, mt - 1), c0 + min(col, mt - 1))];
-      }
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int col = 16 * TJ + lk + 4 * r;
-        if (row < mt && col < mt && row >= col) L[at(c0 + row, c0 + col)] = old[r] - acc[r];
-      }
-    }
-    __syncthreads();
-  }
-  // ---- X = L^{-T}: strict lower part of X (upper part of L^{-1}) is zero ----
-  for (int64_t idx = tid; idx < (int64_t)n * n; idx += nt) {
+  const int64_t mo = t.mat_off[s], nn = (int64_t)n * n;
+  for (int64_t idx = (int64_t)blockIdx.y * 256 + threadIdx.x; idx < nn; idx += (int64_t)gridDim.y * 256) {
+    work[mo + idx] = S[mo + idx];
     const int r = (int)(idx / n), c = (int)(idx - (int64_t)r * n);
-    if (c < r) Xm[idx] = 0.0;
+    if (c < r) X[mo + idx] = 0.0;
   }
-  // diagonal blocks: thread (I, c) solves column c of L_II^{-1}
-  const int NB = (n + 15) >> 4;
-  for (int idx = tid; idx < 16 * NB; idx += nt) {
-    const int I = idx >> 4, c = idx & 15, o = 16 * I, b = min(16, n - o);
-    if (c >= b) continue;
-    double y[16];
+}
+
+__global__ __launch_bounds__(256) void k_chol_panel(Topo t, const int* order, double* work, double* X,
+                                                    SysState* status, int k0) {
+  const int s = order[blockIdx.x];
+  const int n = t.ao_off[s + 1] - t.ao_off[s];
+  const int r0 = k0 + kCholPanel + (int)blockIdx.y * 256;  // this block's first row
+  if (k0 >= n || (blockIdx.y > 0 && r0 >= n)) return;
+  double* __restrict__ L = work + t.mat_off[s];
+  const int tid = threadIdx.x, jn = min(kCholPanel, n - k0);
+  constexpr int P = kCholPanel;
+  __shared__ double sL[P][P + 1];  // sL[c][r] = L11(r, c); diagonal: 1 / pivot
+  // the row below the panel, in flight while the diagonal block is factored
+  const int row = r0 + tid;
+  double x[P];
+  if (row < n) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      y[r] = 0.0;
-      if (r < c || r >= b) continue;
-      double v = r == c ? 1.0 : 0.0;
+    for (int c = 0; c < P; ++c) x[c] = L[(int64_t)row + (int64_t)(k0 + c) * n];  // jn = P where rows follow
+  }
+  if (tid < 64) {
+    // lane r < P: row r, identity past jn; entries above the diagonal are never used
+    double a[P];
+    const int r = min(tid, P - 1);
 #pragma unroll
-      for (int k = 0; k < r; ++k)
-        if (k >= c) v -= L[at(o + r, o + k)] * y[k];
-      y[r] = v / L[at(o + r, o + r)];
-      Xm[(int64_t)(o + c) * n + o + r] = y[r];
+    for (int c = 0; c < P; ++c)
+      a[c] = r < jn && c <= r ? L[(int64_t)(k0 + r) + (int64_t)(k0 + c) * n] : (r == c ? 1.0 : 0.0);
+    bool bad = false;
+    static_for<0, P>([&](auto J) __attribute__((always_inline)) {
+      constexpr int j = decltype(J)::value;
+      double d = lane_value(a[j], j);
+      if (!(d > 0.0)) {
+        bad = true;
+        d = 1.0;
+      }
+      const double piv = sqrt(d), ipiv = 1.0 / piv;
+      const double l = a[j] * ipiv;  // L(r, j) on lanes r > j
+      if (tid > j && tid < P) sL[j][tid] = l;
+      if (tid == j) {
+        sL[j][j] = ipiv;
+        a[j] = piv;
+      } else {
+        a[j] = l;
+      }
+      static_for<j + 1, P>([&](auto K) __attribute__((always_inline)) {
+        constexpr int k = decltype(K)::value;
+        a[k] = fma(-l, lane_value(l, k), a[k]);
+      });
+    });
+    if (blockIdx.y == 0) {
+      double* __restrict__ Xm = X + t.mat_off[s];
+#pragma unroll
+      for (int c = 0; c < P; ++c)
+        if (tid < jn && c <= tid) Xm[(int64_t)(k0 + c) * n + k0 + tid] = a[c];
+      if (bad && tid == 0) status[s].status = 8;
     }
   }
   __syncthreads();
-  // block rows I >= 1: blocks J < I, one per wavefront at a time
-  for (int I = 1; I < NB; ++I) {
+  if (row < n) {
+#pragma unroll
+    for (int c = 0; c < P; ++c) {
+      x[c] *= sL[c][c];
+#pragma unroll
+      for (int k = c + 1; k < P; ++k) x[k] = fma(-x[c], sL[c][k], x[k]);
+    }
+#pragma unroll
+    for (int c = 0; c < P; ++c) L[(int64_t)row + (int64_t)(k0 + c) * n] = x[c];
+  }
+}
+
+__global__ __launch_bounds__(256) void k_chol_trailing(Topo t, const int* order, double* work, const double* X,
+                                                       int k0) {
+  const int s = order[blockIdx.x];
+  const int n = t.ao_off[s + 1] - t.ao_off[s];
+  if (k0 >= n) return;
+  double* __restrict__ L = work + t.mat_off[s];
+  const int jn = min(kCholPanel, n - k0);
+  auto at = [n](int r, int c) __attribute__((always_inline)) { return (int64_t)r + (int64_t)c * n; };
+  if (blockIdx.y == 0)
+    for (int idx = threadIdx.x; idx < jn * jn; idx += 256) {
+      const int r = idx % jn, c = idx / jn;
+      if (c <= r) L[at(k0 + r, k0 + c)] = X[t.mat_off[s] + (int64_t)(k0 + c) * n + k0 + r];
+    }
+  const int c0 = k0 + jn, mt = n - c0;  // rows and columns >= c0
+  const int nb16 = (mt + 15) >> 4;
+  const int ntiles = nb16 * (nb16 + 1) / 2;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, lk = lane >> 4;
+  for (int tile = (int)blockIdx.y * 4 + wv; tile < ntiles; tile += (int)gridDim.y * 4) {
+    int TI = (int)((sqrt(8.0 * tile + 1.0) - 1.0) * 0.5);
+    while (TI * (TI + 1) / 2 > tile) --TI;
+    while ((TI + 1) * (TI + 2) / 2 <= tile) ++TI;
+    const int TJ = tile - TI * (TI + 1) / 2;
+    const int rr = 16 * TI + l16, cc = 16 * TJ + l16;  // this lane's row of P (rows), of Q (columns)
+    const int rrc = c0 + min(rr, mt - 1), ccc = c0 + min(cc, mt - 1);
+    double xa[kCholPanel / 4], xb[kCholPanel / 4], old[4];
+#pragma unroll
+    for (int q = 0; q < kCholPanel / 4; ++q) {
+      xa[q] = L[at(ccc, k0 + 4 * q + lk)];  // a panel with rows below it is full
+      xb[q] = L[at(rrc, k0 + 4 * q + lk)];
+    }
+    // acc[r] = D[row = 16 TI + l16][col = 16 TJ + lk + 4 r]
+#pragma unroll
+    for (int r = 0; r < 4; ++r) old[r] = L[at(rrc, c0 + min(16 * TJ + lk + 4 * r, mt - 1))];
+    mfma_d4 acc = mfma_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int q = 0; q < kCholPanel / 4; ++q)
+      acc = mfma_16x16x4(cc < mt ? xa[q] : 0.0, rr < mt ? xb[q] : 0.0, acc);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int col = 16 * TJ + lk + 4 * r;
+      if (rr < mt && col < mt && rr >= col) L[at(c0 + rr, c0 + col)] = old[r] - acc[r];
+    }
+  }
+}
+
+__global__ __launch_bounds__(64) void k_chol_diagonal(Topo t, const int* order, const double* work, double* X) {
+  const int s = order[blockIdx.x];
+  const int n = t.ao_off[s + 1] - t.ao_off[s];
+  const double* __restrict__ L = work + t.mat_off[s];
+  double* __restrict__ Xm = X + t.mat_off[s];
+  const int idx = (int)blockIdx.y * 64 + threadIdx.x;
+  const int c = idx & 15, o = idx & ~15, b = min(16, n - o);
+  if (c >= b) return;  // also where the block starts past n
+  double y[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    y[r] = 0.0;
+    if (r < c || r >= b) continue;
+    double v = r == c ? 1.0 : 0.0;
+#pragma unroll
+    for (int k = 0; k < r; ++k)
+      if (k >= c) v -= L[(int64_t)(o + r) + (int64_t)(o + k) * n] * y[k];
+    y[r] = v / L[(int64_t)(o + r) + (int64_t)(o + r) * n];
+    Xm[(int64_t)(o + c) * n + o + r] = y[r];
+  }
+}
+
+__global__ __launch_bounds__(512) void k_chol_invert(Topo t, const int* order, const double* work, double* X) {
+  const int s = order[blockIdx.x];
+  const int n = t.ao_off[s + 1] - t.ao_off[s];
+  const int NB = (n + 15) >> 4, J = (int)blockIdx.y;
+  if (J >= NB) return;
+  const double* __restrict__ L = work + t.mat_off[s];
+  double* Xm = X + t.mat_off[s];
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, lk = lane >> 4, oj = 16 * J;
+  __shared__ double sP[8][16][17];
+  for (int I = J + 1; I < NB; ++I) {
     const int oi = 16 * I;
     const int ri = oi + l16;  // this lane's row of block row I
     const bool rin = ri < n;
     const int ric = min(ri, n - 1);
-    for (int J = wv; J < I; J += nw) {
-      const int oj = 16 * J;
-      mfma_d4 acc = mfma_d4{0.0, 0.0, 0.0, 0.0};
-      for (int K = J; K < I; ++K) {
-        const int ok = 16 * K;
-        double xa[4], xb[4];
+    double bv[4];
+    if (wv == 0) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int k = 4 * q + lk;
-          xa[q] = Xm[(int64_t)(oj + l16) * n + ok + k];  // Linv(ok + k, oj + l16)
-          xb[q] = L[at(ric, ok + k)];                    // L(oi + l16, ok + k)
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) acc = mfma_16x16x4(xa[q], rin ? xb[q] : 0.0, acc);
+      for (int q = 0; q < 4; ++q) {
+        const int k = 4 * q + lk;
+        // Linv(oi + l16, oi + k), zero above its diagonal
+        bv[q] = rin && k <= l16 ? Xm[(int64_t)(oi + min(k, n - 1 - oi)) * n + ric] : 0.0;
       }
-      // S[l16][lk + 4 r] -> LDS; then Linv_IJ = -Linv_II S
-      double(*st)[17] = sS[wv];
+    }
+    mfma_d4 acc = mfma_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 2
+    for (int K = J + wv; K < I; K += 8) {
+      const int ok = 16 * K;
+      double xa[4], xb[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) st[l16][lk + 4 * r] = acc[r];
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      for (int q = 0; q < 4; ++q) {
+        const int k = 4 * q + lk;
+        // Linv(ok + k, oj + l16), zero above the diagonal of block J itself
+        xa[q] = Xm[(int64_t)(oj + l16) * n + ok + k];
+        xb[q] = L[(int64_t)ric + (int64_t)(ok + k) * n];  // L(oi + l16, ok + k)
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc = mfma_16x16x4(xa[q], rin ? xb[q] : 0.0, acc);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sP[wv][l16][lk + 4 * r] = acc[r];
+    __syncthreads();
+    if (wv == 0) {
+      const int nw = min(8, I - J);
       mfma_d4 acc2 = mfma_d4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int k = 4 * q + lk;
-        const bool kin = oi + k < n;
-        const double a = st[k][l16];                                          // S[k][l16]
-        const double bv = Xm[(int64_t)(oi + (kin ? k : 0)) * n + ric];       // Linv(oi + l16, oi + k)
-        acc2 = mfma_16x16x4(a, rin && kin ? bv : 0.0, acc2);
+        double a = sP[0][k][l16];  // S[k][l16]
+        for (int w = 1; w < nw; ++w) a += sP[w][k][l16];
+        acc2 = mfma_16x16x4(a, bv[q], acc2);
       }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       if (rin) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) Xm[(int64_t)(oj + lk + 4 * r) * n + ri] = -acc2[r];
@@ -1914,7 +1970,6 @@ __global__ __launch_bounds__(512) void k_cholesky_blocked(Topo t, const int* ord
     }
     __syncthreads();
   }
-  if (tid == 0 && bad) status[s].status = 8;
 }
 
 // ---------------------------------------------------------------------------
