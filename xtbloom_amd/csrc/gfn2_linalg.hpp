@@ -2852,6 +2852,7 @@ __device__ __forceinline__ int eig_occupations(const Topo& t, int s, int n, cons
 // kocc; every member of a needed cluster is computed so the cluster stays
 // orthogonal.  An unsplit T is one block [0, n) of 1-norm tnorm1; split blocks
 // are found and measured by the thread that needs them.
+template <int U>
 __device__ __forceinline__ void eig_vector(int j, int n, int kocc, const double* d, const double* e, const double* lam,
                                            const int* rnk, bool unsplit, double tnorm1, double pivmin,
                                            const EigenScratch& sc, int64_t mo, double* __restrict__ Z, double* zscale,
@@ -2936,68 +2937,131 @@ __device__ __forceinline__ void eig_vector(int j, int n, int kocc, const double*
       F0[at] = c0; F1[at] = 0.0; F2[at] = 0.0; FM[at] = 0.0; FP[at] = 0.0;
     }
     for (int i = b0; i < b1; ++i) Z[(int64_t)i * n + cj] = start_component(jj, i - b0);
+    // The passes below read and write one column of global memory: U rows' loads
+    // are in flight before the first of them is used.  k_eig_vectors takes eight:
+    // close levels at 1142 AOs then hold its wavefront for 1.7 ms instead of 3.1.
+    // k_tridiag_eigen takes one: eight cost it 90 VGPRs and a wavefront per SIMD
+    // (1% of a call of 512 systems).
+    auto scale_rows = [&](double f) __attribute__((always_inline)) {
+      int i = b0;
+      for (; i + U <= b1; i += U) {
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = Z[(int64_t)(i + u) * n + cj];
+#pragma unroll
+        for (int u = 0; u < U; ++u) Z[(int64_t)(i + u) * n + cj] = v[u] * f;
+      }
+      for (; i < b1; ++i) Z[(int64_t)i * n + cj] *= f;
+    };
     for (int it = 0; it <= kInverseIterations; ++it) {
       // orthogonalize against the cluster members already finished
       for (int p = j; p < jj; ++p) {
+        const int cp = rnk[p];
         double dot = 0.0;
-        for (int i = b0; i < b1; ++i) dot += Z[(int64_t)i * n + rnk[p]] * Z[(int64_t)i * n + cj];
-        for (int i = b0; i < b1; ++i) Z[(int64_t)i * n + cj] -= dot * Z[(int64_t)i * n + rnk[p]];
+#pragma unroll U
+        for (int i = b0; i < b1; ++i) dot += Z[(int64_t)i * n + cp] * Z[(int64_t)i * n + cj];
+        int i = b0;
+        for (; i + U <= b1; i += U) {
+          double v[U], w[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            v[u] = Z[(int64_t)(i + u) * n + cj];
+            w[u] = Z[(int64_t)(i + u) * n + cp];
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) Z[(int64_t)(i + u) * n + cj] = v[u] - dot * w[u];
+        }
+        for (; i < b1; ++i) Z[(int64_t)i * n + cj] -= dot * Z[(int64_t)i * n + cp];
       }
       if (it == kInverseIterations) break;
       // scale to unit max-norm, then solve (T_b - x I) y = r
       double rmax = 0.0;
+#pragma unroll U
       for (int i = b0; i < b1; ++i) rmax = fmax(rmax, fabs(Z[(int64_t)i * n + cj]));
       const double rs = rmax > 0.0 ? 1.0 / rmax : 1.0;
-      for (int i = b0; i < b1; ++i) Z[(int64_t)i * n + cj] *= rs;
       // forward elimination; the running entry stays in a register (it is
       // the one stored one row earlier), so only independent loads remain
       {
-        double cur = Z[(int64_t)b0 * n + cj];
-        for (int k = 0; k < bn - 1; ++k) {
-          const int64_t at = (int64_t)(b0 + k) * n + cj;
-          double rk = cur, rn = Z[at + n];
-          if (FP[at] != 0.0) { const double tmp = rk; rk = rn; rn = tmp; }
+        double cur = Z[(int64_t)b0 * n + cj] * rs;
+        auto step = [&](int64_t at, double zn, double fp, double fm) __attribute__((always_inline)) {
+          double rk = cur, rn = zn * rs;
+          if (fp != 0.0) { const double tmp = rk; rk = rn; rn = tmp; }
           Z[at] = rk;
-          cur = rn - FM[at] * rk;
+          cur = rn - fm * rk;
+        };
+        int k = 0;
+        for (; k + U <= bn - 1; k += U) {
+          double zn[U], fp[U], fm[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const int64_t at = (int64_t)(b0 + k + u) * n + cj;
+            zn[u] = Z[at + n];
+            fp[u] = FP[at];
+            fm[u] = FM[at];
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) step((int64_t)(b0 + k + u) * n + cj, zn[u], fp[u], fm[u]);
+        }
+        for (; k < bn - 1; ++k) {
+          const int64_t at = (int64_t)(b0 + k) * n + cj;
+          step(at, Z[at + n], FP[at], FM[at]);
         }
         Z[(int64_t)(b1 - 1) * n + cj] = cur;
       }
-      // back substitution with the two entries below in registers
+      // back substitution with the two entries below in registers (F1 of the
+      // last row and F2 of the last two are zero)
       {
         double z1 = 0.0, z2 = 0.0;  // solution entries k + 1, k + 2
-        for (int k = bn - 1; k >= 0; --k) {
-          const int64_t at = (int64_t)(b0 + k) * n + cj;
-          double r = Z[at];
-          if (k + 1 < bn) r -= F1[at] * z1;
-          if (k + 2 < bn) r -= F2[at] * z2;
-          double u = F0[at];
+        auto step = [&](int64_t at, double r, double f0, double f1, double f2) __attribute__((always_inline)) {
+          r -= f1 * z1;
+          r -= f2 * z2;
+          double u = f0;
           if (fabs(u) < ptol) u = u < 0.0 ? -ptol : ptol;
           const double zk = r / u;
           Z[at] = zk;
           z2 = z1;
           z1 = zk;
+        };
+        int k = bn - 1;
+        for (; k - U + 1 >= 0; k -= U) {
+          double r[U], f0[U], f1[U], f2[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const int64_t at = (int64_t)(b0 + k - u) * n + cj;
+            r[u] = Z[at];
+            f0[u] = F0[at];
+            f1[u] = F1[at];
+            f2[u] = F2[at];
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) step((int64_t)(b0 + k - u) * n + cj, r[u], f0[u], f1[u], f2[u]);
+        }
+        for (; k >= 0; --k) {
+          const int64_t at = (int64_t)(b0 + k) * n + cj;
+          step(at, Z[at], F0[at], F1[at], F2[at]);
         }
       }
       // normalize
       double nrm = 0.0, ymax = 0.0;
+#pragma unroll U
       for (int i = b0; i < b1; ++i) ymax = fmax(ymax, fabs(Z[(int64_t)i * n + cj]));
       const double ys = ymax > 0.0 ? 1.0 / ymax : 1.0;
+#pragma unroll U
       for (int i = b0; i < b1; ++i) {
         const double y = Z[(int64_t)i * n + cj] * ys;
         nrm += y * y;
       }
-      const double sc2 = ys / sqrt(nrm);
-      for (int i = b0; i < b1; ++i) Z[(int64_t)i * n + cj] *= sc2;
+      scale_rows(ys / sqrt(nrm));
     }
     // final normalization; sign: largest-magnitude component positive
     double nrm = 0.0, big = 0.0;
+#pragma unroll U
     for (int i = b0; i < b1; ++i) {
       const double y = Z[(int64_t)i * n + cj];
       nrm += y * y;
       if (fabs(y) > fabs(big)) big = y;
     }
-    const double f = (big < 0.0 ? -1.0 : 1.0) / sqrt(nrm);
-    for (int i = b0; i < b1; ++i) Z[(int64_t)i * n + cj] *= f;
+    scale_rows((big < 0.0 ? -1.0 : 1.0) / sqrt(nrm));
   }
 }
 
@@ -3088,7 +3152,7 @@ __global__ __launch_bounds__(256) void k_tridiag_eigen(Topo t, const int* order,
   __shared__ double tnorm1;
   if (unsplit) eig_norm1(d, e, n, red, tnorm1);
   for (int j = tid; j < n; j += nt)
-    eig_vector(j, n, kocc, d, e, lam, rnk, unsplit, tnorm1, pivmin, sc, mo, Zall + mo, zscale, co, s, t.ao_off[s]);
+    eig_vector<1>(j, n, kocc, d, e, lam, rnk, unsplit, tnorm1, pivmin, sc, mo, Zall + mo, zscale, co, s, t.ao_off[s]);
 }
 
 // Block-wide maximum (blockDim.x <= 1024; red holds blockDim.x / 64 doubles).
@@ -3114,7 +3178,7 @@ __device__ __forceinline__ double block_max(double v, double* red) {
 // Bound: the serial chains of a lane (about nine Sturm passes, four recurrences
 // of n rows).  Measured against one 256-thread block per system: 7.8 -> 1.5 ms
 // a launch at 1142 AOs (eigenvalues 0.82, occupations 0.16, vectors 0.49; a
-// geometry whose close eigenvalues need inverse iteration takes 3.1 for the
+// geometry whose close eigenvalues need inverse iteration takes 1.7 for the
 // vectors), 0.74 -> 0.45 ms for 14 systems of 258-482 AOs.
 constexpr int kEigSplitAO = 2048;
 
@@ -3209,7 +3273,7 @@ __global__ __launch_bounds__(64) void k_eig_vectors(Topo t, const int* order, co
   __syncthreads();
   const int j = 64 * blockIdx.x + threadIdx.x;
   if (j < n)
-    eig_vector(j, n, kocc, d, e, lam, rnk, unsplit, tnorm1, pivmin, sc, mo, Zall + mo, zscale_all + t.ao_off[s], co, s,
+    eig_vector<8>(j, n, kocc, d, e, lam, rnk, unsplit, tnorm1, pivmin, sc, mo, Zall + mo, zscale_all + t.ao_off[s], co, s,
                t.ao_off[s]);
 }
 
