@@ -494,11 +494,12 @@ __device__ __forceinline__ double gamma_row(const double* Gm, int i, int ns, con
 // kSliceAtoms atoms each; every block stages all atoms by itself and needs
 // nothing of the others.  The cut depends on the system alone, so its sums do not
 // change with the batch around it.  Measured at 572 atoms: k_potentials 1650 ->
-// 98 us, the energies and the mixing 1410 -> 152 us.  Below 128 atoms the cut
+// 104 us, the energies and the mixing 1410 -> 165 us (161 and 230 us with 32 atoms
+// a block).  Below 128 atoms the cut
 // gained 1% for one system of 62 atoms and cost 2 to 4% for 128 and 256 systems
 // of that size, which fill the chip by themselves.
 constexpr int kSliceFrom = 128;
-constexpr int kSliceAtoms = 32;
+constexpr int kSliceAtoms = 16;
 
 // Potentials from the state x: v_sh (with the atom potential folded in), v_D, v_Q
 // (reference scc_driver.cpp:2363-2560, aes2.cpp:451-545, d4.cpp:896-1032).
