@@ -613,9 +613,10 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
   // systems above kWideAtoms atoms are among the first n_wide of the size order
   int n_wide = 0, wide_top = 0;
   bool any_narrow = false;
-  // back-transformation tasks of the systems above 2048, 1024, 512 and 256 AOs
-  // (prefixes of `back`)
-  size_t n_back[4] = {0, 0, 0, 0};
+  // back-transformation tasks of the systems above 2048, 1536, 1024, 512 and 256
+  // AOs (prefixes of `back`)
+  constexpr int kBackLimits[5] = {2048, 1536, 1024, 512, 256};
+  size_t n_back[5] = {0, 0, 0, 0, 0};
   for (int i = 0; i < B; ++i) {
     const int s = T.order[i];
     const int n = T.ao_off[s + 1] - T.ao_off[s];
@@ -635,8 +636,8 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
         if (a >= b) lower.push_back({s, a, b});
       }
     for (int j0 = 0; j0 < n; j0 += n > 256 ? kWyCols : kBackCols) back.push_back({s, j0});
-    for (int c = 0; c < 4; ++c)
-      if (n > 2048 >> c) n_back[c] = back.size();
+    for (int c = 0; c < 5; ++c)
+      if (n > kBackLimits[c]) n_back[c] = back.size();
     for (int r0 = 0; r0 < n; r0 += kFockTile)
       for (int c0 = r0; c0 < n; c0 += kFockTile) chunks.push_back({s, r0, c0});
   }
@@ -1326,11 +1327,12 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
     };
     back_wy(k_backtransform_wy<0>, 0, n_back[0]);
     back_wy(k_backtransform_wy<16>, n_back[0], n_back[1]);
-    back_wy(k_backtransform_wy<8>, n_back[1], n_back[2]);
-    back_wy(k_backtransform_wy<4>, n_back[2], n_back[3]);
-    if (back.size() > n_back[3])
-      hipLaunchKernelGGL(k_backtransform, dim3((unsigned)(back.size() - n_back[3])), dim3(kBackThreads), 0, sm, t,
-                         d_back + n_back[3], dA, dZ, d_wyT, dY, d_kocc, d_zscale, d_active);
+    back_wy(k_backtransform_wy<12>, n_back[1], n_back[2]);
+    back_wy(k_backtransform_wy<8>, n_back[2], n_back[3]);
+    back_wy(k_backtransform_wy<4>, n_back[3], n_back[4]);
+    if (back.size() > n_back[4])
+      hipLaunchKernelGGL(k_backtransform, dim3((unsigned)(back.size() - n_back[4])), dim3(kBackThreads), 0, sm, t,
+                         d_back + n_back[4], dA, dZ, d_wyT, dY, d_kocc, d_zscale, d_active);
     HIP_TRY(probe_end(kKBacktransform, 0.0, 0.0));
     if (rp) rp->bt = last_probe();
     // C = X Y (the kocc leading columns), P = C diag(f) C^T

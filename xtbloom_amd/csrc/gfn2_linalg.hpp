@@ -3636,7 +3636,8 @@ __global__ __launch_bounds__(512) void k_wy_factors(Topo t, const int* order, co
 // (issued before the barriers, so that L2's latency overlaps the products).
 // MT row tiles per wavefront in registers (n <= 128 MT); MT = 0 keeps the
 // columns in Y.  Measured against eight reflectors at a time on the vector
-// units: 10.6 -> 0.70 ms at 1142 AOs, 375 -> 96 us for 14 systems of 258-482 AOs.
+// units: 10.6 -> 0.53 ms at 1142 AOs (0.70 with MT = 16, which spills twice as
+// much as MT = 12), 375 -> 96 us for 14 systems of 258-482 AOs.
 constexpr int kWyThreads = 512;
 constexpr int kWyCols = 16;
 
