@@ -258,7 +258,8 @@ __global__ __launch_bounds__(512) void k_energy_mix(Topo t, const int* order, un
     // (beta + 0.01^2) x = coef by Cholesky, one wavefront, lane r on row r
     // (hc <= 64); LDS ordering inside the wavefront, no block barriers.  Bound:
     // the chain of hc pivots.  Serial on one lane the kernel took 25.5 us for
-    // one water molecule and 43 us at 122 AOs; so it takes 20.8 and 38 us.
+    // one water molecule and 43 us at 122 AOs; so it took 20.8 and 38 us (17.5
+    // and 32 with the staging by eight lanes an atom).
     if (tid < 64) {
       auto fence = [] __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
       for (int x = tid; x < hc * hc; x += 64) {
