@@ -71,3 +71,39 @@ def check(sizes):
     assert np.abs(out.energies - ref["energies"]).max() <= E_TOL
     assert np.abs(out.forces + ref["gradient"]).max() <= F_TOL
     assert np.abs(out.charges - ref["charges"]).max() <= Q_TOL
+
+
+def test_result_depends_on_the_system_alone(monkeypatch):
+    """64 systems of 302 AOs take 640 team members, more than the chip holds at once:
+    the bits of one lane are those of two lanes, and of systems computed alone."""
+    rng = np.random.default_rng(64)
+    systems = [workloads.alkane(50, rng) for _ in range(64)]
+    b = workloads.from_systems(systems)
+    ctx = interface.Context("hip", 0)
+
+    def run(batch):
+        return interface.compute_arrays(ctx, batch.atom_offsets, batch.atomic_numbers, batch.positions,
+                                        batch.molecular_charges, batch.unpaired_electrons)
+
+    try:
+        print("case 64 systems of 302 AOs: one lane, two lanes, alone", flush=True)
+        monkeypatch.setenv("XTBLOOM_AMD_LANES", "1")
+        one = run(b)
+        assert np.all(one.per_system_status == 0)
+        monkeypatch.setenv("XTBLOOM_AMD_LANES", "2")
+        two = run(b)
+        monkeypatch.setenv("XTBLOOM_AMD_LANES", "1")
+        for name in ("energies", "charges", "scc_iterations", "per_system_status"):
+            assert np.array_equal(getattr(two, name), getattr(one, name)), name
+        for i in (0, 40, 63):
+            alone = run(workloads.from_systems([systems[i]]))
+            a0, a1 = b.atom_offsets[i], b.atom_offsets[i + 1]
+            assert alone.energies[0] == one.energies[i] and np.array_equal(alone.charges, one.charges[a0:a1])
+            assert alone.scc_iterations[0] == one.scc_iterations[i]
+    finally:
+        ctx.close()
+    ref = O.batch(b.atom_offsets[:3], b.atomic_numbers, b.positions, b.molecular_charges[:2],
+                  b.unpaired_electrons[:2], threads=2)
+    assert np.abs(one.energies[:2] - ref["energies"]).max() <= E_TOL
+    a1 = b.atom_offsets[2]
+    assert np.abs(one.forces[:a1] + ref["gradient"][:a1]).max() <= F_TOL

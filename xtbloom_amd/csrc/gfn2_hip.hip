@@ -641,25 +641,15 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
     for (int r0 = 0; r0 < n; r0 += kFockTile)
       for (int c0 = r0; c0 < n; c0 += kFockTile) chunks.push_back({s, r0, c0});
   }
-  // Systems reduced by teams: [n_team0, n_team1) of the size order, those of 257
-  // to kTeamN AOs, when their members' turns on the chip cost less than one
-  // workgroup per system does.  A turn of teams takes about 5 us a column
-  // (measured 4.5 at 482 AOs, 5.5 at 1142); one workgroup takes 0.04 us per
-  // column and AO (9.0 ms at 482 AOs).
-  int n_team0 = 0, n_team1 = 0;
-  {
-    int64_t members = 0;
-    while (n_team0 < n_large && T.ao_off[T.order[n_team0] + 1] - T.ao_off[T.order[n_team0]] > kTeamN) ++n_team0;
-    for (int i = n_team0; i < n_large; ++i) members += team_size(T.ao_off[T.order[i] + 1] - T.ao_off[T.order[i]]);
-    n_team1 = n_team0;
-    if (n_team0 < n_large) {
-      const int n_top = T.ao_off[T.order[n_team0] + 1] - T.ao_off[T.order[n_team0]];
-      const double team_us = 5.0 * (double)((members + 255) / 256);
-      const double block_us = 0.04 * n_top * (double)((n_large - n_team0 + 255) / 256);
-      if (team_us < block_us) n_team1 = n_large;
-    }
-    if (n_team1 == n_team0) n_team0 = n_team1 = n_large;
-  }
+  // Systems reduced by teams: [n_team0, n_large) of the size order, those of 257
+  // to kTeamN AOs.  The system's size alone decides, so that its result depends
+  // neither on the batch around it nor on the lanes.  Reduction of eleven rounds
+  // by teams against one workgroup per system: 8.8 and 33.1 ms for 32 systems of
+  // 260 AOs, 61.6 and 113 ms for 64 of 482, 178 and 457 ms for 32 of 902.  Only
+  // where the single workgroups fill the chip are teams slower (239 and 142 ms
+  // for 256 systems of 482).
+  int n_team0 = 0;
+  while (n_team0 < n_large && T.ao_off[T.order[n_team0] + 1] - T.ao_off[T.order[n_team0]] > kTeamN) ++n_team0;
   // WY blocks of the largest system, in groups of eight (k_wy_factors)
   const unsigned wy_groups =
       n_large > 0 ? (unsigned)((T.ao_off[T.order[0] + 1] - T.ao_off[T.order[0]] - 2 + 8 * kWyBlock - 1) / (8 * kWyBlock)) : 0;
@@ -1263,15 +1253,15 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
     // eigenpairs of H' (A is overwritten by the reflectors; T, H, C, P, W serve as scratch)
     HIP_TRY(probe_begin(kKTridiag));
     // systems are ordered largest first: of the n_large above 256 AOs those in
-    // [n_team0, n_team1) are reduced by teams of workgroups, the others (and
+    // [n_team0, n_large) are reduced by teams of workgroups, the others (and
     // the ones whose team left at the gate) by one workgroup each; k_tridiag
     // takes the teams' last columns and the systems of at most 256 AOs
-    const bool teams = n_team1 > n_team0;
+    const bool teams = n_large > n_team0;
     if (teams) {
       const int n_top = T.ao_off[T.order[n_team0] + 1] - T.ao_off[T.order[n_team0]];
-      hipLaunchKernelGGL(k_team_init, dim3(n_team1 - n_team0), dim3(256), 0, sm, t, d_order + n_team0, d_active, dZ,
+      hipLaunchKernelGGL(k_team_init, dim3(n_large - n_team0), dim3(256), 0, sm, t, d_order + n_team0, d_active, dZ,
                          opt.teams ? 0u : kTeamClosed);
-      hipLaunchKernelGGL(k_tridiag_team, dim3(team_size(n_top), n_team1 - n_team0), dim3(512), 0, sm, t,
+      hipLaunchKernelGGL(k_tridiag_team, dim3(team_size(n_top), n_large - n_team0), dim3(512), 0, sm, t,
                          d_order + n_team0, dA, d_td, d_te, dZ, d_active, d_st);
     }
     auto blocked = [&](auto* kernel, int first, int end, double* zteam) {
@@ -1279,14 +1269,12 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
         hipLaunchKernelGGL(kernel, dim3(end - first), dim3(512), 0, sm, t, d_order + first, dA, d_td, d_te, dT,
                            d_active, d_xl, zteam);
     };
-    blocked(k_tridiag_blocked<true>, 0, std::min(n_xl, n_team0), nullptr);
-    blocked(k_tridiag_blocked<true>, n_team0, std::min(n_xl, n_team1), dZ);
-    blocked(k_tridiag_blocked<false>, std::max(n_xl, n_team0), n_team1, dZ);
-    blocked(k_tridiag_blocked<false>, n_xl, n_team0, nullptr);
-    const int tri0 = teams ? n_team0 : n_large;
-    if (tri0 < B)
-      hipLaunchKernelGGL(k_tridiag, dim3(B - tri0), dim3(512), 0, sm, t, d_order + tri0, dA, d_td, d_te, d_wyT, dZ,
-                         d_active);
+    blocked(k_tridiag_blocked<true>, 0, n_team0, nullptr);
+    blocked(k_tridiag_blocked<true>, n_team0, n_xl, dZ);
+    blocked(k_tridiag_blocked<false>, n_xl, n_large, dZ);
+    if (n_team0 < B)
+      hipLaunchKernelGGL(k_tridiag, dim3(B - n_team0), dim3(512), 0, sm, t, d_order + n_team0, dA, d_td, d_te, d_wyT,
+                         dZ, d_active);
     HIP_TRY(probe_end(kKTridiag, 0.0, 0.0));
     if (rp) rp->tri = last_probe();
     HIP_TRY(probe_begin(kKTridiagEigen));
