@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle as O
-from xtbloom_amd import interface, workloads
+from xtbloom_amd import interface, library, workloads
 
 pytestmark = pytest.mark.gpu
 
@@ -107,3 +107,32 @@ def test_result_depends_on_the_system_alone(monkeypatch):
     assert np.abs(one.energies[:2] - ref["energies"]).max() <= E_TOL
     a1 = b.atom_offsets[2]
     assert np.abs(one.forces[:a1] + ref["gradient"][:a1]).max() <= F_TOL
+
+
+def test_closed_gate_changes_no_bit(monkeypatch):
+    """The one workgroup that reduces a system whose team left at the gate forms every
+    sum as the team does; that it ran shows in the time of the reduction (a team of 40
+    workgroups against one)."""
+    rng = np.random.default_rng(1280)
+    b = workloads.from_systems([workloads.alkane(213, rng), workloads.alkane(50, rng), stack(257, rng)])
+    ctx = interface.Context("hip", 0)
+
+    def run():
+        return interface.compute_arrays(ctx, b.atom_offsets, b.atomic_numbers, b.positions, b.molecular_charges,
+                                        b.unpaired_electrons, determinism=library.DETERMINISM_REPRODUCIBLE,
+                                        kernel_stats=["tridiag"])
+
+    try:
+        print("case gate: 1280, 302 and 257 AOs by teams", flush=True)
+        team = run()
+        monkeypatch.setenv("XTBLOOM_AMD_TEAMS", "0")
+        print("case gate: the same, gates closed", flush=True)
+        solo = run()
+    finally:
+        ctx.close()
+    assert np.all(team.per_system_status == 0)
+    for name in ("energies", "forces", "charges", "scc_iterations", "per_system_status"):
+        assert np.array_equal(getattr(solo, name), getattr(team, name)), name
+    ms = [o.extension["kernel_stats"]["tridiag"]["ms"] for o in (team, solo)]
+    print("reduction: teams %.1f ms, one workgroup %.1f ms" % tuple(ms), flush=True)
+    assert ms[1] > 3.0 * ms[0]

@@ -55,8 +55,9 @@ struct RunOptions {
   // split-precision FP32 matrix-core density products: P in the SCC rounds
   // whose mixer residual is above 1e-3 (and the first round), W always
   bool split32 = false;
-  // reductions by teams of workgroups; off, every team finds its gate closed
-  // and leaves (the path it takes when the chip is held by something else)
+  // reductions by teams of workgroups; off, every team finds its gate closed and
+  // leaves (the path it takes when the chip is held by something else), and one
+  // workgroup does the same arithmetic
   bool teams = true;
   // allocate nothing: the device workspace is the fixed per-GPU array of
   // kNoAllocWorkspaceBytes (a larger batch is rejected before any kernel),

@@ -1253,9 +1253,9 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
     // eigenpairs of H' (A is overwritten by the reflectors; T, H, C, P, W serve as scratch)
     HIP_TRY(probe_begin(kKTridiag));
     // systems are ordered largest first: of the n_large above 256 AOs those in
-    // [n_team0, n_large) are reduced by teams of workgroups, the others (and
-    // the ones whose team left at the gate) by one workgroup each; k_tridiag
-    // takes the teams' last columns and the systems of at most 256 AOs
+    // [n_team0, n_large) are reduced by teams of workgroups (k_tridiag_solo takes
+    // the ones whose team left at the gate), the others by one workgroup each;
+    // k_tridiag takes the teams' last columns and the systems of at most 256 AOs
     const bool teams = n_large > n_team0;
     if (teams) {
       const int n_top = T.ao_off[T.order[n_team0] + 1] - T.ao_off[T.order[n_team0]];
@@ -1263,15 +1263,12 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
                          opt.teams ? 0u : kTeamClosed);
       hipLaunchKernelGGL(k_tridiag_team, dim3(team_size(n_top), n_large - n_team0), dim3(512), 0, sm, t,
                          d_order + n_team0, dA, d_td, d_te, dZ, d_active, d_st);
+      hipLaunchKernelGGL(k_tridiag_solo, dim3(n_large - n_team0), dim3(512), 0, sm, t, d_order + n_team0, dA, d_td,
+                         d_te, dZ, d_active);
     }
-    auto blocked = [&](auto* kernel, int first, int end, double* zteam) {
-      if (end > first)
-        hipLaunchKernelGGL(kernel, dim3(end - first), dim3(512), 0, sm, t, d_order + first, dA, d_td, d_te, dT,
-                           d_active, d_xl, zteam);
-    };
-    blocked(k_tridiag_blocked<true>, 0, n_team0, nullptr);
-    blocked(k_tridiag_blocked<true>, n_team0, n_xl, dZ);
-    blocked(k_tridiag_blocked<false>, n_xl, n_large, dZ);
+    if (n_team0 > 0)
+      hipLaunchKernelGGL(k_tridiag_blocked, dim3(n_team0), dim3(512), 0, sm, t, d_order, dA, d_td, d_te, dT, d_active,
+                         d_xl);
     if (n_team0 < B)
       hipLaunchKernelGGL(k_tridiag, dim3(B - n_team0), dim3(512), 0, sm, t, d_order + n_team0, dA, d_td, d_te, d_wyT,
                          dZ, d_active);

@@ -346,7 +346,7 @@ struct ClusterOut {
 };
 constexpr int kInverseIterations = 3;
 
-// Householder reduction for n > 256 in panels of kTriPanel reflectors, the
+// Householder reduction for n > kTeamN in panels of kTriPanel reflectors, the
 // arrangement of LAPACK's dsytrd/dlatrd.  Within a panel the trailing matrix
 // is not written: after reflectors 0 .. j-1 of the panel it equals
 //   A_j = A_0 - V W^T - W V^T,
@@ -357,22 +357,20 @@ constexpr int kInverseIterations = 3;
 // corrected by V and W, the lower triangle of A_0's trailing block once (the
 // symmetric product), and V and W twice; the trailing lower triangle is
 // rewritten once per panel, on the matrix cores.  Only the lower triangle of
-// A is read or written.  512 threads, n <= kMaxAO.
+// A is read or written.  512 threads.
 //
 // Every phase issues all of its global loads before the first use (fully
 // unrolled, out-of-range lanes clamped to valid addresses and their values
 // selected away), so that a wavefront waits once per column pair rather than
 // once per 64-row slot.
 constexpr int kTriPanel = 16;
-// LDS: `part` >= 8 kMaxAO doubles, `aux` >= kMaxAO + 4 kTriPanel doubles
-constexpr int kTriAux = kMaxAO + 4 * kTriPanel;
 
 // One unit of the symmetric product p = A v over an m x m trailing block
 // (column-major at `blk`, leading dimension n, lower triangle): the columns
 // c = cu .. cu + 2 kTriPairs - 1 (cu a multiple of 2 kTriPairs, so that all
-// start in row slot t0 = cu / 64), rows 64 (t0 + u) + lane, u < NS.  Column
+// start in row slot cu / 64), rows 64 (tb + u) + lane, u < NS.  Column
 // c adds a_rc x_c to the row partials (registers, flushed to the wavefront's
-// LDS row `prow` at the end) and its dot with x over the rows below the
+// row `prow` at the end) and its dot with x over the rows below the
 // diagonal, plus the diagonal term, to pcol[c].  The next column pair is
 // fetched while the current one is consumed.
 //
@@ -439,17 +437,16 @@ __device__ __forceinline__ void symv_consume(int c, int m, int r0, const double*
   }
 }
 
-// CH: the unit's rows start at slot tb instead of cu / 64 (row chunks of a
-// trailing block above 16 slots); chunks after the first add their column
-// dots to pcol, and their rows lie below every column of the unit.
-template <int NS, bool CH = false>
+// tb: the first row slot of the unit's chunk, cu / 64 or more (row chunks of at
+// most 16 slots); chunks after the first add their column dots to pcol, and
+// their rows lie below every column of the unit.
+template <int NS>
 __device__ __forceinline__ void symv_unit(const double* __restrict__ blk, int64_t n, int m, int cu, int tb,
                                           const double* __restrict__ x, double* __restrict__ prow,
                                           double* __restrict__ pcol) {
   const int lane = threadIdx.x & 63;
-  const int t0 = CH ? tb : cu >> 6;
-  const bool add = CH && tb != (cu >> 6);
-  const int r0 = 64 * t0 + lane;  // this lane's row in slot 0
+  const bool add = tb != (cu >> 6);
+  const int r0 = 64 * tb + lane;  // this lane's row in slot 0
   unsigned boff[NS];              // byte offsets of this lane's rows in a column
   double xr[NS], acc[NS];
 #pragma unroll
@@ -479,7 +476,7 @@ __device__ __forceinline__ void symv_unit(const double* __restrict__ blk, int64_
 template <int NS>
 __device__ __forceinline__ void dots_pair(const double* __restrict__ col0, const double* __restrict__ col1,
                                           int m, const double* __restrict__ x, double* __restrict__ out0,
-                                          double* __restrict__ out1, bool add = false) {
+                                          double* __restrict__ out1, bool add) {
   const int lane = threadIdx.x & 63;
   double a0[NS], a1[NS];
 #pragma unroll
@@ -523,12 +520,10 @@ __device__ __forceinline__ void dots_pair(const double* __restrict__ col0, const
     case 16: { constexpr int NS = 16; CALL; } break;                                 \
     default: break;                                                                  \
   }
-static_assert(kMaxAO == 16 * 64, "the slot switch covers up to 16 slots of 64 rows");
 
-// BIG (n > kMaxAO): v, pq, part and aux are global, with a row stride of
-// `part` of n rounded up to 64; the symmetric product and the W^T v, V^T v
-// dots run over row chunks of at most 16 slots.
-template <bool BIG = false>
+// v, pq, part and aux are global, with a row stride of `part` of n rounded up to
+// 64; the symmetric product and the W^T v, V^T v dots run over row chunks of at
+// most 16 slots.
 __device__ __forceinline__ void tridiag_blocked(double* __restrict__ A, double* __restrict__ W, int n,
                                                 double* d, double* e, double* v, double* pq,
                                                 double* part, double* aux, double* red, double* bc) {
@@ -536,7 +531,7 @@ __device__ __forceinline__ void tridiag_blocked(double* __restrict__ A, double* 
   // the wavefront index is uniform: keep it (and the column indices derived
   // from it) in scalar registers
   const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), nw = nt >> 6;
-  const int ldp = BIG ? (n + 63) & ~63 : kMaxAO;
+  const int ldp = (n + 63) & ~63;
   double* pcol = aux;                   // [ldp] column dots of the symmetric product
   double* rowk = aux + ldp;             // [2 kTriPanel] row k of V, of W
   double* yv = rowk + 2 * kTriPanel;    // [2 kTriPanel] W^T v, V^T v
@@ -622,23 +617,14 @@ __device__ __forceinline__ void tridiag_blocked(double* __restrict__ A, double* 
         if (u >= nunits) continue;
         const int cu = 2 * kTriPairs * u;
         const double* blk = A + at(b, b);
-        if constexpr (BIG) {
-          for (int tb = cu >> 6; tb < tend; tb += 16)
-            XTB_SLOT_SWITCH(min(16, tend - tb), (symv_unit<NS, true>(blk, n, m, cu, tb, v, prow, pcol)))
-        } else {
-          XTB_SLOT_SWITCH(tend - (cu >> 6), (symv_unit<NS>(blk, n, m, cu, 0, v, prow, pcol)))
-        }
+        for (int tb = cu >> 6; tb < tend; tb += 16)
+          XTB_SLOT_SWITCH(min(16, tend - tb), (symv_unit<NS>(blk, n, m, cu, tb, v, prow, pcol)))
       }
       for (int q = (wv + nw - nunits % nw) % nw; q < j; q += nw) {
-        if constexpr (BIG) {
-          for (int tb = 0; tb < tend; tb += 16)
-            XTB_SLOT_SWITCH(min(16, tend - tb),
-                            (dots_pair<NS>(W + at(b + 64 * tb, k0 + q), A + at(b + 64 * tb, k0 + q),
-                                           m - 64 * tb, v + 64 * tb, yv + q, yv + kTriPanel + q, tb > 0)))
-        } else {
-          XTB_SLOT_SWITCH(tend, (dots_pair<NS>(W + at(b, k0 + q), A + at(b, k0 + q), m, v, yv + q,
-                                                yv + kTriPanel + q)))
-        }
+        for (int tb = 0; tb < tend; tb += 16)
+          XTB_SLOT_SWITCH(min(16, tend - tb),
+                          (dots_pair<NS>(W + at(b + 64 * tb, k0 + q), A + at(b + 64 * tb, k0 + q),
+                                         m - 64 * tb, v + 64 * tb, yv + q, yv + kTriPanel + q, tb > 0)))
       }
       __syncthreads();
       // p_j = A_j v = p - V (W^T v) - W (V^T v);  K = v^T p_j
@@ -1173,8 +1159,8 @@ __device__ __forceinline__ void tridiag_full(double* A, int64_t ld, int n, doubl
 // Waiting is safe: no member writes anything before all G have met at the gate,
 // so from then on every partner is resident and runs.  Members that do not all
 // arrive within kTeamWaitTicks (the chip is held by something else) close the
-// gate together and leave; the system then takes k_tridiag_blocked.  The spins
-// are bounded too; one that runs out fails the system (status 8).
+// gate together and leave; k_tridiag_solo then does the same arithmetic.  The
+// spins are bounded too; one that runs out fails the system (status 8).
 //
 // Bound: the latency of a step, 4.5 us at 482 AOs (16 members) and 5.5 us at
 // 1142 (36), most of it the exchange through memory.  Measured against one
@@ -1195,6 +1181,81 @@ __host__ __device__ constexpr int team_size(int n) { return (n + 8 * kTeamRows -
 // eigenvectors are written): p ring, row ring, then the gate and done words.
 __device__ __forceinline__ unsigned* team_words(double* Z, int n) {
   return reinterpret_cast<unsigned*>(Z + 2 * kTeamRing * (int64_t)n);
+}
+
+// One step's arithmetic outside the product, the same instructions for a team and
+// for k_tridiag_solo (contraction off: each kernel would otherwise fuse as its
+// surroundings suggest), so that both leave the same bits.
+struct TeamStep {
+  double v0, alpha, inv, beta;  // noref (already reduced): inv = beta = 0
+  bool noref;
+};
+__device__ __forceinline__ TeamStep team_step(const double* redn, double x0) {
+#pragma clang fp contract(off)
+  TeamStep z;
+  const double tail = ((redn[0] + redn[1]) + (redn[2] + redn[3])) + ((redn[4] + redn[5]) + (redn[6] + redn[7]));
+  const double ss = fma(x0, x0, tail);
+  z.noref = tail == 0.0 || ss < kTinyNorm;
+  const double xn = ss * rsqrt_refined(fmax(ss, kTinyNorm));
+  z.alpha = x0 >= 0.0 ? -xn : xn;
+  z.v0 = x0 - z.alpha;
+  z.inv = z.noref ? 0.0 : rsqrt_refined(fmax(fma(z.v0, z.v0, tail), kTinyNorm));
+  z.beta = 2.0 * (z.inv * z.inv);
+  return z;
+}
+// Column 0: this thread's entries xo, the vectors and the norm's partial sums.
+__device__ __forceinline__ void team_first(const double* A, int off, bool keeps_d, double* d, double (&xo)[kTeamOwn],
+                                           double* x, double* u, double* r, double* redn) {
+  const int tid = threadIdx.x;
+  double part = 0.0;
+#pragma unroll
+  for (int q = 0; q < kTeamOwn; ++q) {
+    const int L = tid + 512 * q;
+    double v = 0.0;
+    if (L >= off && L < kTeamN) v = A[L - off];
+    if (L == off && keeps_d) d[0] = v;
+    xo[q] = L > off ? v : 0.0;
+    if (L > off + 1) part = fma(xo[q], xo[q], part);
+    if (L < kTeamN) {
+      x[L] = xo[q];
+      u[L] = 0.0;
+      r[L] = 0.0;
+    }
+  }
+  part = wave_sum(part);
+  if ((tid & 63) == 0) redn[tid >> 6] = part;
+}
+// r of step K and the next column from this thread's entries of p and row k + 1;
+// x: the vector of this step (its entry K + 1 becomes v0), xn: the next one.
+// Returns the next column's diagonal on the thread that holds it.
+__device__ __forceinline__ void team_vectors(const TeamStep& z, int K, const double* redk, double p1,
+                                             const double (&po)[kTeamOwn], const double (&ro)[kTeamOwn],
+                                             double (&xo)[kTeamOwn], double* x, double* xn, double* rb, double* redn,
+                                             double* dnext) {
+#pragma clang fp contract(off)
+  const int tid = threadIdx.x;
+  const double hK = 0.5 * z.beta *
+                    (((redk[0] + redk[1]) + (redk[2] + redk[3])) + ((redk[4] + redk[5]) + (redk[6] + redk[7])));
+  const double r1 = z.beta * fma(-hK, z.v0, p1);
+  double part = 0.0;
+#pragma unroll
+  for (int q = 0; q < kTeamOwn; ++q) {
+    const int L = tid + 512 * q;
+    const double r = z.beta * fma(-hK, xo[q], po[q]);
+    const double y = fma(-z.v0, r, fma(-r1, xo[q], ro[q]));
+    if (L == K + 1) {
+      if (dnext) *dnext = y;
+      x[L] = z.v0;
+    }
+    xo[q] = L > K + 1 ? y : 0.0;
+    if (L > K + 2) part = fma(xo[q], xo[q], part);
+    if (L < kTeamN) {
+      rb[L] = r;
+      xn[L] = xo[q];
+    }
+  }
+  part = wave_sum(part);
+  if ((tid & 63) == 0) redn[tid >> 6] = part;
 }
 
 __global__ __launch_bounds__(256) void k_team_init(Topo t, const int* order, const unsigned char* active,
@@ -1257,25 +1318,7 @@ __global__ __launch_bounds__(512) void k_tridiag_team(Topo t, const int* order, 
     __builtin_amdgcn_sched_barrier(0);
   }
   double xo[kTeamOwn];  // this thread's entries L = tid + 512 q of the current column
-  {
-    double part = 0.0;
-#pragma unroll
-    for (int q = 0; q < kTeamOwn; ++q) {
-      const int L = tid + 512 * q;
-      double x = 0.0;
-      if (L >= off && L < kTeamN) x = A[L - off];
-      if (L == off && g == 0) d[0] = x;
-      xo[q] = L > off ? x : 0.0;
-      if (L > off + 1) part = fma(xo[q], xo[q], part);
-      if (L < kTeamN) {
-        xb[0][L] = xo[q];
-        xb[1][L] = 0.0;
-        rb[L] = 0.0;
-      }
-    }
-    part = wave_sum(part);
-    if (lane == 0) redn[w] = part;
-  }
+  team_first(A, off, g == 0, d, xo, xb[0], xb[1], rb, redn);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   // the gate
@@ -1300,22 +1343,13 @@ __global__ __launch_bounds__(512) void k_tridiag_team(Topo t, const int* order, 
   __syncthreads();
   if (sh_bad) return;
   const int kend = n - kFullN;  // columns reduced here
-  double v0 = 0.0;
   int cur = 0;
   int k = 0;
   for (;; ++k) {
     const int K = k + off, slot = k & (kTeamRing - 1);
     double* pk = ring_p + (int64_t)slot * n;
     double* rk = ring_r + (int64_t)slot * n;
-    const double tail = ((redn[0] + redn[1]) + (redn[2] + redn[3])) + ((redn[4] + redn[5]) + (redn[6] + redn[7]));
-    const double x0 = xb[cur][K + 1];
-    const double ss = fma(x0, x0, tail);
-    const bool noref = tail == 0.0 || ss < kTinyNorm;  // already reduced: inv = beta = 0
-    const double xn = ss * rsqrt_refined(fmax(ss, kTinyNorm));
-    const double alpha = x0 >= 0.0 ? -xn : xn;
-    v0 = x0 - alpha;
-    const double inv = noref ? 0.0 : rsqrt_refined(fmax(fma(v0, v0, tail), kTinyNorm));
-    const double beta = 2.0 * (inv * inv);
+    const TeamStep z = team_step(redn, xb[cur][K + 1]);
     // one sweep over the registers: the pending update of step k - 1 (zero in
     // step 0) and p = A u.  Finished rows ride along: their entries of u and r
     // keep them finite, and the exchange hides them.
@@ -1331,7 +1365,7 @@ __global__ __launch_bounds__(512) void k_tridiag_team(Topo t, const int* order, 
       constexpr int T = decltype(CT)::value;
       if (64 * T + 63 >= K) {  // a column tile with a live column
         const int L = 64 * T + lane;
-        const double x = L == K + 1 ? v0 : xb[cur][L], u = xb[cur ^ 1][L], r = rb[L];
+        const double x = L == K + 1 ? z.v0 : xb[cur][L], u = xb[cur ^ 1][L], r = rb[L];
 #pragma unroll
         for (int q = 0; q < kTeamRows; ++q) {
           a[q][T] = fma(-ur[q], r, fma(-rr[q], u, a[q][T]));
@@ -1367,9 +1401,9 @@ __global__ __launch_bounds__(512) void k_tridiag_team(Topo t, const int* order, 
 #pragma unroll
       for (int q = 0; q < kTeamOwn; ++q) {
         const int L = tid + 512 * q;
-        if (L > K && L < kTeamN) A[(L - off) + (int64_t)k * n] = (L == K + 1 ? v0 : xo[q]) * inv;
+        if (L > K && L < kTeamN) A[(L - off) + (int64_t)k * n] = (L == K + 1 ? z.v0 : xo[q]) * z.inv;
       }
-      if (tid == 0) e[k] = noref ? x0 : alpha;
+      if (tid == 0) e[k] = z.noref ? xb[cur][K + 1] : z.alpha;
     }
     // everybody's p and the row
     double po[kTeamOwn], ro[kTeamOwn];
@@ -1407,7 +1441,7 @@ __global__ __launch_bounds__(512) void k_tridiag_team(Topo t, const int* order, 
         po[q] = __longlong_as_double((long long)bp[q]);  // 0 where L <= K
         ro[q] = __longlong_as_double((long long)br[q]);
         if (L == K + 1) {
-          xo[q] = v0;
+          xo[q] = z.v0;
           sh_p = po[q];
         }
         kp = fma(xo[q], po[q], kp);
@@ -1420,30 +1454,8 @@ __global__ __launch_bounds__(512) void k_tridiag_team(Topo t, const int* order, 
       if (tid == 0) st[s].status = 8;
       return;
     }
-    {
-      const double hK = 0.5 * beta *
-                        (((redk[0] + redk[1]) + (redk[2] + redk[3])) + ((redk[4] + redk[5]) + (redk[6] + redk[7])));
-      const double r1 = beta * fma(-hK, v0, sh_p);
-      double part = 0.0;
-#pragma unroll
-      for (int q = 0; q < kTeamOwn; ++q) {
-        const int L = tid + 512 * q;
-        const double r = beta * fma(-hK, xo[q], po[q]);
-        const double x = fma(-v0, r, fma(-r1, xo[q], ro[q]));
-        if (L == K + 1) {
-          if (g == 0 && k + 1 < kend) d[k + 1] = x;
-          xb[cur][L] = v0;
-        }
-        xo[q] = L > K + 1 ? x : 0.0;
-        if (L > K + 2) part = fma(xo[q], xo[q], part);
-        if (L < kTeamN) {
-          rb[L] = r;
-          xb[cur ^ 1][L] = xo[q];
-        }
-      }
-      part = wave_sum(part);
-      if (lane == 0) redn[w] = part;
-    }
+    team_vectors(z, K, redk, sh_p, po, ro, xo, xb[cur], xb[cur ^ 1], rb, redn,
+                 g == 0 && k + 1 < kend ? d + k + 1 : nullptr);
     // every member has published step k, so it has read step k - 1: empty that slot
     if (k > 0) {
       double* pl = ring_p + (int64_t)((k - 1) & (kTeamRing - 1)) * n;
@@ -1472,6 +1484,94 @@ __global__ __launch_bounds__(512) void k_tridiag_team(Topo t, const int* order, 
       });
   }
   if (g == 0 && tid == 0) gate[1] = 1u;  // done
+}
+
+// The team's reduction by one workgroup, for systems whose team left at the gate:
+// the rows stay in A, a wavefront per row, and every sum is formed from the same
+// terms in the same order, so that the results do not depend on whether a team
+// could assemble.  Bound: the sweep over the trailing block (16 n^2 bytes a step
+// through one CU): 205 ms at 1280 AOs (240 with four tiles in flight instead of
+// ten), where the team takes 6.6 ms.
+__global__ __launch_bounds__(512) void k_tridiag_solo(Topo t, const int* order, double* Aall, double* dall,
+                                                      double* eall, double* Zall, const unsigned char* active) {
+  const int s = order[blockIdx.x];
+  if (active && !active[s]) return;
+  const int n = t.ao_off[s + 1] - t.ao_off[s];
+  unsigned* words = team_words(Zall + t.mat_off[s], n);
+  if (words[1] != 0u) return;  // reduced by its team
+  double* A = Aall + t.mat_off[s];
+  double* d = dall + t.ao_off[s];
+  double* e = eall + t.ao_off[s];
+  __shared__ double xb[2][kTeamN];
+  __shared__ double rb[kTeamN];
+  __shared__ double pb[kTeamN];
+  __shared__ double redn[8], redk[8];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int off = kTeamN - n;
+  double xo[kTeamOwn];
+  team_first(A, off, true, d, xo, xb[0], xb[1], rb, redn);
+  __syncthreads();
+  const int kend = n - kFullN;
+  int cur = 0;
+  for (int k = 0;; ++k) {
+    const int K = k + off;
+    const TeamStep z = team_step(redn, xb[cur][K + 1]);
+    // the pending update of step k - 1 and p = A u: rows past k (all that is left
+    // of the trailing block after the last column), columns from K's tile on
+    const int first = k < kend ? k + 1 : k, T0 = K >> 6;
+    for (int i = first + ((w - first) & 7); i < n; i += 8) {
+      const double ur = xb[cur ^ 1][i + off], rr = rb[i + off];
+      double* row = A + (int64_t)i * n;
+      double p[1] = {0.0};
+      auto sweep = [&](auto U, int T) __attribute__((always_inline)) {
+        constexpr int NU = decltype(U)::value;
+        double a[NU];
+#pragma unroll
+        for (int v = 0; v < NU; ++v) {
+          const int c = 64 * (T + v) + lane - off;
+          a[v] = c >= 0 ? row[c] : 0.0;
+        }
+#pragma unroll
+        for (int v = 0; v < NU; ++v) {
+          const int L = 64 * (T + v) + lane;
+          const double x = L == K + 1 ? z.v0 : xb[cur][L], u = xb[cur ^ 1][L], r = rb[L];
+          a[v] = fma(-ur, r, fma(-rr, u, a[v]));
+          p[0] = fma(a[v], x, p[0]);
+          if (L >= off) row[L - off] = a[v];
+        }
+      };
+      int T = T0;
+      for (; T + 10 <= kTeamTiles; T += 10) sweep(std::integral_constant<int, 10>{}, T);
+      for (; T + 4 <= kTeamTiles; T += 4) sweep(std::integral_constant<int, 4>{}, T);
+      for (; T < kTeamTiles; ++T) sweep(std::integral_constant<int, 1>{}, T);
+      double r = row16_sums<1>(p, lane & 15);
+      r += __shfl_xor(r, 16, 64);
+      r += __shfl_xor(r, 32, 64);
+      if (lane == 0) pb[i + off] = r;
+    }
+    if (k == kend) break;
+    __syncthreads();
+    double po[kTeamOwn], ro[kTeamOwn], kp = 0.0;
+#pragma unroll
+    for (int q = 0; q < kTeamOwn; ++q) {
+      const int L = tid + 512 * q;
+      const bool live = L > K && L < kTeamN;
+      po[q] = live ? pb[L] : 0.0;
+      ro[q] = live ? A[(int64_t)(k + 1) * n + (L - off)] : 0.0;
+      if (live) A[(L - off) + (int64_t)k * n] = (L == K + 1 ? z.v0 : xo[q]) * z.inv;
+      if (L == K + 1) xo[q] = z.v0;
+      kp = fma(xo[q], po[q], kp);
+    }
+    if (tid == 0) e[k] = z.noref ? xb[cur][K + 1] : z.alpha;
+    kp = wave_sum(kp);
+    if (lane == 0) redk[w] = kp;
+    __syncthreads();
+    team_vectors(z, K, redk, pb[K + 1], po, ro, xo, xb[cur], xb[cur ^ 1], rb, redn,
+                 k + 1 < kend ? d + k + 1 : nullptr);
+    __syncthreads();
+    cur ^= 1;
+  }
+  if (tid == 0) words[1] = 1u;
 }
 
 // The back-transformation applies the reflectors in compact WY blocks of
@@ -1533,7 +1633,7 @@ __device__ __forceinline__ void wy_factor(const double* A, int n, int ch, double
 // n <= 256, 512 threads per system (two waves per SIMD, 256 VGPRs per thread):
 // the columns before the last kFullN from the triangle in registers, the rest
 // with both triangles.  n > 256: the last kFullN columns of the systems that
-// k_tridiag_team has reduced to them.
+// k_tridiag_team or k_tridiag_solo has reduced to them.
 __global__ __launch_bounds__(512) void k_tridiag(Topo t, const int* order, double* Aall, double* dall,
                                                  double* eall, double* Tall, double* Zall,
                                                  const unsigned char* active) {
@@ -1566,37 +1666,25 @@ __global__ __launch_bounds__(512) void k_tridiag(Topo t, const int* order, doubl
     wy_factor(A, n, ch, Tall + wy_offset(t, s), rowpart + 256 * wv);
 }
 
-// n > 256: the blocked reduction, one 512-thread block per system (the host
-// launches the large systems only; with Zteam the ones whose team left at the
-// gate); W is per-system n x n scratch.  BIG: the
-// systems above kMaxAO AOs, with the work vectors in their global slice of `big`.
-template <bool BIG>
+// n > kTeamN: the blocked reduction, one 512-thread block per system; W is
+// per-system n x n scratch, the work vectors sit in the system's slice of `big`.
 __global__ __launch_bounds__(512) void k_tridiag_blocked(Topo t, const int* order, double* Aall,
                                                          double* dall, double* eall, double* Wall,
-                                                         const unsigned char* active, double* big,
-                                                         double* Zteam) {
+                                                         const unsigned char* active, double* big) {
   const int s = order[blockIdx.x];
   if (active && !active[s]) return;
   const int n = t.ao_off[s + 1] - t.ao_off[s];
-  if (Zteam && team_words(Zteam + t.mat_off[s], n)[1] != 0u) return;  // reduced by its team
-  __shared__ double v_l[BIG ? 1 : kMaxAO];
-  __shared__ double pq_l[BIG ? 1 : kMaxAO];
-  __shared__ double part_l[BIG ? 1 : 8 * kMaxAO];
-  __shared__ double aux_l[BIG ? 1 : kTriAux];
   static_assert(kTriPanel % 4 == 0, "panel in K steps of 4");
   __shared__ double red[16];
   __shared__ double bc[2];
-  double *v = v_l, *pq = pq_l, *part = part_l, *aux = aux_l;
-  if constexpr (BIG) {
-    // 2 n + 8 ldp + ldp + 4 kTriPanel <= kBigPerAO n + kBigPerSys doubles
-    const int ldp = (n + 63) & ~63;
-    v = big + big_offset(t, s);
-    pq = v + n;
-    part = pq + n;
-    aux = part + 8 * ldp;
-  }
-  tridiag_blocked<BIG>(Aall + t.mat_off[s], Wall + t.mat_off[s], n, dall + t.ao_off[s],
-                       eall + t.ao_off[s], v, pq, part, aux, red, bc);
+  // 2 n + 8 ldp + ldp + 4 kTriPanel <= kBigPerAO n + kBigPerSys doubles
+  const int ldp = (n + 63) & ~63;
+  double* v = big + big_offset(t, s);
+  double* pq = v + n;
+  double* part = pq + n;
+  double* aux = part + 8 * ldp;
+  tridiag_blocked(Aall + t.mat_off[s], Wall + t.mat_off[s], n, dall + t.ao_off[s], eall + t.ao_off[s], v, pq, part,
+                  aux, red, bc);
 }
 
 // Overlap Cholesky S = L L^T (L column-major into `L`) and X = L^{-T} (row-major,
