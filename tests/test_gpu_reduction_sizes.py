@@ -1,11 +1,12 @@
 """The tridiagonal reduction and the back-transformation at the edges of their tiles.
 
-Stacks of H2 molecules (one AO per atom, a helium atom for odd counts) give
+Stacks of H2 molecules (one AO per atom, a hydrogen atom for odd counts) give
 systems of every AO count: around the 16-column phases and 32-row tiles of the
 register reduction, the 192-column switch between its two forms, the
 16-reflector blocks and 16-row tiles of the back-transformation, and the
 256-AO limit of the register kernels.  Energies, forces and charges against the
-oracle at the package's bars.
+oracle.  Molecules of 640 to 1280 AOs: the edges of the teams' classes and the
+switches at 1024.
 """
 import numpy as np
 import pytest
@@ -15,22 +16,39 @@ from xtbloom_amd import interface, library, workloads
 
 pytestmark = pytest.mark.gpu
 
-E_TOL, F_TOL, Q_TOL = 1e-7, 1e-6, 1e-6
+# Same iterations on both sides, so only rounding separates them: an eigenvector
+# carries n eps |H| / gap <= 1280 * 2.2e-16 * 10 / 0.1 = 3e-11 of its neighbours, which
+# enters the density to first order and the forces with derivatives of order 1; the
+# SCC's amplification is below 10.  1e-9 is above that and two orders below an error
+# of the package's bars.
+E_TOL, F_TOL, Q_TOL = 1e-9, 1e-9, 1e-9
 
 
 def stack(n, rng):
-    """n atoms with one AO each: H2 molecules on a grid, one He when n is odd."""
-    z, xyz = [], []
+    """n hydrogen atoms, one AO each: H2 molecules on a grid and one atom when n is odd."""
+    xyz = []
     for m in range(n // 2):
         c = 5.0 * np.array([m % 5, (m // 5) % 5, m // 25]) + rng.normal(0.0, 0.1, 3)
         u = rng.normal(size=3)
         u *= 0.5 * (1.40 + rng.uniform(-0.05, 0.05)) / np.linalg.norm(u)
-        z += [1, 1]
         xyz += [c - u, c + u]
     if n % 2:
-        z.append(2)
         xyz.append(np.array([-5.0, -5.0, 0.0]))
-    return dict(Z=np.array(z, np.int32), xyz=np.array(xyz), charge=0.0, uhf=0)
+    return dict(Z=np.ones(n, np.int32), xyz=np.array(xyz), charge=0.0, uhf=n % 2)
+
+
+def molecule(n, rng):
+    """n >= 19 AOs, closed shell: the largest alkane (odd n: alkyl amine) that fits and
+    H2 molecules 8 bohr and more beside it."""
+    k = (n - 7) // 6 if n % 2 else (n - 2) // 6
+    s = workloads.alkane(k, rng, substituent="NH2" if n % 2 else None)
+    left = n - (6 * k + (7 if n % 2 else 2))
+    if left == 0:
+        return s
+    rest = stack(left, rng)["xyz"]
+    beside = rest + s["xyz"].min(axis=0) - rest.max(axis=0) - np.array([0.0, 8.0, 0.0])
+    return dict(s, Z=np.concatenate([s["Z"], np.ones(left, np.int32)]).astype(np.int32),
+                xyz=np.concatenate([s["xyz"], beside]))
 
 
 @pytest.mark.parametrize("sizes", [
@@ -47,6 +65,12 @@ def test_sizes_against_the_oracle(sizes):
     check(sizes)
 
 
+def test_team_classes_against_the_oracle():
+    """The first and last size of each class of teams; 1025 and above also switch the
+    conditioning estimate and the back-transformation."""
+    check([640, 641, 832, 833, 1024, 1025, 1280], molecule, threads=8)
+
+
 def test_teams_that_leave_at_the_gate(monkeypatch):
     """A closed gate: every team leaves before it writes anything and one workgroup
     per system reduces the matrices instead."""
@@ -54,9 +78,10 @@ def test_teams_that_leave_at_the_gate(monkeypatch):
     check([258, 289, 353])
 
 
-def check(sizes):
+def check(sizes, make=stack, threads=4):
     rng = np.random.default_rng(sizes[0])
-    b = workloads.from_systems([stack(n, rng) for n in sizes])
+    b = workloads.from_systems([make(n, rng) for n in sizes])
+    assert [O.basis_counts(b.system(i)["Z"])[1] for i in range(len(sizes))] == list(sizes)
     ctx = interface.Context("hip", 0)
     try:
         print("case reduction sizes", sizes, flush=True)
@@ -65,8 +90,11 @@ def check(sizes):
     finally:
         ctx.close()
     ref = O.batch(b.atom_offsets, b.atomic_numbers, b.positions, b.molecular_charges,
-                  b.unpaired_electrons, threads=4)
+                  b.unpaired_electrons, threads=threads)
     assert np.all(out.per_system_status == 0) and np.all(ref["status"] == 0)
+    print("|dE| %.1e |dF| %.1e |dq| %.1e" % (np.abs(out.energies - ref["energies"]).max(),
+                                             np.abs(out.forces + ref["gradient"]).max(),
+                                             np.abs(out.charges - ref["charges"]).max()), flush=True)
     assert np.abs(out.scc_iterations - ref["iterations"]).max() <= 1
     assert np.abs(out.energies - ref["energies"]).max() <= E_TOL
     assert np.abs(out.forces + ref["gradient"]).max() <= F_TOL
@@ -114,7 +142,7 @@ def test_closed_gate_changes_no_bit(monkeypatch):
     sum as the team does; that it ran shows in the time of the reduction (a team of 40
     workgroups against one)."""
     rng = np.random.default_rng(1280)
-    b = workloads.from_systems([workloads.alkane(213, rng), workloads.alkane(50, rng), stack(257, rng)])
+    b = workloads.from_systems([workloads.alkane(k, rng) for k in (213, 150, 108, 50)] + [stack(257, rng)])
     ctx = interface.Context("hip", 0)
 
     def run():
@@ -123,7 +151,7 @@ def test_closed_gate_changes_no_bit(monkeypatch):
                                         kernel_stats=["tridiag"])
 
     try:
-        print("case gate: 1280, 302 and 257 AOs by teams", flush=True)
+        print("case gate: 1280, 902, 650, 302 and 257 AOs by teams", flush=True)
         team = run()
         monkeypatch.setenv("XTBLOOM_AMD_TEAMS", "0")
         print("case gate: the same, gates closed", flush=True)
