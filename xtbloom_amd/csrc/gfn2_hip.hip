@@ -644,10 +644,9 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
   // Systems reduced by teams: [n_team0, n_large) of the size order, those of 257
   // to kTeamN AOs.  The system's size alone decides, so that its result depends
   // neither on the batch around it nor on the lanes.  Reduction of eleven rounds
-  // by teams against one workgroup per system: 8.8 and 33.1 ms for 32 systems of
-  // 260 AOs, 61.6 and 113 ms for 64 of 482, 178 and 457 ms for 32 of 902.  Only
-  // where the single workgroups fill the chip are teams slower (239 and 142 ms
-  // for 256 systems of 482).
+  // by teams against one workgroup per system: 11.4 and 44.5 ms for 64 systems of
+  // 302 AOs, 108 and 142 ms for 256 of 482, 316 and 319 ms for 256 of 650, 437 and
+  // 594 ms for 128 of 902, 191 and 1318 ms for 16 of 1142.
   int n_team0 = 0;
   while (n_team0 < n_large && T.ao_off[T.order[n_team0] + 1] - T.ao_off[T.order[n_team0]] > kTeamN) ++n_team0;
   // WY blocks of the largest system, in groups of eight (k_wy_factors)

@@ -1137,8 +1137,8 @@ __device__ __forceinline__ void tridiag_full(double* A, int64_t ld, int n, doubl
 // AOs, down to its last kFullN columns (k_tridiag finishes those).
 //
 // The whole matrix, both triangles, sits in the team's registers: member g of G
-// holds the rows i = g (mod G), its wavefront w the rows (8 s + w) G + g, s <
-// kTeamRows, lane l the columns l + 64 t.  A step k on every member:
+// holds the rows i = g (mod G), its wavefront w the rows (8 q + w) G + g, q <
+// team_rows(n), lane l the columns l + 64 t.  A step k on every member:
 //   pass     A -= u r^T + r u^T of step k - 1 and p = A u_k on the member's
 //            rows, one sweep over the registers (u, r from LDS); row sums stay
 //            inside a wavefront;
@@ -1167,15 +1167,32 @@ __device__ __forceinline__ void tridiag_full(double* A, int64_t ld, int n, doubl
 // workgroup per system with panels of 16 reflectors (k_tridiag_blocked): 9.0 ->
 // 1.3 + 0.4 ms a round for 14 systems of 258-482 AOs, 111 -> 5.3 ms at 1142.
 // Members on one XCD (every eighth block) were 10 % slower than neighbours.
-constexpr int kTeamRows = 4, kTeamTiles = 20, kTeamN = 64 * kTeamTiles;
+constexpr int kTeamN = 1280;
 constexpr int kTeamRing = 8;
-constexpr int kTeamOwn = (kTeamN + 511) / 512;  // vector entries per thread
+constexpr int team_own(int tiles) { return (64 * tiles + 511) / 512; }  // vector entries per thread
 constexpr unsigned long long kTeamEmpty = 0xfff7a5a5c3c3e1e1ull;
 constexpr long long kTeamWaitTicks = 20000000;  // 100 MHz counter: 0.2 s
 constexpr int kTeamSpins = 1 << 22;
 constexpr unsigned kTeamClosed = 1u << 30;
-// team size: at most 8 kTeamRows rows per member
-__host__ __device__ constexpr int team_size(int n) { return (n + 8 * kTeamRows - 1) / (8 * kTeamRows); }
+// Rows of a wavefront: as many as about 80 doubles a lane hold, tiles of 64 columns
+// for the largest n of the class.  Smaller teams leave CUs to other systems: with
+// four rows for every n the teams of 256 systems of 482 AOs took 239 ms of a call
+// (eleven rounds) and with eight 108, where one workgroup per system took 142; 256
+// of 650 AOs 515 and 316 (six rows), 319 with one workgroup per system.
+__host__ __device__ constexpr int team_rows(int n) { return n <= 640 ? 8 : n <= 832 ? 6 : n <= 1024 ? 5 : 4; }
+__host__ __device__ constexpr int team_size(int n) { return (n + 8 * team_rows(n) - 1) / (8 * team_rows(n)); }
+// f(rows of a wavefront, column tiles) of n's class
+template <typename F>
+__device__ __forceinline__ void team_class(int n, F&& f) {
+  if (n <= 640)
+    f(std::integral_constant<int, 8>{}, std::integral_constant<int, 10>{});
+  else if (n <= 832)
+    f(std::integral_constant<int, 6>{}, std::integral_constant<int, 13>{});
+  else if (n <= 1024)
+    f(std::integral_constant<int, 5>{}, std::integral_constant<int, 16>{});
+  else
+    f(std::integral_constant<int, 4>{}, std::integral_constant<int, 20>{});
+}
 
 // A system's exchange area (in the eigenvector matrix, free until the
 // eigenvectors are written): p ring, row ring, then the gate and done words.
@@ -1204,19 +1221,21 @@ __device__ __forceinline__ TeamStep team_step(const double* redn, double x0) {
   return z;
 }
 // Column 0: this thread's entries xo, the vectors and the norm's partial sums.
-__device__ __forceinline__ void team_first(const double* A, int off, bool keeps_d, double* d, double (&xo)[kTeamOwn],
-                                           double* x, double* u, double* r, double* redn) {
+template <int TILES>
+__device__ __forceinline__ void team_first(const double* A, int off, bool keeps_d, double* d,
+                                           double (&xo)[team_own(TILES)], double* x, double* u, double* r,
+                                           double* redn) {
   const int tid = threadIdx.x;
   double part = 0.0;
 #pragma unroll
-  for (int q = 0; q < kTeamOwn; ++q) {
+  for (int q = 0; q < team_own(TILES); ++q) {
     const int L = tid + 512 * q;
     double v = 0.0;
-    if (L >= off && L < kTeamN) v = A[L - off];
+    if (L >= off && L < 64 * TILES) v = A[L - off];
     if (L == off && keeps_d) d[0] = v;
     xo[q] = L > off ? v : 0.0;
     if (L > off + 1) part = fma(xo[q], xo[q], part);
-    if (L < kTeamN) {
+    if (L < 64 * TILES) {
       x[L] = xo[q];
       u[L] = 0.0;
       r[L] = 0.0;
@@ -1228,10 +1247,11 @@ __device__ __forceinline__ void team_first(const double* A, int off, bool keeps_
 // r of step K and the next column from this thread's entries of p and row k + 1;
 // x: the vector of this step (its entry K + 1 becomes v0), xn: the next one.
 // Returns the next column's diagonal on the thread that holds it.
+template <int TILES>
 __device__ __forceinline__ void team_vectors(const TeamStep& z, int K, const double* redk, double p1,
-                                             const double (&po)[kTeamOwn], const double (&ro)[kTeamOwn],
-                                             double (&xo)[kTeamOwn], double* x, double* xn, double* rb, double* redn,
-                                             double* dnext) {
+                                             const double (&po)[team_own(TILES)], const double (&ro)[team_own(TILES)],
+                                             double (&xo)[team_own(TILES)], double* x, double* xn, double* rb,
+                                             double* redn, double* dnext) {
 #pragma clang fp contract(off)
   const int tid = threadIdx.x;
   const double hK = 0.5 * z.beta *
@@ -1239,7 +1259,7 @@ __device__ __forceinline__ void team_vectors(const TeamStep& z, int K, const dou
   const double r1 = z.beta * fma(-hK, z.v0, p1);
   double part = 0.0;
 #pragma unroll
-  for (int q = 0; q < kTeamOwn; ++q) {
+  for (int q = 0; q < team_own(TILES); ++q) {
     const int L = tid + 512 * q;
     const double r = z.beta * fma(-hK, xo[q], po[q]);
     const double y = fma(-z.v0, r, fma(-r1, xo[q], ro[q]));
@@ -1249,7 +1269,7 @@ __device__ __forceinline__ void team_vectors(const TeamStep& z, int K, const dou
     }
     xo[q] = L > K + 1 ? y : 0.0;
     if (L > K + 2) part = fma(xo[q], xo[q], part);
-    if (L < kTeamN) {
+    if (L < 64 * TILES) {
       rb[L] = r;
       xn[L] = xo[q];
     }
@@ -1282,34 +1302,25 @@ __device__ __forceinline__ unsigned long long team_peek(const double* p) {
                            __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__global__ __launch_bounds__(512) void k_tridiag_team(Topo t, const int* order, double* Aall, double* dall,
-                                                      double* eall, double* Zall, const unsigned char* active,
-                                                      SysState* st) {
-  const int s = order[blockIdx.y];
-  if (active && !active[s]) return;
-  const int n = t.ao_off[s + 1] - t.ao_off[s];
-  const int G = team_size(n), g = blockIdx.x;
-  if (g >= G) return;
-  double* A = Aall + t.mat_off[s];
-  double* d = dall + t.ao_off[s];
-  double* e = eall + t.ao_off[s];
-  double* ring_p = Zall + t.mat_off[s];
+// member g of G; xb: u of this step and of the last one, rb: r of the last step
+template <int ROWS, int TILES>
+__device__ __forceinline__ void team_member(int n, int G, int g, double* A, double* d, double* e, double* ring_p,
+                                            int* status, double (&xb)[2][kTeamN], double (&rb)[kTeamN]) {
+  constexpr int N = 64 * TILES, OWN = team_own(TILES);
   double* ring_r = ring_p + (int64_t)kTeamRing * n;
   unsigned* gate = team_words(ring_p, n);
-  __shared__ double xb[2][kTeamN];  // u of this step and of the last one
-  __shared__ double rb[kTeamN];     // r of the last step
   __shared__ double redn[8], redk[8];
   __shared__ double sh_p;  // p at row k + 1
   __shared__ int sh_bad;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int off = kTeamN - n;  // local index = global + off: the last tiles are always full
+  const int off = N - n;  // local index = global + off: the last tiles are always full
   // the member's rows and column 0 (both read before the gate: from there on
   // the owner of row k overwrites that row with its reflector)
-  double a[kTeamRows][kTeamTiles];
+  double a[ROWS][TILES];
 #pragma unroll
-  for (int q = 0; q < kTeamRows; ++q) {
+  for (int q = 0; q < ROWS; ++q) {
     const int i = (8 * q + w) * G + g;
-    static_for<0, kTeamTiles>([&](auto CT) __attribute__((always_inline)) {
+    static_for<0, TILES>([&](auto CT) __attribute__((always_inline)) {
       constexpr int T = decltype(CT)::value;
       const int c = 64 * T + lane - off;
       a[q][T] = 0.0;
@@ -1317,8 +1328,8 @@ __global__ __launch_bounds__(512) void k_tridiag_team(Topo t, const int* order, 
     });
     __builtin_amdgcn_sched_barrier(0);
   }
-  double xo[kTeamOwn];  // this thread's entries L = tid + 512 q of the current column
-  team_first(A, off, g == 0, d, xo, xb[0], xb[1], rb, redn);
+  double xo[OWN];  // this thread's entries L = tid + 512 q of the current column
+  team_first<TILES>(A, off, g == 0, d, xo, xb[0], xb[1], rb, redn);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   // the gate
@@ -1353,21 +1364,21 @@ __global__ __launch_bounds__(512) void k_tridiag_team(Topo t, const int* order, 
     // one sweep over the registers: the pending update of step k - 1 (zero in
     // step 0) and p = A u.  Finished rows ride along: their entries of u and r
     // keep them finite, and the exchange hides them.
-    double p[kTeamRows], ur[kTeamRows], rr[kTeamRows];
+    double p[ROWS], ur[ROWS], rr[ROWS];
 #pragma unroll
-    for (int q = 0; q < kTeamRows; ++q) {
-      const int L = min((8 * q + w) * G + g + off, kTeamN - 1);
+    for (int q = 0; q < ROWS; ++q) {
+      const int L = min((8 * q + w) * G + g + off, N - 1);
       ur[q] = xb[cur ^ 1][L];
       rr[q] = rb[L];
       p[q] = 0.0;
     }
-    static_for<0, kTeamTiles>([&](auto CT) __attribute__((always_inline)) {
+    static_for<0, TILES>([&](auto CT) __attribute__((always_inline)) {
       constexpr int T = decltype(CT)::value;
       if (64 * T + 63 >= K) {  // a column tile with a live column
         const int L = 64 * T + lane;
         const double x = L == K + 1 ? z.v0 : xb[cur][L], u = xb[cur ^ 1][L], r = rb[L];
 #pragma unroll
-        for (int q = 0; q < kTeamRows; ++q) {
+        for (int q = 0; q < ROWS; ++q) {
           a[q][T] = fma(-ur[q], r, fma(-rr[q], u, a[q][T]));
           p[q] = fma(a[q][T], x, p[q]);
         }
@@ -1382,51 +1393,51 @@ __global__ __launch_bounds__(512) void k_tridiag_team(Topo t, const int* order, 
     asm volatile("" : "+v"(ln));
     double* rl0 = rk + (ln - off);  // this lane's column of tile 0
 #pragma unroll
-    for (int q = 0; q < kTeamRows; ++q) {
+    for (int q = 0; q < ROWS; ++q) {
       if ((8 * q + w) * G + g == k + 1) {
-        static_for<0, kTeamTiles>([&](auto CT) __attribute__((always_inline)) {
+        static_for<0, TILES>([&](auto CT) __attribute__((always_inline)) {
           constexpr int T = decltype(CT)::value;
           if (64 * T + ln > K) team_put(rl0 + 64 * T, a[q][T]);
         });
       }
     }
     {
-      double r = row16_sums<kTeamRows>(p, lane & 15);
+      double r = row16_sums<ROWS>(p, lane & 15);
       r += __shfl_xor(r, 16, 64);
       r += __shfl_xor(r, 32, 64);
-      const int i = (8 * row16_index<kTeamRows>(lane & 15) + w) * G + g;
+      const int i = (8 * row16_index<ROWS>(lane & 15) + w) * G + g;
       if (lane < 16 && (lane & 1) == 0 && i > k && i < n) team_put(pk + i, r);
     }
     if (g == k % G) {  // this member keeps column k's unit reflector (zero for no reflection)
 #pragma unroll
-      for (int q = 0; q < kTeamOwn; ++q) {
+      for (int q = 0; q < OWN; ++q) {
         const int L = tid + 512 * q;
-        if (L > K && L < kTeamN) A[(L - off) + (int64_t)k * n] = (L == K + 1 ? z.v0 : xo[q]) * z.inv;
+        if (L > K && L < N) A[(L - off) + (int64_t)k * n] = (L == K + 1 ? z.v0 : xo[q]) * z.inv;
       }
       if (tid == 0) e[k] = z.noref ? xb[cur][K + 1] : z.alpha;
     }
     // everybody's p and the row
-    double po[kTeamOwn], ro[kTeamOwn];
+    double po[OWN], ro[OWN];
     {
       int bad = 0;
-      unsigned long long bp[kTeamOwn], br[kTeamOwn];
+      unsigned long long bp[OWN], br[OWN];
 #pragma unroll
-      for (int q = 0; q < kTeamOwn; ++q) {
+      for (int q = 0; q < OWN; ++q) {
         bp[q] = 0;
         br[q] = 0;
       }
       for (int spin = 0;; ++spin) {
         bool wait = false;
 #pragma unroll
-        for (int q = 0; q < kTeamOwn; ++q) {
+        for (int q = 0; q < OWN; ++q) {
           const int L = tid + 512 * q;
-          if (L > K && L < kTeamN) {
+          if (L > K && L < N) {
             bp[q] = team_peek(pk + (L - off));
             br[q] = team_peek(rk + (L - off));
           }
         }
 #pragma unroll
-        for (int q = 0; q < kTeamOwn; ++q) wait = wait || bp[q] == kTeamEmpty || br[q] == kTeamEmpty;
+        for (int q = 0; q < OWN; ++q) wait = wait || bp[q] == kTeamEmpty || br[q] == kTeamEmpty;
         if (!wait) break;
         if (spin >= kTeamSpins) {
           bad = 1;
@@ -1436,7 +1447,7 @@ __global__ __launch_bounds__(512) void k_tridiag_team(Topo t, const int* order, 
       if (bad) sh_bad = 1;
       double kp = 0.0;
 #pragma unroll
-      for (int q = 0; q < kTeamOwn; ++q) {
+      for (int q = 0; q < OWN; ++q) {
         const int L = tid + 512 * q;
         po[q] = __longlong_as_double((long long)bp[q]);  // 0 where L <= K
         ro[q] = __longlong_as_double((long long)br[q]);
@@ -1451,16 +1462,16 @@ __global__ __launch_bounds__(512) void k_tridiag_team(Topo t, const int* order, 
     }
     __syncthreads();
     if (sh_bad) {
-      if (tid == 0) st[s].status = 8;
+      if (tid == 0) *status = 8;
       return;
     }
-    team_vectors(z, K, redk, sh_p, po, ro, xo, xb[cur], xb[cur ^ 1], rb, redn,
+    team_vectors<TILES>(z, K, redk, sh_p, po, ro, xo, xb[cur], xb[cur ^ 1], rb, redn,
                  g == 0 && k + 1 < kend ? d + k + 1 : nullptr);
     // every member has published step k, so it has read step k - 1: empty that slot
     if (k > 0) {
       double* pl = ring_p + (int64_t)((k - 1) & (kTeamRing - 1)) * n;
       double* rl = ring_r + (int64_t)((k - 1) & (kTeamRing - 1)) * n;
-      if (lane < kTeamRows) {
+      if (lane < ROWS) {
         const int i = (8 * lane + w) * G + g;
         if (i >= k && i < n) team_clear(pl + i);
       }
@@ -1474,16 +1485,32 @@ __global__ __launch_bounds__(512) void k_tridiag_team(Topo t, const int* order, 
   int ln = lane;
   asm volatile("" : "+v"(ln));
 #pragma unroll
-  for (int q = 0; q < kTeamRows; ++q) {
+  for (int q = 0; q < ROWS; ++q) {
     const int i = (8 * q + w) * G + g;
     if (i >= kend && i < n)
-      static_for<0, kTeamTiles>([&](auto CT) __attribute__((always_inline)) {
+      static_for<0, TILES>([&](auto CT) __attribute__((always_inline)) {
         constexpr int T = decltype(CT)::value;
         // columns >= kend are the last kFullN local ones
-        if constexpr (64 * T >= kTeamN - kFullN) A[(int64_t)i * n + (64 * T + ln - off)] = a[q][T];
+        if constexpr (64 * T >= N - kFullN) A[(int64_t)i * n + (64 * T + ln - off)] = a[q][T];
       });
   }
   if (g == 0 && tid == 0) gate[1] = 1u;  // done
+}
+
+__global__ __launch_bounds__(512) void k_tridiag_team(Topo t, const int* order, double* Aall, double* dall,
+                                                      double* eall, double* Zall, const unsigned char* active,
+                                                      SysState* st) {
+  const int s = order[blockIdx.y];
+  if (active && !active[s]) return;
+  const int n = t.ao_off[s + 1] - t.ao_off[s];
+  const int G = team_size(n), g = blockIdx.x;
+  if (g >= G) return;
+  __shared__ double xb[2][kTeamN], rb[kTeamN];
+  const int64_t mo = t.mat_off[s], o = t.ao_off[s];
+  team_class(n, [&](auto R, auto T) __attribute__((always_inline)) {
+    team_member<decltype(R)::value, decltype(T)::value>(n, G, g, Aall + mo, dall + o, eall + o, Zall + mo,
+                                                        &st[s].status, xb, rb);
+  });
 }
 
 // The team's reduction by one workgroup, for systems whose team left at the gate:
@@ -1492,24 +1519,15 @@ __global__ __launch_bounds__(512) void k_tridiag_team(Topo t, const int* order, 
 // could assemble.  Bound: the sweep over the trailing block (16 n^2 bytes a step
 // through one CU): 205 ms at 1280 AOs (240 with four tiles in flight instead of
 // ten), where the team takes 6.6 ms.
-__global__ __launch_bounds__(512) void k_tridiag_solo(Topo t, const int* order, double* Aall, double* dall,
-                                                      double* eall, double* Zall, const unsigned char* active) {
-  const int s = order[blockIdx.x];
-  if (active && !active[s]) return;
-  const int n = t.ao_off[s + 1] - t.ao_off[s];
-  unsigned* words = team_words(Zall + t.mat_off[s], n);
-  if (words[1] != 0u) return;  // reduced by its team
-  double* A = Aall + t.mat_off[s];
-  double* d = dall + t.ao_off[s];
-  double* e = eall + t.ao_off[s];
-  __shared__ double xb[2][kTeamN];
-  __shared__ double rb[kTeamN];
-  __shared__ double pb[kTeamN];
+template <int TILES>
+__device__ __forceinline__ void team_solo(int n, double* A, double* d, double* e, double (&xb)[2][kTeamN],
+                                          double (&rb)[kTeamN], double (&pb)[kTeamN]) {
+  constexpr int N = 64 * TILES, OWN = team_own(TILES);
   __shared__ double redn[8], redk[8];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int off = kTeamN - n;
-  double xo[kTeamOwn];
-  team_first(A, off, true, d, xo, xb[0], xb[1], rb, redn);
+  const int off = N - n;
+  double xo[OWN];
+  team_first<TILES>(A, off, true, d, xo, xb[0], xb[1], rb, redn);
   __syncthreads();
   const int kend = n - kFullN;
   int cur = 0;
@@ -1541,9 +1559,9 @@ __global__ __launch_bounds__(512) void k_tridiag_solo(Topo t, const int* order, 
         }
       };
       int T = T0;
-      for (; T + 10 <= kTeamTiles; T += 10) sweep(std::integral_constant<int, 10>{}, T);
-      for (; T + 4 <= kTeamTiles; T += 4) sweep(std::integral_constant<int, 4>{}, T);
-      for (; T < kTeamTiles; ++T) sweep(std::integral_constant<int, 1>{}, T);
+      for (; T + 10 <= TILES; T += 10) sweep(std::integral_constant<int, 10>{}, T);
+      for (; T + 4 <= TILES; T += 4) sweep(std::integral_constant<int, 4>{}, T);
+      for (; T < TILES; ++T) sweep(std::integral_constant<int, 1>{}, T);
       double r = row16_sums<1>(p, lane & 15);
       r += __shfl_xor(r, 16, 64);
       r += __shfl_xor(r, 32, 64);
@@ -1551,11 +1569,11 @@ __global__ __launch_bounds__(512) void k_tridiag_solo(Topo t, const int* order, 
     }
     if (k == kend) break;
     __syncthreads();
-    double po[kTeamOwn], ro[kTeamOwn], kp = 0.0;
+    double po[OWN], ro[OWN], kp = 0.0;
 #pragma unroll
-    for (int q = 0; q < kTeamOwn; ++q) {
+    for (int q = 0; q < OWN; ++q) {
       const int L = tid + 512 * q;
-      const bool live = L > K && L < kTeamN;
+      const bool live = L > K && L < N;
       po[q] = live ? pb[L] : 0.0;
       ro[q] = live ? A[(int64_t)(k + 1) * n + (L - off)] : 0.0;
       if (live) A[(L - off) + (int64_t)k * n] = (L == K + 1 ? z.v0 : xo[q]) * z.inv;
@@ -1566,12 +1584,26 @@ __global__ __launch_bounds__(512) void k_tridiag_solo(Topo t, const int* order, 
     kp = wave_sum(kp);
     if (lane == 0) redk[w] = kp;
     __syncthreads();
-    team_vectors(z, K, redk, pb[K + 1], po, ro, xo, xb[cur], xb[cur ^ 1], rb, redn,
+    team_vectors<TILES>(z, K, redk, pb[K + 1], po, ro, xo, xb[cur], xb[cur ^ 1], rb, redn,
                  k + 1 < kend ? d + k + 1 : nullptr);
     __syncthreads();
     cur ^= 1;
   }
-  if (tid == 0) words[1] = 1u;
+}
+
+__global__ __launch_bounds__(512) void k_tridiag_solo(Topo t, const int* order, double* Aall, double* dall,
+                                                      double* eall, double* Zall, const unsigned char* active) {
+  const int s = order[blockIdx.x];
+  if (active && !active[s]) return;
+  const int n = t.ao_off[s + 1] - t.ao_off[s];
+  unsigned* words = team_words(Zall + t.mat_off[s], n);
+  if (words[1] != 0u) return;  // reduced by its team
+  __shared__ double xb[2][kTeamN], rb[kTeamN], pb[kTeamN];
+  const int64_t mo = t.mat_off[s], o = t.ao_off[s];
+  team_class(n, [&](auto, auto T) __attribute__((always_inline)) {
+    team_solo<decltype(T)::value>(n, Aall + mo, dall + o, eall + o, xb, rb, pb);
+  });
+  if (threadIdx.x == 0) words[1] = 1u;
 }
 
 // The back-transformation applies the reflectors in compact WY blocks of
