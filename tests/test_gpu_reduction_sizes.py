@@ -164,3 +164,29 @@ def test_closed_gate_changes_no_bit(monkeypatch):
     ms = [o.extension["kernel_stats"]["tridiag"]["ms"] for o in (team, solo)]
     print("reduction: teams %.1f ms, one workgroup %.1f ms" % tuple(ms), flush=True)
     assert ms[1] > 3.0 * ms[0]
+
+
+def test_gate_failure_shortens_later_waits(monkeypatch):
+    """Gates that no count fills: the first round waits 0.2 s, the others 20 ms each, and
+    the result is that of the teams."""
+    rng = np.random.default_rng(5)
+    b = workloads.from_systems([workloads.alkane(50, rng), workloads.alkane(45, rng)])
+    ctx = interface.Context("hip", 0)
+
+    def run():
+        return interface.compute_arrays(ctx, b.atom_offsets, b.atomic_numbers, b.positions, b.molecular_charges,
+                                        b.unpaired_electrons, kernel_stats=["tridiag"])
+
+    try:
+        team = run()
+        monkeypatch.setenv("XTBLOOM_AMD_TEAMS", "never")
+        print("case gates that never fill, 302 and 272 AOs", flush=True)
+        held = run()
+    finally:
+        ctx.close()
+    rounds = int(team.scc_iterations.max())
+    assert np.array_equal(held.energies, team.energies) and np.array_equal(held.charges, team.charges)
+    ms = held.extension["kernel_stats"]["tridiag"]["ms"]
+    print("reduction of %d rounds: %.0f ms" % (rounds, ms), flush=True)
+    # 200 + 20 (rounds - 1) ms of waiting and one workgroup's work, below 20 ms a round
+    assert 200.0 <= ms <= 200.0 + 40.0 * rounds

@@ -884,7 +884,10 @@ xtbloom_status_t admit(xtbloom_context_t* context, xtbloom_plan_t* plan, const x
     const char* env = getenv("XTBLOOM_AMD_SPLIT32");
     job.ro.split32 = env != nullptr && std::strcmp(env, "1") == 0;
     env = getenv("XTBLOOM_AMD_TEAMS");
-    job.ro.teams = env == nullptr || std::strcmp(env, "0") != 0;
+    job.ro.teams = env == nullptr                   ? xtb::TeamGate::open
+                   : std::strcmp(env, "0") == 0     ? xtb::TeamGate::closed
+                   : std::strcmp(env, "never") == 0 ? xtb::TeamGate::never
+                                                    : xtb::TeamGate::open;
   }
   std::memset(&job.result, 0, sizeof(job.result));
   std::memcpy(&job.result, result, std::min<size_t>(sizeof(job.result), result->struct_size));

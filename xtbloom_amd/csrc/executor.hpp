@@ -30,6 +30,8 @@ struct HostBatch {
   const int32_t* spin = nullptr;          // [B] spin channels (1 or 2), or null (all 1)
 };
 
+enum class TeamGate : int { open, closed, never };
+
 struct RunOptions {
   int max_iterations = 250;
   double charge_tolerance = 1e-6;
@@ -55,10 +57,10 @@ struct RunOptions {
   // split-precision FP32 matrix-core density products: P in the SCC rounds
   // whose mixer residual is above 1e-3 (and the first round), W always
   bool split32 = false;
-  // reductions by teams of workgroups; off, every team finds its gate closed and
-  // leaves (the path it takes when the chip is held by something else), and one
-  // workgroup does the same arithmetic
-  bool teams = true;
+  // reductions by teams of workgroups; closed, every team leaves at once, never,
+  // it waits for a member that does not come (the path it takes when the chip is
+  // held by something else): one workgroup then does the same arithmetic
+  TeamGate teams = TeamGate::open;
   // allocate nothing: the device workspace is the fixed per-GPU array of
   // kNoAllocWorkspaceBytes (a larger batch is rejected before any kernel),
   // host staging is pinned only when the context's pinned block is already

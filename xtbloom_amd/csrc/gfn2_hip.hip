@@ -383,6 +383,7 @@ struct Device {
   hipGraphExec_t graph_exec = nullptr;
   std::vector<char> graph_key;
 
+  int cus = 0;                         // compute units, the most workgroups of a team
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
   hipEvent_t round_ev[2] = {nullptr, nullptr};  // end of the SCC rounds of each parity
   std::vector<hipEvent_t> probe_pool;  // per-launch timing events, grow-only
@@ -448,6 +449,7 @@ Device* device_create(int device_id, void* stream, std::string& error) {
     device_destroy(d);
     return nullptr;
   }
+  ok = ok && hipDeviceGetAttribute(&d->cus, hipDeviceAttributeMultiprocessorCount, device_id) == hipSuccess;
   for (int i = 0; i < 4 && ok; ++i) ok = hipEventCreate(&d->ev[i]) == hipSuccess;
   for (int i = 0; i < 2 && ok; ++i)
     ok = hipEventCreateWithFlags(&d->round_ev[i], hipEventDisableTiming) == hipSuccess;
@@ -728,7 +730,7 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
   bytes += plan_bytes<SysState>(B);
   addb(B); addb(B);            // active, valid
   addi(2);                     // counter
-  addi(1);                     // device round counter (batched path)
+  addi(2);                     // device round counter (batched path), failure of a team's gate
   addi((size_t)opt.max_iterations + kGraphRounds);  // active count after each round (batched path)
   addi(B);                     // kocc
   addd(3 * (size_t)N);         // grad
@@ -974,7 +976,7 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
   unsigned char* d_active = cv.take<unsigned char>(B);
   unsigned char* d_valid = cv.take<unsigned char>(B);
   int* d_count = cv.take<int>(2);
-  int* d_round = cv.take<int>(1);
+  int* d_round = cv.take<int>(2);
   int* d_cnt_round = cv.take<int>((size_t)opt.max_iterations + kGraphRounds);
   int* d_kocc = cv.take<int>(B);
   double* d_grad = cv.take<double>(3 * (size_t)N);
@@ -1259,9 +1261,9 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
     if (teams) {
       const int n_top = T.ao_off[T.order[n_team0] + 1] - T.ao_off[T.order[n_team0]];
       hipLaunchKernelGGL(k_team_init, dim3(n_large - n_team0), dim3(256), 0, sm, t, d_order + n_team0, d_active, dZ,
-                         opt.teams ? 0u : kTeamClosed);
+                         opt.teams == TeamGate::closed ? 0 : dev->cus, opt.teams == TeamGate::never ? kTeamNever : 0u);
       hipLaunchKernelGGL(k_tridiag_team, dim3(team_size(n_top), n_large - n_team0), dim3(512), 0, sm, t,
-                         d_order + n_team0, dA, d_td, d_te, dZ, d_active, d_st);
+                         d_order + n_team0, dA, d_td, d_te, dZ, d_active, d_st, d_round + 1);
       hipLaunchKernelGGL(k_tridiag_solo, dim3(n_large - n_team0), dim3(512), 0, sm, t, d_order + n_team0, dA, d_td,
                          d_te, dZ, d_active);
     }
@@ -1367,6 +1369,7 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
     if (sm == nullptr || hipStreamIsCapturing(sm, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone)
       graph_rounds = false;
   }
+  if (graph_rounds || n_large > n_team0) HIP_TRY(hipMemsetAsync(d_round, 0, 2 * sizeof(int), sm));
   if (graph_rounds) {
     // Batched path: kGraphRounds rounds per captured graph, the round number
     // and the per-round active counts on the device.  The counters are reset
@@ -1374,7 +1377,6 @@ static int run_batch_core(Device* dev, const HostBatch& hb, const RunOptions& op
     // graph is kept on the device while the arena, the topology and the policy
     // it was captured for are unchanged (every kernel argument is a function
     // of those).
-    HIP_TRY(hipMemsetAsync(d_round, 0, sizeof(int), sm));
     HIP_TRY(hipMemsetAsync(d_cnt_round, 0, sizeof(int) * ((size_t)opt.max_iterations + kGraphRounds), sm));
     std::vector<char> key;
     auto put = [&](const auto& v) {

@@ -1159,8 +1159,12 @@ __device__ __forceinline__ void tridiag_full(double* A, int64_t ld, int n, doubl
 // Waiting is safe: no member writes anything before all G have met at the gate,
 // so from then on every partner is resident and runs.  Members that do not all
 // arrive within kTeamWaitTicks (the chip is held by something else) close the
-// gate together and leave; k_tridiag_solo then does the same arithmetic.  The
-// spins are bounded too; one that runs out fails the system (status 8).
+// gate together and leave; k_tridiag_solo then does the same arithmetic.  After
+// one such failure the call's teams wait kTeamRetryTicks only: above the 7 ms for
+// which a running team can hold a partner's CU, and a call of ten rounds on a chip
+// that stays held loses 0.4 s to waiting instead of 2 s.  A team larger than the
+// device finds its gate closed from the start.  The spins are bounded too; one that
+// runs out fails the system (status 8).
 //
 // Bound: the latency of a step, 4.5 us at 482 AOs (16 members) and 5.5 us at
 // 1142 (36), most of it the exchange through memory.  Measured against one
@@ -1172,8 +1176,10 @@ constexpr int kTeamRing = 8;
 constexpr int team_own(int tiles) { return (64 * tiles + 511) / 512; }  // vector entries per thread
 constexpr unsigned long long kTeamEmpty = 0xfff7a5a5c3c3e1e1ull;
 constexpr long long kTeamWaitTicks = 20000000;  // 100 MHz counter: 0.2 s
+constexpr long long kTeamRetryTicks = 2000000;
 constexpr int kTeamSpins = 1 << 22;
 constexpr unsigned kTeamClosed = 1u << 30;
+constexpr unsigned kTeamNever = 1u << 29;  // a start value from which no count reaches G
 // Rows of a wavefront: as many as about 80 doubles a lane hold, tiles of 64 columns
 // for the largest n of the class.  Smaller teams leave CUs to other systems: with
 // four rows for every n the teams of 256 systems of 482 AOs took 239 ms of a call
@@ -1279,13 +1285,13 @@ __device__ __forceinline__ void team_vectors(const TeamStep& z, int K, const dou
 }
 
 __global__ __launch_bounds__(256) void k_team_init(Topo t, const int* order, const unsigned char* active,
-                                                   double* Zall, unsigned gate) {
+                                                   double* Zall, int cus, unsigned start) {
   const int s = order[blockIdx.x];
   if (active && !active[s]) return;
   const int n = t.ao_off[s + 1] - t.ao_off[s];
   double* Z = Zall + t.mat_off[s];
   for (int i = threadIdx.x; i < 2 * kTeamRing * n; i += 256) Z[i] = __longlong_as_double((long long)kTeamEmpty);
-  if (threadIdx.x < 2) team_words(Z, n)[threadIdx.x] = threadIdx.x == 0 ? gate : 0u;
+  if (threadIdx.x < 2) team_words(Z, n)[threadIdx.x] = threadIdx.x != 0 ? 0u : team_size(n) > cus ? kTeamClosed : start;
 }
 
 __device__ __forceinline__ void team_put(double* p, double x) {
@@ -1305,7 +1311,8 @@ __device__ __forceinline__ unsigned long long team_peek(const double* p) {
 // member g of G; xb: u of this step and of the last one, rb: r of the last step
 template <int ROWS, int TILES>
 __device__ __forceinline__ void team_member(int n, int G, int g, double* A, double* d, double* e, double* ring_p,
-                                            int* status, double (&xb)[2][kTeamN], double (&rb)[kTeamN]) {
+                                            int* status, int* failed, double (&xb)[2][kTeamN],
+                                            double (&rb)[kTeamN]) {
   constexpr int N = 64 * TILES, OWN = team_own(TILES);
   double* ring_r = ring_p + (int64_t)kTeamRing * n;
   unsigned* gate = team_words(ring_p, n);
@@ -1342,11 +1349,15 @@ __device__ __forceinline__ void team_member(int n, int G, int g, double* A, doub
       __builtin_amdgcn_s_sleep(2);
       old = __hip_atomic_load(gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       closed = (old & kTeamClosed) != 0;
-      if (!closed && (old & ~kTeamClosed) != (unsigned)G && wall_clock64() - t0 > kTeamWaitTicks) {
+      const long long limit = __hip_atomic_load(failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ? kTeamRetryTicks
+                                                                                                    : kTeamWaitTicks;
+      if (!closed && (old & ~kTeamClosed) != (unsigned)G && wall_clock64() - t0 > limit) {
         unsigned want = old;
         if (__hip_atomic_compare_exchange_strong(gate, &want, old | kTeamClosed, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT))
+                                                 __HIP_MEMORY_SCOPE_AGENT)) {
           closed = 1;
+          __hip_atomic_store(failed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
       }
     }
     sh_bad = closed;
@@ -1499,7 +1510,7 @@ __device__ __forceinline__ void team_member(int n, int G, int g, double* A, doub
 
 __global__ __launch_bounds__(512) void k_tridiag_team(Topo t, const int* order, double* Aall, double* dall,
                                                       double* eall, double* Zall, const unsigned char* active,
-                                                      SysState* st) {
+                                                      SysState* st, int* failed) {
   const int s = order[blockIdx.y];
   if (active && !active[s]) return;
   const int n = t.ao_off[s + 1] - t.ao_off[s];
@@ -1509,7 +1520,7 @@ __global__ __launch_bounds__(512) void k_tridiag_team(Topo t, const int* order, 
   const int64_t mo = t.mat_off[s], o = t.ao_off[s];
   team_class(n, [&](auto R, auto T) __attribute__((always_inline)) {
     team_member<decltype(R)::value, decltype(T)::value>(n, G, g, Aall + mo, dall + o, eall + o, Zall + mo,
-                                                        &st[s].status, xb, rb);
+                                                        &st[s].status, failed, xb, rb);
   });
 }
 
