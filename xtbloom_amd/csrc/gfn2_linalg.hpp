@@ -1152,9 +1152,15 @@ __device__ __forceinline__ void tridiag_full(double* A, int64_t ld, int n, doubl
 //
 // The exchanged words validate themselves: a buffer starts out filled with
 // kTeamEmpty (a NaN no arithmetic produces) and a reader spins on each word
-// until it is something else.  Slot k % kTeamRing is emptied by its writers in
-// step k + 1, when every member has published that step and so has read slot k;
-// it is written again kTeamRing - 1 exchanges later.
+// until it is something else.  Slot k % kTeamRing is emptied in step k + 1, when
+// every member has published that step and so has read slot k; it is written
+// again in step k + kTeamRing, a row's slot by another member than the one that
+// emptied it.  Emptying comes before that write: the emptying stores are waited
+// for before the first barrier of step k + 2; behind it the member publishes p of
+// step k + 3 (every member owns one of the last kFullN rows, so it always has one
+// to publish); and the next writer has read that p, from every member, before it
+// goes on to step k + kTeamRing.  The words are agent-scope stores, complete at the level
+// that every member's loads read when the wait for them returns.
 //
 // Waiting is safe: no member writes anything before all G have met at the gate,
 // so from then on every partner is resident and runs.  Members that do not all
@@ -1187,6 +1193,7 @@ constexpr unsigned kTeamNever = 1u << 29;  // a start value from which no count 
 // of 650 AOs 515 and 316 (six rows), 319 with one workgroup per system.
 __host__ __device__ constexpr int team_rows(int n) { return n <= 640 ? 8 : n <= 832 ? 6 : n <= 1024 ? 5 : 4; }
 __host__ __device__ constexpr int team_size(int n) { return (n + 8 * team_rows(n) - 1) / (8 * team_rows(n)); }
+static_assert(team_size(kTeamN) <= kFullN && team_size(640) <= kFullN, "a row of the last kFullN for every member");
 // f(rows of a wavefront, column tiles) of n's class
 template <typename F>
 __device__ __forceinline__ void team_class(int n, F&& f) {
@@ -1396,9 +1403,7 @@ __device__ __forceinline__ void team_member(int n, int G, int g, double* A, doub
       }
     });
     if (k == kend) break;  // the last update is in: the trailing block is done
-    // publish row k + 1 and the rows' p.  The stores that emptied a slot were
-    // issued before the loads of the next exchange, whose return they precede,
-    // so they are long done when that slot comes round again.
+    // publish row k + 1 and the rows' p
     // (opaque lane: addresses kept from step to step would live in scratch)
     int ln = lane;
     asm volatile("" : "+v"(ln));
@@ -1471,6 +1476,9 @@ __device__ __forceinline__ void team_member(int n, int G, int g, double* A, doub
       kp = wave_sum(kp);
       if (lane == 0) redk[w] = kp;
     }
+    // the stores that emptied a slot in the last step are done (nothing to wait
+    // for: they were issued a whole exchange ago)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (sh_bad) {
       if (tid == 0) *status = 8;
