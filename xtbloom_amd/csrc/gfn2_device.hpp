@@ -12,12 +12,12 @@
 namespace xtb {
 
 // Systems of at most kMaxAO AOs keep their per-system work vectors (the
-// eigensolver's tridiagonal and eigenvalue arrays, the reduction's partial
-// sums, the conditioning estimate's vectors, per-atom force accumulators) in
-// LDS.  Larger systems, up to kMaxSystemAO, run instantiations of the same
-// kernels that keep these vectors in a global slice of kBigPerAO doubles per
-// AO plus kBigPerSys per system, at big_offset(); the host launches them over
-// the prefix of the size order above kMaxAO.
+// conditioning estimate's vectors, the spin fold's) in LDS.  Larger systems, up
+// to kMaxSystemAO, run instantiations of the same kernels that keep these vectors
+// in a global slice of kBigPerAO doubles per AO plus kBigPerSys per system, at
+// big_offset(); the host launches them over the prefix of the size order above
+// kMaxAO.  The same slice holds the work vectors of k_tridiag_blocked (above
+// kTeamN AOs) and of k_tridiag_eigen<true> (above kEigSplitAO).
 constexpr int kMaxAO = 1024;
 constexpr int kMaxSystemAO = 8192;
 constexpr int kBigPerAO = 12;

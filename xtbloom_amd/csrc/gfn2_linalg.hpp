@@ -1,6 +1,7 @@
 // Dense FP64 linear algebra for the ragged batch: tiled GEMM over a tile
-// queue, per-system Cholesky/inverse and the symmetric eigensolver
-// (Householder tridiagonalization + implicit QL + back-transformation).
+// queue, per-system Cholesky/inverse and the symmetric eigensolver (Householder
+// tridiagonalization, Sturm bisection and Newton steps, twisted or inverse
+// iteration, back-transformation).
 #pragma once
 
 #include <type_traits>
@@ -270,59 +271,22 @@ __global__ __launch_bounds__(256) void k_gemm_split32(Topo t, const TileTask* ta
     }
 }
 
-// Cholesky S = L L^T and X = L^{-T} with everything in global memory (any n);
-// sets *bad on a non-positive pivot.
-__device__ void cholesky_global(const double* Sm, double* L, double* Xm, int n, int& bad) {
-  for (int64_t idx = threadIdx.x; idx < (int64_t)n * n; idx += blockDim.x) L[idx] = Sm[idx];
-  __syncthreads();
-  // right-looking column Cholesky
-  for (int k = 0; k < n; ++k) {
-    __shared__ double piv;
-    if (threadIdx.x == 0) {
-      double d = L[k + (int64_t)k * n];
-      if (!(d > 0.0)) { bad = 1; d = 1.0; }
-      piv = sqrt(d);
-      L[k + (int64_t)k * n] = piv;
-    }
-    __syncthreads();
-    for (int i = k + 1 + threadIdx.x; i < n; i += blockDim.x) L[i + (int64_t)k * n] /= piv;
-    __syncthreads();
-    // trailing update of the lower triangle: L[i][j] -= L[i][k] L[j][k], j in (k, i]
-    const int m = n - k - 1;
-    for (int64_t idx = threadIdx.x; idx < (int64_t)m * m; idx += blockDim.x) {
-      const int jj = (int)(idx / m), ii = (int)(idx % m);
-      if (ii < jj) continue;
-      const int i = k + 1 + ii, j = k + 1 + jj;
-      L[i + (int64_t)j * n] -= L[i + (int64_t)k * n] * L[j + (int64_t)k * n];
-    }
-    __syncthreads();
-  }
-  // inverse of L by columns: Linv e_j, thread per column j; X = Linv^T (row-major X[r][c] = Linv[c][r])
-  // Linv is lower triangular; column j of Linv -> row j of X.
-  for (int j = threadIdx.x; j < n; j += blockDim.x) {
-    double* xr = Xm + (int64_t)j * n;  // row j of X holds column j of Linv
-    for (int i = 0; i < j; ++i) xr[i] = 0.0;
-    for (int i = j; i < n; ++i) {
-      double v = (i == j) ? 1.0 : 0.0;
-      for (int k = j; k < i; ++k) v -= L[i + (int64_t)k * n] * xr[k];
-      xr[i] = v / L[i + (int64_t)i * n];
-    }
-  }
-  __syncthreads();
-}
-
 // ---------------------------------------------------------------------------
-// Symmetric eigensolver in three launches (all FP64):
-//   k_tridiag         Householder reduction A = Q T Q^T, one 256-thread block per
-//                     system; T's diagonal/off-diagonal go to d/e, the reflectors
-//                     (H = I - 2 v v^T, |v| = 1) stay in A's strict lower triangle.
-//   k_tridiag_eigen   eigenpairs of T, one block per system: T is split where an
-//                     off-diagonal is negligible, every eigenvalue is found by
-//                     Sturm-count bisection (one thread per eigenvalue), every
-//                     eigenvector by inverse iteration with a partially pivoted
-//                     tridiagonal LU (one thread per cluster of close eigenvalues,
-//                     modified Gram-Schmidt inside a cluster).  Eigenvalues are
-//                     ranked ascending (ties by index).
+// Symmetric eigensolver in three stages (all FP64):
+//   reduction         Householder A = Q T Q^T; T's diagonal/off-diagonal go to d/e,
+//                     the reflectors (H = I - 2 v v^T, |v| = 1) stay in A's strict
+//                     lower triangle.  k_tridiag up to 256 AOs (a 512-thread block
+//                     per system), k_tridiag_team up to kTeamN, k_tridiag_blocked
+//                     above.
+//   eigenpairs of T   k_tridiag_eigen, one block per system, or k_eig_values,
+//                     _occupations and _vectors over the chip (257 to kEigSplitAO
+//                     AOs): T is split where an off-diagonal is negligible, every
+//                     eigenvalue is found by Sturm counts and Newton steps (a
+//                     thread per eigenvalue), every eigenvector from its twisted
+//                     factorization or, in a cluster of close eigenvalues, by
+//                     inverse iteration with a partially pivoted tridiagonal LU and
+//                     modified Gram-Schmidt (a thread per cluster).  Eigenvalues
+//                     are ranked ascending (ties by index).
 //   k_backtransform   Y = Q Z on column blocks, many blocks per system, on the
 //                     matrix cores (k_backtransform_wy above 256 AOs).
 // Layouts: Z and Y are row-major (row i = component i, column j = vector j).
@@ -1854,7 +1818,7 @@ __device__ __forceinline__ void cholesky_registers(const double* Sm, double* L, 
   __syncthreads();
 }
 
-// Per-system overlap factorization, 512 threads: X = L^{-T} with L in `work`
+// Per-system overlap factorization, n <= 256, 512 threads: X = L^{-T} with L in `work`
 // (column-major).  status = 8 on a non-positive pivot; the conditioning gate
 // follows in k_overlap_rcond.
 __global__ __launch_bounds__(512) void k_cholesky_inverse(Topo t, const int* order, const double* S,
@@ -1873,8 +1837,7 @@ __global__ __launch_bounds__(512) void k_cholesky_inverse(Topo t, const int* ord
   if (n <= 64) cholesky_registers<4>(Sm, L, Xm, n, lcol, xr, bad);
   else if (n <= 128) cholesky_registers<8>(Sm, L, Xm, n, lcol, xr, bad);
   else if (n <= 192) cholesky_registers<12>(Sm, L, Xm, n, lcol, xr, bad);
-  else if (n <= 256) cholesky_registers<16>(Sm, L, Xm, n, lcol, xr, bad);
-  else cholesky_global(Sm, L, Xm, n, bad);
+  else cholesky_registers<16>(Sm, L, Xm, n, lcol, xr, bad);
   if (threadIdx.x == 0 && bad) status[s].status = 8;
 }
 
@@ -2829,14 +2792,6 @@ struct FermiOut {
   double kt;
 };
 
-// Eigenvalues of T (all), then the Fermi occupations, then eigenvectors for the
-// kocc lowest eigenvalues only, written to Z column = ascending rank.
-// From the second SCC round on, wall holds the previous round's ascending
-// eigenvalues on entry; shift[s] carries the largest eigenvalue change of the
-// system's previous round (written here for the next one).  BIG: the systems
-// above kMaxAO AOs, with d, e, e^2, the eigenvalues and their ranks in their
-// global slice of `big`.  Clusters of more than kSerialCluster close
-// eigenvalues are left to k_cluster_vectors through `co`.
 // T of one system into d, e and e2 = e^2 with the negligible off-diagonals
 // zeroed, by the whole block; the pivot floor, and whether T did not split.
 __device__ __forceinline__ bool eig_load(const double* dg, const double* eg, int n, double* d, double* e, double* e2,
@@ -3204,6 +3159,14 @@ __device__ __forceinline__ void eig_vector(int j, int n, int kocc, const double*
   }
 }
 
+// Eigenvalues of T (all), then the Fermi occupations, then eigenvectors for the
+// kocc lowest eigenvalues only, written to Z column = ascending rank.
+// From the second SCC round on, wall holds the previous round's ascending
+// eigenvalues on entry; shift[s] carries the largest eigenvalue change of the
+// system's previous round (written here for the next one).  BIG: the systems
+// above kEigSplitAO AOs, with d, e, e^2, the eigenvalues and their ranks in their
+// global slice of `big`.  Clusters of more than kSerialCluster close
+// eigenvalues are left to k_cluster_vectors through `co`.
 template <bool BIG>
 __global__ __launch_bounds__(256) void k_tridiag_eigen(Topo t, const int* order,
                                                        const unsigned char* active,
@@ -3615,9 +3578,8 @@ __global__ __launch_bounds__(256) void k_cluster_vectors(Topo t, const int* orde
   }
 }
 
-// One column block of one system: Y[:, j0 .. j0+cw) = Q Z[:, j0 .. j0+cw), for
-// the columns below the system's kocc (Z holds eigenvectors by ascending rank).
-// One block's columns of the back-transformation.
+// One block's columns of the back-transformation, from j0 on; those at or past the
+// system's kocc are left out (Z holds eigenvectors by ascending rank).
 struct BackTask {
   int sys;
   int j0;

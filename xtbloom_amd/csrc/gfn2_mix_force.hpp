@@ -994,21 +994,17 @@ __global__ __launch_bounds__(256) void k_wide_atoms(Topo t, const int* order, co
   }
 }
 
-// D4 three-body ATM energy and gradient with zero-charge weights
-// (reference d4.cpp:1120-1362).  Every factor of a triple's term that belongs
+// D4 three-body ATM term with zero-charge weights (reference d4.cpp:1120-1362),
+// for k_force_atm and k_wide_*.  Every factor of a triple's term that belongs
 // to one pair is computed once per ordered pair and staged (structure of
 // arrays at 5 apair_off[s]):
 //   r2 = |R_x - R_y|^2,  ir = 1/|R_x - R_y|,  q = (R0_xy / |R_x - R_y|)^(16/3),
 //   sc = sqrt|C6_xy|,    dcr = (dC6_xy/dCN_x) / C6_xy,
 // so that with r1p = r_ij r_ik r_jk, (R0_ij R0_ik R0_jk / r1p)^(16/3) = q_ij q_ik q_jk
 // and sqrt|C6_ij C6_ik C6_jk| = sc_ij sc_ik sc_jk: a triple needs no power,
-// square root or division except the damping's reciprocal.  One thread per pair
-// (j, k), j > k, loops over i > j, so the lanes of a wavefront share the loop
-// length; gradient and CN adjoint of i go to LDS atomics (one system of at most
-// kWideAtoms atoms per block), those of j and k stay in registers.  The D4-CN
-// chain finishes the kernel.
-// FIX: the LDS sums of the i-atom adjoints run in fixed point (reproducible
-// mode), so their value does not depend on the order of the LDS atom// one ordered pair's entries of the tables, NN apart
+// square root or division except the damping's reciprocal.
+
+// one ordered pair's entries of the tables, NN apart
 __device__ __forceinline__ void atm_pair(const Topo& t, int a0, int lx, int ly, const double* w4, const double* dw4c,
                                          double* tab, int64_t NN) {
   const int x = a0 + lx, y = a0 + ly;
@@ -1059,6 +1055,12 @@ __device__ __forceinline__ void triangle_pair(int64_t p, int& lj, int& lk) {
   lk = (int)(p - (int64_t)lj * (lj - 1) / 2);
 }
 
+// The three-body energy and gradient of a system of at most kWideAtoms atoms, one
+// block.  One thread per pair (j, k), j > k, loops over i > j, so the lanes of a
+// wavefront share the loop length; gradient and CN adjoint of i go to LDS atomics,
+// those of j and k stay in registers.  The D4-CN chain finishes the kernel.
+// FIX: the LDS sums of the i-atom adjoints run in fixed point (reproducible
+// mode), so their value does not depend on the order of the LDS atomics.
 template <bool FIX>
 __global__ __launch_bounds__(512) void k_force_atm(Topo t, const int* order, const unsigned char* valid,
                                                    const double* cnd4, double* w4, double* dw4c,
