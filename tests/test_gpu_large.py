@@ -1,24 +1,19 @@
 """Systems above 1024 AOs on the GPU.
 
-Systems of at most 1024 AOs keep their per-system work vectors in LDS.  Larger
-ones, up to 8192 AOs, run instantiations of the same kernels with these
-vectors in a global slice per system:
-- the conditioning estimate;
-- the blocked Householder reduction, whose symmetric product and panel dots
-  run over row chunks of 16 slots of 64 rows;
-- the eigensolver;
-- the back-transformation;
-- the spin fold;
-- the three-body force kernel.
+Up to 8192 AOs.  Above 1024 the conditioning estimate and the spin fold keep
+their per-system work vectors in a global slice instead of LDS; above 1280 the
+blocked Householder reduction takes over from the teams (its symmetric product
+and panel dots run over row chunks of 16 slots of 64 rows); above 2048 the
+eigenpairs of T come from one block per system, and the back-transformation
+keeps its columns in global memory.
 The reference CPU path has no size limit (LAPACK dsyevd per system,
 eigensolver.cpp:1221-1254).
 
 Checks:
 - a ragged batch against the oracle: C190H382 (1142 AOs), an unrestricted
-  C190H381 radical (1141 AOs), and members on the blocked (362 AOs) and
-  register (122 AOs) paths;
-- C350H702 (2102 AOs, 33 slots: three row chunks) against the committed
-  oracle fixture;
+  C190H381 radical (1141 AOs), and members of 367 (teams) and 122 AOs;
+- sizes at the switches from 1281 to 2049 AOs and C350H702 (2102 AOs, 33 slots:
+  three row chunks) against the committed oracle fixtures;
 - central differences of the GPU's own energies at 1142 AOs;
 - the plain and graph-captured paths agree, and reproducible mode repeats
   bit for bit;
@@ -248,3 +243,27 @@ def test_large_clusters_in_a_split_tridiagonal():
     assert np.abs(out.energies - ref["energies"]).max() <= E_TOL
     a1 = b.atom_offsets[1]
     assert np.abs(out.charges[:a1] - ref["charges"][:a1]).max() <= 1e-5
+
+
+def test_size_switches_above_1280_aos():
+    # 1281 (the blocked reduction before the spread eigen stage), 1536 and 1537 (the
+    # back-transformation's 12 and 16 row tiles a wavefront), 2048 and 2049 (the spread
+    # eigen stage's last size; one block and the columns in global memory above it)
+    fx = np.load(os.path.join(os.path.dirname(FIXTURE), "switch_sizes.npz"))
+    off = fx["atom_offsets"]
+    systems = [dict(Z=fx["Z"][a:z], xyz=fx["xyz"][a:z], charge=0.0, uhf=0) for a, z in zip(off[:-1], off[1:])]
+    assert [O.basis_counts(s["Z"])[1] for s in systems] == fx["sizes"].tolist() == [1281, 1536, 1537, 2048, 2049]
+    b = workloads.from_systems(systems)
+    ctx = interface.Context("hip", 0)
+    try:
+        print("case 1281, 1536, 1537, 2048 and 2049 AOs", flush=True)
+        out = _run(ctx, b)
+    finally:
+        ctx.close()
+    assert np.all(out.per_system_status == 0)
+    deviation = [np.abs(out.energies - fx["energies"]).max(), np.abs(out.forces + fx["gradient"]).max(),
+                 np.abs(out.charges - fx["charges"]).max()]
+    print("|dE| %.1e |dF| %.1e |dq| %.1e" % tuple(deviation), flush=True)
+    assert np.abs(out.scc_iterations - fx["iterations"]).max() <= 1
+    # rounding: eigenvectors carry 2049 eps |H| / gap <= 2049 * 2.2e-16 * 10 / 0.1 = 5e-11
+    assert max(deviation) <= 1e-9
