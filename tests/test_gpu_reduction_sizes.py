@@ -102,7 +102,7 @@ def check(sizes, make=stack, threads=4):
 
 
 def test_result_depends_on_the_system_alone(monkeypatch):
-    """64 systems of 302 AOs take 640 team members, more than the chip holds at once:
+    """64 systems of 302 AOs take 320 team members, more than the chip holds at once:
     the bits of one lane are those of two lanes, and of systems computed alone."""
     rng = np.random.default_rng(64)
     systems = [workloads.alkane(50, rng) for _ in range(64)]

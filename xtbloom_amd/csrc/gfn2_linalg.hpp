@@ -1136,10 +1136,10 @@ __device__ __forceinline__ void tridiag_full(double* A, int64_t ld, int n, doubl
 // device finds its gate closed from the start.  The spins are bounded too; one that
 // runs out fails the system (status 8).
 //
-// Bound: the latency of a step, 4.5 us at 482 AOs (16 members) and 5.5 us at
+// Bound: the latency of a step, 4.1 us at 482 AOs (8 members) and 5.1 us at
 // 1142 (36), most of it the exchange through memory.  Measured against one
 // workgroup per system with panels of 16 reflectors (k_tridiag_blocked): 9.0 ->
-// 1.3 + 0.4 ms a round for 14 systems of 258-482 AOs, 111 -> 5.3 ms at 1142.
+// 1.2 + 0.4 ms a round for 14 systems of 258-482 AOs, 111 -> 4.8 ms at 1142.
 // Members on one XCD (every eighth block) were 10 % slower than neighbours.
 constexpr int kTeamN = 1280;
 constexpr int kTeamRing = 8;
@@ -1501,7 +1501,7 @@ __global__ __launch_bounds__(512) void k_tridiag_team(Topo t, const int* order, 
 // terms in the same order, so that the results do not depend on whether a team
 // could assemble.  Bound: the sweep over the trailing block (16 n^2 bytes a step
 // through one CU): 205 ms at 1280 AOs (240 with four tiles in flight instead of
-// ten), where the team takes 6.6 ms.
+// ten), where the team takes 6 ms.
 template <int TILES>
 __device__ __forceinline__ void team_solo(int n, double* A, double* d, double* e, double (&xb)[2][kTeamN],
                                           double (&rb)[kTeamN], double (&pb)[kTeamN]) {
